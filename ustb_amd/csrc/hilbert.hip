@@ -7,10 +7,12 @@
 // LDS (one complex signal a + i b; forward and inverse radix-8 Stockham FFTs,
 // a last radix-2/4 stage where log2 L is not a multiple of 3, twiddles from a
 // per-device table rounded from FP64), so HBM sees the traces read once and
-// the analytic signals written once. Other lengths of the form 2^a 3^b 5^c
-// 7^d up to 4096: the same with mixed-radix stages. The rest: hipFFT (R2C
-// forward, C2C inverse, with the weights in between); plans and their
-// spectrum buffers are cached per (device, L, traces, stream).
+// the analytic signals written once. Lengths 2^a 3^b 5^c 7^d in (2048, 4096]:
+// the same with mixed-radix stages. Every other length from 3 to 8192 (primes
+// included): H(x) by a cyclic convolution of a power-of-two length in LDS.
+// The rest (and 3 * 2^a above 4096): hipFFT (R2C forward, C2C inverse, with
+// the weights in between); plans and their spectrum buffers are cached per
+// (device, L, traces, stream).
 #include <hip/hip_runtime.h>
 #include <hipfft/hipfft.h>
 #include <stdarg.h>
@@ -149,8 +151,13 @@ __device__ __forceinline__ int pad8(int e) { return e + (e >> 3); }
 // stage Ns = 8 and 64 (radix 8), then Ns = 512 (radix N / 512); entry
 // (r - 1) Ns + k of a stage is exp(-2 pi i k r / (Ns R)), so the lanes of a
 // wave (consecutive k) read consecutive entries.
-constexpr int kTw8 = 0, kTw64 = 7 * 8, kTw512 = kTw64 + 7 * 64;  // 504 entries before the last stage
-__host__ __device__ constexpr int twiddle_count(int N) { return kTw512 + (N / 512 - 1) * 512; }
+// N > 4096 (the convolution path): stage 512 is radix 8 and a stage Ns = 4096
+// (radix N / 4096) follows.
+constexpr int kTw8 = 0, kTw64 = 7 * 8, kTw512 = kTw64 + 7 * 64;  // 504 entries before stage 512
+constexpr int kTw4096 = kTw512 + 7 * 512;
+__host__ __device__ constexpr int twiddle_count(int N) {
+  return N <= 4096 ? kTw512 + (N / 512 - 1) * 512 : kTw4096 + (N / 4096 - 1) * 4096;
+}
 
 // One Stockham stage of radix R over buf (N points, N / 8 threads, 8 points
 // per thread): butterfly j reads j + r N/R, twiddles by exp(s 2 pi i k r /
@@ -259,7 +266,7 @@ __global__ __launch_bounds__(N / 8) void hilbert_lds_kernel(const float* __restr
   }
 }
 
-// ---- LDS path, other lengths: N = 2^a 3^b 5^c 7^d <= 4096 ----
+// ---- LDS path, N = 2^a 3^b 5^c 7^d <= 4096 (used above 2048) ----
 // Mixed-radix Stockham stages (radix 8 while 8 divides what is left, then 4
 // or 2, then 3, 5, 7), kMixT threads per block, each holding up to
 // mix_maxb(R) butterflies of a stage; twiddles exp(-2 pi i m / N) from a plain device
@@ -498,8 +505,10 @@ __global__ void twiddle_kernel(float2* __restrict__ tw, int N) {
     Ns = 8, R = 8, q = i - kTw8;
   } else if (i < kTw512) {
     Ns = 64, R = 8, q = i - kTw64;
+  } else if (N <= 4096 || i < kTw4096) {
+    Ns = 512, R = N <= 4096 ? N / 512 : 8, q = i - kTw512;
   } else {
-    Ns = 512, R = N / 512, q = i - kTw512;
+    Ns = 4096, R = N / 4096, q = i - kTw4096;
   }
   const int r = q / Ns + 1, k = q % Ns;
   double sv, cv;
@@ -533,6 +542,243 @@ hipError_t twiddles(int dev, int N, hipStream_t s, const float2** out) {
   g_twiddles.emplace(key, tw);
   *out = tw;
   return hipSuccess;
+}
+
+// ---- LDS path, any length 3 <= L <= kConvMaxL: circular convolution ----
+// The Hilbert transform H(x) (the analytic signal's imaginary part) is the
+// circular convolution of x with the odd kernel h[n] = (2 / L) sum_{k=1}^{K}
+// sin(2 pi k n / L), K = floor((L - 1) / 2). Periodic in L, it is a linear
+// convolution with h[-(L-1) .. L-1], which one cyclic convolution of N >= 2 L
+// - 1 points, N a power of two, gives on outputs 0 .. L-1: two FFTs of N
+// points per two traces (packed a + i b, h real), where Bluestein's algorithm
+// needs four. h is odd, so its spectrum is i g with g real: the product costs
+// two multiplications per point and the table N floats.
+//
+// A thread holds PT points tid + m N/PT in registers through the whole
+// kernel; each stage passes through LDS once, except the first of either
+// transform and the last, whose points are the thread's own (so the product
+// with g and the global loads and stores need no LDS pass). Bound by the LDS
+// passes and their barriers (6 passes per pair at N = 4096; the floor of HBM
+// traffic is 0.035 ms where this takes 0.081). 9600 traces, against hipFFT
+// (Bluestein's algorithm, or its own radices 11 and 13 at 2176):
+//   L = 257: 0.022 (0.130) ms; 1021: 0.036 (0.308); 1527: 0.082 (0.615);
+//   2049: 0.218 (1.56); 2176: 0.22 (0.63); 4095: 0.28 (1.83); 5000: 0.68
+//   (1.10); 7919: 0.75 (4.67); 8192: 0.74 (0.90)
+// with errors against FP64 of 0.9-1.3e-7 (2-4e-7): the real parts are the
+// samples themselves and there is half the arithmetic.
+constexpr int kConvMaxL = 8192;
+constexpr int conv_points(int N) { return N <= 4096 ? 8 : 16; }
+
+// Stage Ns (radix R) on the registers' points; LAST: the results stay in the
+// registers (output tid + m NT is where the inputs were).
+template <int N, int PT, int R, bool LAST>
+__device__ __forceinline__ void conv_stage(float2 (&v)[PT], float2* buf, const float2* __restrict__ tw, int Ns,
+                                           float s) {
+  constexpr int NT = N / PT, IT = PT / R;
+  const int tid = threadIdx.x;
+#pragma unroll
+  for (int it = 0; it < IT; ++it) {
+    const int j = tid + it * NT;
+    const int k = j & (Ns - 1);
+    float2 x[R];
+#pragma unroll
+    for (int r = 0; r < R; ++r) x[r] = v[it + r * IT];
+    if (Ns > 1) {
+#pragma unroll
+      for (int r = 1; r < R; ++r) {
+        float2 t = tw[(r - 1) * Ns + k];  // exp(-2 pi i k r / (Ns R)); conjugated for the inverse
+        t.y = -s * t.y;
+        x[r] = cmulf(x[r], t);
+      }
+    }
+    if (R == 8) dft8(x, s);
+    else if (R == 4) dft4(x, s);
+    else dft2(x, s);
+    if (LAST) {
+#pragma unroll
+      for (int r = 0; r < R; ++r) v[it + r * IT] = x[r];
+    } else {
+      // pad8(d + r Ns): r Ns is a multiple of 8, or (Ns = 1, R = 8) d is
+      const int d = pad8((j - k) * R + k), step = Ns > 1 ? pad8(Ns) : 1;
+#pragma unroll
+      for (int r = 0; r < R; ++r) buf[d + r * step] = x[r];
+    }
+    if (PT > 8) __builtin_amdgcn_sched_barrier(0);  // one butterfly's registers at a time
+  }
+  if (!LAST) {
+    __syncthreads();
+#pragma unroll
+    for (int m = 0; m < PT; ++m) v[m] = buf[pad8(tid) + m * pad8(NT)];
+    __syncthreads();
+  }
+}
+
+template <int N, int PT>
+__device__ __forceinline__ void conv_fft(float2 (&v)[PT], float2* buf, const float2* tws,
+                                         const float2* __restrict__ twg, float s) {
+  conv_stage<N, PT, 8, false>(v, buf, tws, 1, s);
+  conv_stage<N, PT, 8, false>(v, buf, tws + kTw8, 8, s);
+  conv_stage<N, PT, 8, N == 512>(v, buf, tws + kTw64, 64, s);
+  if (N == 1024) conv_stage<N, PT, 2, true>(v, buf, twg + kTw512, 512, s);
+  if (N == 2048) conv_stage<N, PT, 4, true>(v, buf, twg + kTw512, 512, s);
+  if (N >= 4096) conv_stage<N, PT, 8, N == 4096>(v, buf, twg + kTw512, 512, s);
+  if (N == 8192) conv_stage<N, PT, 2, true>(v, buf, twg + kTw4096, 4096, s);
+  if (N == 16384) conv_stage<N, PT, 4, true>(v, buf, twg + kTw4096, 4096, s);
+}
+
+template <int N>
+__global__ __launch_bounds__(N / conv_points(N), 4) void hilbert_conv_kernel(const float* __restrict__ rf,
+                                                                         float2* __restrict__ z,
+                                                                         const float2* __restrict__ twg,
+                                                                         const float* __restrict__ g,
+                                                                         long long traces, int L) {
+  constexpr int PT = conv_points(N), NT = N / PT;
+  __shared__ float2 buf[N + N / 8];
+  __shared__ float2 tws[kTw512];
+  __shared__ int nonfinite[NT / 64];
+  const int tid = threadIdx.x;
+  const size_t ta = 2 * (size_t)blockIdx.x;
+  const bool has_b = (long long)ta + 1 < traces;
+  const float* __restrict__ xa = rf + ta * L;
+  const float* __restrict__ xb = xa + L;
+  // 2 L - 1 <= N, so the points m >= PT / 2 (beyond N / 2 >= L) are zeros
+  float2 x[PT / 2];
+  float bad_a = 0.0f, bad_b = 0.0f;  // NaN where a sample is not finite
+#pragma unroll
+  for (int m = 0; m < PT / 2; ++m) {
+    const int i = tid + m * NT;
+    x[m] = make_float2(i < L ? xa[i] : 0.0f, i < L && has_b ? xb[i] : 0.0f);
+    bad_a += x[m].x * 0.0f;
+    bad_b += x[m].y * 0.0f;
+  }
+  for (int i = tid; i < kTw512; i += NT) tws[i] = twg[i];
+  // a trace with a sample that is not finite is NaN throughout (as its own
+  // FFT would make it) and must not reach the other trace of the pair
+  const unsigned long long am = __ballot(bad_a != 0.0f), bm = __ballot(bad_b != 0.0f);
+  if ((tid & 63) == 0) nonfinite[tid >> 6] = (am ? 1 : 0) | (bm ? 2 : 0);
+  __syncthreads();
+  int bad = 0;
+#pragma unroll
+  for (int w = 0; w < NT / 64; ++w) bad |= nonfinite[w];
+  float2 v[PT];
+#pragma unroll
+  for (int m = 0; m < PT; ++m)
+    v[m] = m < PT / 2 ? make_float2(bad & 1 ? 0.0f : x[m < PT / 2 ? m : 0].x, bad & 2 ? 0.0f : x[m < PT / 2 ? m : 0].y)
+                      : make_float2(0.0f, 0.0f);
+  conv_fft<N, PT>(v, buf, tws, twg, -1.0f);
+#pragma unroll
+  for (int m = 0; m < PT; ++m) {
+    const float gm = g[tid + m * NT];
+    v[m] = make_float2(-gm * v[m].y, gm * v[m].x);
+  }
+  conv_fft<N, PT>(v, buf, tws, twg, 1.0f);
+  float2* __restrict__ za = z + ta * L;
+  float2* __restrict__ zb = za + L;
+#pragma unroll
+  for (int m = 0; m < PT / 2; ++m) {
+    const int i = tid + m * NT;
+    if (i < L) {
+      // 16 points per thread: the samples again (L2) instead of 16 registers
+      const float a = PT == 16 ? xa[i] : x[m].x, b = PT == 16 ? (has_b ? xb[i] : 0.0f) : x[m].y;
+      const float nan = __builtin_nanf("");
+      za[i] = bad & 1 ? make_float2(nan, nan) : make_float2(a, v[m].x);
+      if (has_b) zb[i] = bad & 2 ? make_float2(nan, nan) : make_float2(b, v[m].y);
+    }
+  }
+}
+
+// The smallest power of two >= max(512, 2 L - 1).
+int conv_length(int L) {
+  int n = 512;
+  while (n < 2 * L - 1) n *= 2;
+  return n;
+}
+
+// h[n], n < L, in FP64: sum_{k=1}^{K} sin(k t) = sin(K t / 2) sin((K + 1) t /
+// 2) / sin(t / 2), t = 2 pi n / L, the arguments reduced exactly mod 2 L.
+__global__ void conv_kernel_kernel(double* __restrict__ h, int L) {
+  const int n = blockIdx.x * blockDim.x + threadIdx.x;
+  if (n >= L) return;
+  const long long K = (L - 1) / 2, M = 2LL * L;
+  if (n == 0) {
+    h[0] = 0.0;
+    return;
+  }
+  const double a = sinpi((double)((K * n) % M) / L), b = sinpi((double)(((K + 1) * n) % M) / L);
+  h[n] = (2.0 / L) * a * b / sinpi((double)n / L);
+}
+
+// g[k] = -(2 / N) sum_{n=1}^{L-1} h[n] sin(2 pi n k / N), one block per k.
+__global__ __launch_bounds__(256) void conv_spectrum_kernel(const double* __restrict__ h, float* __restrict__ g,
+                                                           int L, int N) {
+  __shared__ double part[256];
+  const int k = blockIdx.x;
+  double s = 0.0;
+  for (int n = 1 + (int)threadIdx.x; n < L; n += 256)
+    s += h[n] * sinpi(2.0 * (double)(((long long)n * k) % N) / N);
+  part[threadIdx.x] = s;
+  __syncthreads();
+  for (int d = 128; d > 0; d >>= 1) {
+    if ((int)threadIdx.x < d) part[threadIdx.x] += part[threadIdx.x + d];
+    __syncthreads();
+  }
+  if (threadIdx.x == 0) g[k] = (float)(-2.0 * part[0] / N);
+}
+
+struct ConvTable {
+  double* h = nullptr;  // [L], then g (the allocation's start)
+  float* g = nullptr;   // [N]
+  unsigned long long last_use = 0;
+};
+constexpr int kMaxConvTables = 64;  // per device; at most 128 KiB each
+std::map<std::pair<int, int>, ConvTable> g_conv;
+
+// The spectrum table of length L on device dev (the current one): built once
+// (and waited for on the caller's stream); the least recently used beyond
+// kMaxConvTables is released after a device synchronisation. Caller holds g_mu.
+hipError_t conv_table(int dev, int L, hipStream_t s, const float** out) {
+  const auto key = std::make_pair(dev, L);
+  auto it = g_conv.find(key);
+  if (it == g_conv.end()) {
+    int n = 0;
+    auto lru = g_conv.end();
+    for (auto c = g_conv.begin(); c != g_conv.end(); ++c) {
+      if (c->first.first != dev) continue;
+      ++n;
+      if (lru == g_conv.end() || c->second.last_use < lru->second.last_use) lru = c;
+    }
+    if (n >= kMaxConvTables) {
+      const hipError_t e = hipDeviceSynchronize();  // no queued work still reads it
+      if (e != hipSuccess) return e;
+      (void)hipFree(lru->second.h);
+      g_conv.erase(lru);
+    }
+    const int N = conv_length(L);
+    ConvTable t;
+    hipError_t e = hipMalloc((void**)&t.h, sizeof(double) * (size_t)L + sizeof(float) * (size_t)N);
+    if (e != hipSuccess) return e;
+    t.g = reinterpret_cast<float*>(t.h + L);
+    hipLaunchKernelGGL(conv_kernel_kernel, dim3((unsigned)((L + 255) / 256)), dim3(256), 0, s, t.h, L);
+    hipLaunchKernelGGL(conv_spectrum_kernel, dim3((unsigned)N), dim3(256), 0, s, t.h, t.g, L, N);
+    e = hipGetLastError();
+    if (e == hipSuccess) e = hipStreamSynchronize(s);
+    if (e != hipSuccess) {
+      (void)hipFree(t.h);
+      return e;
+    }
+    it = g_conv.emplace(key, t).first;
+  }
+  it->second.last_use = ++g_plan_clock;
+  *out = it->second.g;
+  return hipSuccess;
+}
+
+template <int N>
+hipError_t launch_hilbert_conv(const float* rf, float2* z, long long traces, int L, const float2* tw, const float* g,
+                               hipStream_t s) {
+  hipLaunchKernelGGL(hilbert_conv_kernel<N>, dim3((unsigned)((traces + 1) / 2)), dim3(N / conv_points(N)), 0, s, rf, z,
+                     tw, g, traces, L);
+  return hipGetLastError();
 }
 
 template <int N>
@@ -574,14 +820,45 @@ extern "C" int ustbx_hilbert(const float* rf, void* analytic, int32_t L, int64_t
     }
     return USTBX_OK;
   }
+  // L = 2^a 3^b 5^c 7^d: its own mixed-radix transforms where the convolution
+  // would need 8192 points (9600 traces of 3500: 0.24 against 0.27 ms; of 1500,
+  // 4096 points: 0.130 against 0.089 ms)
   MixPlan pl;
-  if (mix_plan(L, pl)) {
+  if ((L < 3 || conv_length(L) > 4096) && mix_plan(L, pl)) {
     const float2* tw = nullptr;
     e = plain_twiddles(dev, L, s, &tw);
     if (e == hipSuccess) {
       hipLaunchKernelGGL(hilbert_mixed_kernel, dim3((unsigned)((traces + 1) / 2)), dim3(kMixT), 0, s, rf,
                          reinterpret_cast<float2*>(analytic), tw, (long long)traces, (int)L, pl);
       e = hipGetLastError();
+    }
+    if (e != hipSuccess) return fail(st, USTBX_E_GPU, "HIP error: %s", hipGetErrorString(e));
+    if (st) {
+      st->code = USTBX_OK;
+      st->message[0] = 0;
+    }
+    return USTBX_OK;
+  }
+  // above 4096 the convolution takes 16384 points, one block per CU; hipFFT's
+  // own kernels for 3 * 2^a are the faster ones there (L = 6144: 0.635 against
+  // 0.70 ms; other products of small primes 0.90-1.7 against 0.67-0.75 ms)
+  auto three_pow2 = [](int n) { return n % 3 == 0 && ((n / 3) & (n / 3 - 1)) == 0; };
+  if (L >= 3 && L <= kConvMaxL && !(L > 4096 && three_pow2(L))) {
+    const int N = conv_length(L);
+    const float2* tw = nullptr;
+    const float* g = nullptr;
+    e = twiddles(dev, N, s, &tw);
+    if (e == hipSuccess) e = conv_table(dev, L, s, &g);
+    if (e == hipSuccess) {
+      float2* z = reinterpret_cast<float2*>(analytic);
+      switch (N) {
+        case 512: e = launch_hilbert_conv<512>(rf, z, traces, L, tw, g, s); break;
+        case 1024: e = launch_hilbert_conv<1024>(rf, z, traces, L, tw, g, s); break;
+        case 2048: e = launch_hilbert_conv<2048>(rf, z, traces, L, tw, g, s); break;
+        case 4096: e = launch_hilbert_conv<4096>(rf, z, traces, L, tw, g, s); break;
+        case 8192: e = launch_hilbert_conv<8192>(rf, z, traces, L, tw, g, s); break;
+        default: e = launch_hilbert_conv<16384>(rf, z, traces, L, tw, g, s); break;
+      }
     }
     if (e != hipSuccess) return fail(st, USTBX_E_GPU, "HIP error: %s", hipGetErrorString(e));
     if (st) {
