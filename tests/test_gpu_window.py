@@ -1,0 +1,112 @@
+"""Dimension receive and none on patch tiles with staged sample windows: scans
+whose axes leave part tiles, every wave count around a step, traces that end
+inside the image (terms out of the window), partly weighted tiles and coarse
+grids (long rows), against the FP64 beamformer on the plan's own matrices; RF
+data against das_c's arithmetic bit for bit."""
+from __future__ import annotations
+
+import math
+
+import numpy as np
+import pytest
+
+torch = pytest.importorskip("torch")
+
+from oracle import oracle as O
+from ustb_amd import ops
+from ustb_amd.enums import Window
+from ustb_amd.geometry import make_plan
+from ustb_amd.uff import Apodization, LinearArray, LinearScan, MatrixArray, SectorScan, Wave
+
+pytestmark = pytest.mark.gpu
+C = 1540.0
+
+
+def _setup(kind, W, nx, nz, zmax=25e-3, N=21):
+    if kind == "sector":
+        prb = LinearArray(N, 0.2e-3)
+        ang = np.deg2rad(np.linspace(-30, 30, W)) if W > 1 else np.zeros(1)
+        src = [(-10e-3 * math.sin(a), 0.0, -10e-3 * math.cos(a)) for a in ang]
+        seq = [Wave.spherical(*s, sound_speed=C, origin=s) for s in src]
+        return prb, SectorScan(np.deg2rad(np.linspace(-40, 40, nx)), np.linspace(2e-3, zmax, nz)), seq
+    if kind == "volume":
+        seq = [Wave.spherical(x, 0.0, -8e-3, sound_speed=C, origin=(x, 0.0, -8e-3)) for x in np.linspace(-2e-3, 2e-3, W)]
+        return (MatrixArray(5, 4, 0.3e-3), LinearScan(np.linspace(-3e-3, 3e-3, nx), np.linspace(4e-3, zmax, nz),
+                                                       np.linspace(-2e-3, 2e-3, 7)), seq)
+    seq = [Wave.plane(a, sound_speed=C) for a in (np.deg2rad(np.linspace(-16, 16, W)) if W > 1 else np.zeros(1))]
+    return LinearArray(N, 0.3e-3), LinearScan(np.linspace(-8e-3, 8e-3, nx), np.linspace(4e-3, zmax, nz)), seq
+
+
+def _run(cuda, kind, dim, W, nx, nz, F, rf, cubic, phase, L, rx, zmax=25e-3, tx=Apodization()):
+    prb, scan, seq = _setup(kind, W, nx, nz, zmax)
+    fs, fd = (20.8e6, 0.0) if rf else (10.4e6, 5.2e6)
+    plan = make_plan(prb, scan, seq, n_samples=L, n_frames=F, sampling_frequency=fs, initial_time=0.0,
+                     modulation_frequency=fd, sound_speed=C, receive_apodization=rx, transmit_apodization=tx,
+                     dimension=dim, interpolation=int(cubic), separable_phase=phase == "separable")
+    rng = np.random.default_rng(W * 100 + nz)
+    ch = (rng.standard_normal((F, W, prb.N_elements, L)) +
+          1j * rng.standard_normal((F, W, prb.N_elements, L))).astype(np.complex64)
+    dch = torch.from_numpy(ch).to(cuda)
+    got = plan.run(dch)
+    ta, ra, td, rd = plan.materialize()
+    plan.close()
+    return got, dch, (ta, ra, td, rd), fs, fd
+
+
+TUKEY = Apodization(Window.tukey25, f_number=1.7)
+BOX = Apodization(Window.boxcar, f_number=2.5)
+CASES = [
+    # kind, W, nx, nz, F, cubic, phase, L, rx, zmax
+    ("linear", 1, 37, 61, 1, False, "separable", 512, TUKEY, 25e-3),
+    ("linear", 4, 16, 16, 1, False, "separable", 512, Apodization(), 25e-3),
+    ("linear", 5, 33, 65, 2, False, "dasc", 512, BOX, 25e-3),
+    ("linear", 8, 17, 130, 1, True, "separable", 300, TUKEY, 25e-3),   # traces end inside the image
+    ("linear", 9, 40, 31, 3, True, "dasc", 260, BOX, 25e-3),
+    ("linear", 3, 35, 24, 2, False, "separable", 512, TUKEY, 40e-3),   # coarse depths: rows of 128 samples
+    ("sector", 7, 29, 50, 1, False, "dasc", 512, BOX, 25e-3),
+    ("sector", 13, 18, 33, 5, False, "separable", 310, TUKEY, 25e-3),
+    ("volume", 5, 9, 35, 1, False, "separable", 400, Apodization(Window.tukey25, f_number=(1.2, 1.2)), 12e-3),
+    ("volume", 2, 6, 18, 2, True, "dasc", 400, Apodization(), 12e-3),
+]
+
+
+@pytest.mark.parametrize("dim", [0, 1])
+@pytest.mark.parametrize("case", CASES, ids=lambda c: "-".join(str(v) for v in c[:7]))
+def test_iq_against_fp64(cuda, case, dim):
+    kind, W, nx, nz, F, cubic, phase, L, rx, zmax = case
+    print(f"case window {case[:8]} dim={dim}", flush=True)
+    got, ch, (ta, ra, td, rd), fs, fd = _run(cuda, kind, dim, W, nx, nz, F, False, cubic, phase, L, rx, zmax)
+    ref = O.beamform_fp64(ch.cpu().numpy(), fs, 0.0, ta.cpu().numpy(), ra.cpu().numpy(), td.cpu().numpy(),
+                          rd.cpu().numpy(), fd, dim, interp="cubic" if cubic else "linear", w0=O.dasc_wd(fd),
+                          index="fp32")
+    # FP32 products and sums of at most 21 terms and the FP32 phase argument
+    # of das_c (wd * delay up to 1700 rad at 6e-8 relative: 1e-4 per term)
+    tol = 2e-4 if phase == "dasc" else 1e-5
+    assert np.max(np.abs(got.cpu().numpy() - ref)) <= tol * np.max(np.abs(ref))
+
+
+@pytest.mark.parametrize("dim", [0, 1])
+@pytest.mark.parametrize("kind,W,nx,nz,F,L", [("linear", 1, 37, 61, 1, 900), ("linear", 6, 20, 45, 1, 500),
+                                               ("sector", 5, 31, 33, 3, 500), ("volume", 3, 9, 20, 2, 500)])
+def test_rf_is_das_c(cuda, kind, W, nx, nz, F, L, dim):
+    print(f"case window rf {kind} W={W} dim={dim}", flush=True)
+    got, ch, (ta, ra, td, rd), fs, fd = _run(cuda, kind, dim, W, nx, nz, F, True, False, "separable", L, BOX, 12e-3)
+    ref = ops.das(ch, fs, 0.0, ta, ra, td, rd, fd, dim, dasc_order=True)
+    assert torch.equal(got, ref)
+
+
+@pytest.mark.parametrize("dim", [0, 1])
+def test_samples_outside_the_weights_stay_out(cuda, dim):
+    """Non-finite samples reach no term that das_c skips (zero receive weight)."""
+    prb, scan, seq = _setup("linear", 3, 40, 64)
+    plan = make_plan(prb, scan, seq, n_samples=512, n_frames=1, sampling_frequency=10.4e6, initial_time=0.0,
+                     modulation_frequency=5.2e6, sound_speed=C, receive_apodization=BOX, transmit_apodization=Apodization(),
+                     dimension=dim, interpolation=0)
+    rng = np.random.default_rng(3)
+    ch = (rng.standard_normal((1, 3, 21, 512)) + 1j * rng.standard_normal((1, 3, 21, 512))).astype(np.complex64)
+    ch[0, :, 4, 100:140] = np.nan
+    got = plan.run(torch.from_numpy(ch).to(cuda)).cpu().numpy()
+    ta, ra, td, rd = (t.cpu().numpy() for t in plan.materialize())
+    plan.close()
+    ref = O.beamform_fp64(ch, 10.4e6, 0.0, ta, ra, td, rd, 5.2e6, dim, w0=O.dasc_wd(5.2e6), index="fp32")
+    assert np.array_equal(np.isnan(got), np.isnan(ref)) and np.isnan(ref).any()

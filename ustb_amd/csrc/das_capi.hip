@@ -493,6 +493,22 @@ int ustbx_das_run_host(const ustbx_das_desc* d, const void* ch, const float* tx_
 
 namespace {
 
+// Tiles 0 .. tiles - 1, tpl of them down each line (group): each of `shares`
+// contiguous shares visited depth band by depth band.
+std::vector<int> line_band_order(int tpl, int tiles, int shares) {
+  std::vector<int> order(tiles);
+  for (int t = 0; t < tiles; ++t) order[t] = t;
+  const int q = tiles / shares, r = tiles % shares;
+  for (int k = 0; k < shares; ++k) {
+    const int s0 = k * q + std::min(k, r);
+    const int cnt = q + (k < r ? 1 : 0);
+    std::stable_sort(order.begin() + s0, order.begin() + s0 + cnt, [tpl](int a, int b) {
+      return a % tpl != b % tpl ? a % tpl < b % tpl : a / tpl < b / tpl;
+    });
+  }
+  return order;
+}
+
 // Tile order of the receive-table kernels. Dimension both (shares = 8):
 // blocks go to the 8 XCDs round-robin and each XCD takes a contiguous range of
 // tile indices (the XCD remap), i.e. whole scan lines (depth-fastest pixel
@@ -509,16 +525,7 @@ std::vector<int> band_major_order(const DevScan& sc, int tile_ps, int tiles, int
   for (int t = 0; t < tiles; ++t) order[t] = t;
   if (!(sc.kind == SCAN_LINEAR || sc.kind == SCAN_SECTOR) || (tile_ps == 0 && sc.n0 % 64 != 0) || tiles < shares)
     return order;
-  const int tpl = tile_ps ? sc.n0 >> tile_ps : sc.n0 / 64;  // tiles per line (per line group: patches)
-  const int q = tiles / shares, r = tiles % shares;
-  for (int k = 0; k < shares; ++k) {
-    const int s0 = k * q + std::min(k, r);
-    const int cnt = q + (k < r ? 1 : 0);
-    std::stable_sort(order.begin() + s0, order.begin() + s0 + cnt, [tpl](int a, int b) {
-      return a % tpl != b % tpl ? a % tpl < b % tpl : a / tpl < b / tpl;
-    });
-  }
-  return order;
+  return line_band_order(tile_ps ? sc.n0 >> tile_ps : sc.n0 / 64, tiles, shares);  // tiles per line (group)
 }
 
 // The on-the-fly receive state covers dimension both with a windowed (or no)
@@ -728,6 +735,155 @@ bool coef_build(ustbx_plan* pl, hipError_t& err) {
   if (err != hipSuccess) return false;
   pl->G.coef = c;
   pl->coef_bytes = bytes;
+  return true;
+}
+
+// The window-staged kernels (das_window.h) cover dimension receive and none on
+// linear and sector scans with das_c's edge rule, frames below 2 GiB, every
+// nonzero weight and every delay finite, and scans fine enough that a patch
+// tile's windows fit an LDS row. Their receive table may take this fraction of
+// the device memory; where it cannot be had the per-lane kernel runs, as for
+// every other plan.
+constexpr double kWindowTableMaxFraction = 0.125;
+
+void window_free(ustbx_plan* pl) {
+  (void)hipFree(pl->win_mem);
+  pl->win_mem = nullptr;
+  pl->win_bytes = 0;
+  pl->G.win.on = 0;
+  pl->G.win_rx = nullptr;
+  pl->G.win_ref = nullptr;
+}
+
+// Builds the tile lists (and for dimension receive and none the receive table
+// and the reference phase). Where it does not apply, or memory is short, the
+// plan stays as it was; false only on a device error.
+bool window_build(ustbx_plan* pl, hipError_t& err) {
+  err = hipSuccess;
+  GeomLaunch& G = pl->G;
+  if (!(G.dim == 0 || G.dim == 1)) return true;
+  if (!(G.scan.kind == SCAN_LINEAR || G.scan.kind == SCAN_SECTOR)) return true;
+  if (G.edge == USTBX_EDGE_PYTHON && G.interp == USTBX_INTERP_LINEAR) return true;
+  if ((int64_t)G.L * G.N * G.W * 8 > 0x7FFFFE00 || G.L < 4) return true;
+  G.rx_compact = G.wd == 0.0f ? 1 : 0;
+  const size_t P = (size_t)G.P;
+  auto al = [](size_t b) { return (b + 255) & ~size_t(255); };
+  const size_t b_rx = al((G.rx_compact ? sizeof(float2) : sizeof(float4)) * (size_t)G.N * P);
+  const size_t b_ref = G.ref_phase ? al(sizeof(float2) * P) : 0;
+  size_t free_b = 0, total_b = 0;
+  if (hipMemGetInfo(&free_b, &total_b) != hipSuccess) return true;
+  if (b_rx > (size_t)(kWindowTableMaxFraction * (double)total_b)) return true;
+
+  // tile shapes (depth bits, x bits, y bits), the squarest windows first; a
+  // shape that pads the scan by more than a tenth over the least goes last
+  struct Shape {
+    int dzb, lxb, lyb;
+    size_t padded;
+  };
+  std::vector<Shape> shapes;
+  if (G.scan.n2 > 1)
+    shapes = {{4, 2, 2, 0}, {3, 3, 2, 0}, {5, 2, 1, 0}};
+  else
+    shapes = {{4, 4, 0, 0}, {3, 5, 0, 0}, {5, 3, 0, 0}, {6, 2, 0, 0}};
+  size_t least = SIZE_MAX;
+  auto ceil_to = [](int n, int b) { return (size_t)((n + (1 << b) - 1) >> b); };
+  for (Shape& s : shapes) {
+    s.padded = (ceil_to(G.scan.n0, s.dzb) * ceil_to(G.scan.n1, s.lxb) * ceil_to(G.scan.n2, s.lyb)) << 8;
+    least = std::min(least, s.padded);
+  }
+  std::stable_partition(shapes.begin(), shapes.end(), [&](const Shape& s) { return s.padded <= least + least / 10; });
+  if (least > 2 * P + 1024) return true;  // a scan of a few lines or depths
+
+  size_t tiles_max = 0;
+  for (const Shape& s : shapes) tiles_max = std::max(tiles_max, s.padded >> 8);
+  const size_t b_wl = al(sizeof(int4) * tiles_max * (size_t)G.W), b_cl = al(sizeof(int4) * tiles_max * (size_t)G.N);
+  const size_t b_cnt = al(sizeof(int) * tiles_max), b_info = al(sizeof(int) * 8);
+  const size_t total = b_rx + b_ref + b_wl + b_cl + 3 * b_cnt + b_info;
+  char* m = nullptr;
+  if (hipMalloc(&m, total) != hipSuccess) {
+    (void)hipGetLastError();
+    return true;
+  }
+  size_t off = 0;
+  auto take = [&](size_t b) {
+    char* q = m + off;
+    off += b;
+    return q;
+  };
+  float4* rx = (float4*)take(b_rx);
+  float2* ref = b_ref ? (float2*)take(b_ref) : nullptr;
+  int4* wl = (int4*)take(b_wl);
+  int4* cl = (int4*)take(b_cl);
+  int* nw = (int*)take(b_cnt);
+  int* nc = (int*)take(b_cnt);
+  int* ord = (int*)take(b_cnt);
+  int* info = (int*)take(b_info);
+  err = launch_window_state(G, rx, ref, nullptr);
+  G.win_rx = rx;
+  G.win_ref = ref;
+  pl->win_mem = m;
+  pl->win_bytes = total;
+  WinTiles& T = G.win;
+  T.n0 = G.scan.n0;
+  T.n1 = G.scan.n1;
+  T.n2 = G.scan.n2;
+  auto lists = [&](const Shape& s, int* h) {
+    T.dzb = s.dzb;
+    T.lxb = s.lxb;
+    T.lyb = s.lyb;
+    // neighbouring lanes: 4 depths, then the lines, whose samples all but
+    // coincide (few LDS bank conflicts); dimension none writes so much that
+    // its stores want whole depth runs
+    T.zl = G.dim == 0 ? s.dzb : 2;
+    T.ntz = (int)ceil_to(T.n0, s.dzb);
+    T.nlx = (int)ceil_to(T.n1, s.lxb);
+    T.nly = (int)ceil_to(T.n2, s.lyb);
+    T.tiles = T.ntz * T.nlx * T.nly;
+    for (int i = 0; i < 8; ++i) h[i] = 0;
+    if (err == hipSuccess) err = hipMemcpy(info, h, sizeof(int) * 8, hipMemcpyHostToDevice);
+    // dimension none writes every (wave, channel), receive every wave
+    if (err == hipSuccess) err = launch_window_lists(G, nw, nc, wl, cl, info, 1, G.dim == 0, nullptr);
+    if (err == hipSuccess) err = hipMemcpy(h, info, sizeof(int) * 8, hipMemcpyDeviceToHost);
+    return err == hipSuccess;
+  };
+  const int slack = G.interp == USTBX_INTERP_CUBIC ? 7 : 5;  // WinSpan::kSlack
+  int best = -1, best_span = 129, last = -1;
+  for (int k = 0; k < (int)shapes.size(); ++k) {
+    int h[8];
+    if (!lists(shapes[k], h)) {
+      window_free(pl);
+      return false;
+    }
+    last = k;
+    if (h[1]) break;  // weights or delays that are not finite: the per-lane kernel
+    if (h[0] + slack < best_span) {
+      best = k;
+      best_span = h[0] + slack;
+    }
+    if (best_span <= 64) break;
+  }
+  if (best >= 0) {
+    int h[8];
+    if (best != last && !lists(shapes[best], h)) {
+      window_free(pl);
+      return false;
+    }
+    const std::vector<int> order = line_band_order(T.ntz, T.tiles, 8);
+    err = hipMemcpy(ord, order.data(), sizeof(int) * order.size(), hipMemcpyHostToDevice);
+    if (err != hipSuccess) {
+      window_free(pl);
+      return false;
+    }
+    T.row = best_span <= 64 ? 64 : 128;
+    T.order = ord;
+    T.nw = nw;
+    T.nc = nc;
+    T.wl = wl;
+    T.cl = cl;
+    T.on = 1;
+    return true;
+  }
+  window_free(pl);
   return true;
 }
 
@@ -1229,6 +1385,14 @@ int ustbx_plan_create(const ustbx_geometry* g, ustbx_plan** plan, ustbx_status* 
     delete pl;
     return hip_fail(st, e, "receive table");
   }
+  if (!window_build(pl, e)) {
+    (void)hipFree(pl->rxtab);
+    (void)hipFree(pl->tx_table);
+    (void)hipFree(pl->unified_tx);
+    (void)hipFree(pl->dev);
+    delete pl;
+    return hip_fail(st, e, "window tables");
+  }
   *plan = pl;
   return ok(st);
 }
@@ -1473,7 +1637,7 @@ int ustbx_plan_active_terms(const ustbx_plan* plan, int64_t* terms, ustbx_status
 int64_t ustbx_plan_pixels(const ustbx_plan* plan) { return plan ? plan->G.P : 0; }
 
 int64_t ustbx_plan_device_bytes(const ustbx_plan* plan) {
-  return plan ? (int64_t)(plan->dev_bytes + plan->tx_table_bytes + plan->unified_bytes + plan->rxtab_bytes +
+  return plan ? (int64_t)(plan->dev_bytes + plan->tx_table_bytes + plan->unified_bytes + plan->rxtab_bytes + plan->win_bytes +
                           plan->coef_bytes)
               : 0;
 }
@@ -1526,6 +1690,7 @@ int32_t ustbx_plan_variant(const ustbx_plan* plan, int32_t* wave_chunk, int32_t*
 void ustbx_plan_destroy(ustbx_plan* plan) {
   if (!plan) return;
   (void)hipFree(plan->G.coef);
+  (void)hipFree(plan->win_mem);
   (void)hipFree(plan->rxtab);
   (void)hipFree(plan->tx_table);
   (void)hipFree(plan->unified_tx);

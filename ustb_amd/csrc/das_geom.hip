@@ -2,6 +2,7 @@
 // that writes the FP32 matrices das.m would hand to the MEX
 // (+midprocess/das.m:95,100,106,206).
 #include "das_geom_impl.h"
+#include "das_window.h"
 
 namespace ustbx {
 
@@ -11,6 +12,8 @@ hipError_t launch_das_geom(const GeomLaunch& G, hipStream_t stream) {
   if (G.variant == 2 && G.dim == MODE_TX) return launch_tx_rxtab(G, stream);
   if (G.variant == 1 && G.dim == MODE_BOTH && ph == PH_SEP && G.F == 1)
     return launch_both_shared(G, stream);
+  if (G.win.on && G.dim == MODE_RX) return launch_window_rx(G, ph, stream);
+  if (G.win.on && G.dim == MODE_NONE) return launch_window_none(G, ph, stream);
   switch (G.dim) {
     case MODE_BOTH: return launch_geom_both(G, ph, G.wave_chunk, G.split, stream);
     case MODE_TX: return launch_geom_tx(G, ph, G.wave_chunk, G.split, stream);

@@ -435,6 +435,13 @@ hipError_t launch_otf_elements(const GeomLaunch& G, float4* e32, hipStream_t str
   return hipGetLastError();
 }
 
+hipError_t launch_window_state(const GeomLaunch& G, float4* rx_table, float2* ref_table, hipStream_t stream) {
+  const unsigned pb = (unsigned)((G.P + kBlock - 1) / kBlock);
+  if (rx_table) hipLaunchKernelGGL(geom_rx_table_kernel, dim3(pb, (unsigned)G.N), dim3(kBlock), 0, stream, G, rx_table);
+  if (ref_table) hipLaunchKernelGGL(geom_ref_table_kernel, dim3(pb), dim3(kBlock), 0, stream, G, ref_table);
+  return hipGetLastError();
+}
+
 hipError_t launch_rxtab_tables(const GeomLaunch& G, float4* rx_table, float2* ref_table, int* tile_nc,
                                int* tile_chl, int* tile_waves, int* tile_nw, int* tile_bad,
                                unsigned long long* nan_mask, hipStream_t stream) {

@@ -27,6 +27,26 @@ hipError_t launch_das_matrix(const MatLaunch& m, hipStream_t stream);
 // Fills n complex64 values with zeros (a kernel, so it can be graph-captured).
 hipError_t launch_zero_fill(void* p, size_t n_complex, hipStream_t stream);
 
+// Tiles of the window-staged kernels (das_window.h): patches of 2^dzb depths
+// x 2^lxb x 2^lyb scan lines, 256 pixels. Lane bits, low to high: zl depth
+// bits, the line bits (x first), the remaining depth bits. Tile index =
+// (line group) * ntz + depth block, line groups x first.
+struct WinTiles {
+  int on;              // the tables below are built
+  int row;             // samples of an LDS row: 64, or 128 on coarse scans
+  int dzb, lxb, lyb, zl;
+  int n0, n1, n2;      // the scan's axis lengths
+  int ntz, nlx, nly, tiles;
+  const int* order;    // [tiles] visiting order
+  const int* nw;       // [tiles] entries of wl, cl
+  const int* nc;
+  // [tiles][W], [tiles][N] {index, floor of the tile's least delay in samples,
+  // floor of its largest, bit 0: the weight is nonzero on every pixel of the
+  // tile, bit 1: on some}; receive delays less t0
+  const int4* wl;
+  const int4* cl;
+};
+
 // Geometry (on-the-fly) path: everything resident in device memory.
 struct GeomLaunch {
   const void* ch;
@@ -98,6 +118,11 @@ struct GeomLaunch {
   // 4 = patches of 16 depths x 4 scan lines (dimension transmit on a linear
   // or sector scan whose axes divide evenly). Fixed when the plan is made.
   int tile_ps;
+  // Window-staged kernels (das_window.h), where win.on: receive table and
+  // reference phase they read.
+  WinTiles win;
+  const float4* win_rx;
+  const float2* win_ref;
   // Stage sample windows through LDS (1) or gather every term's samples
   // (0): dimension both through stage_mask, dimension transmit (variant 2)
   // per (channel, wave). Results do not depend on it.
@@ -125,6 +150,17 @@ hipError_t launch_otf_elements(const GeomLaunch& g, float4* e32, hipStream_t str
 // as launch_rxtab_tables left it; those tiles get no bits).
 hipError_t launch_stage_mask(const GeomLaunch& g, const int* tile_bad, unsigned long long* stage_mask,
                              hipStream_t stream);
+
+// Receive table and reference phase of a window-staged plan (either may be
+// null: not written).
+hipError_t launch_window_state(const GeomLaunch& g, float4* rx_table, float2* ref_table, hipStream_t stream);
+// Tile lists of the window-staged kernels (g.win's shape, g.win_rx): nw, nc,
+// wl, cl as WinTiles names them; info[0] = largest hi - lo sum of a tile's
+// waves and channels, info[1] = 1 where a nonzero weight or a delay is not
+// finite, info[2] = largest wave count of a tile. full: every wave and channel
+// is listed.
+hipError_t launch_window_lists(const GeomLaunch& g, int* nw, int* nc, int4* wl, int4* cl, int* info, int full_w,
+                               int full_n, hipStream_t stream);
 
 hipError_t launch_das_geom(const GeomLaunch& g, hipStream_t stream);
 

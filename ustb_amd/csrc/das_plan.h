@@ -22,6 +22,8 @@ struct ustbx_plan {
   int max_nw;            // largest active-wave count of a tile
   char* rxtab;           // one allocation: receive table, tile data, reference phase
   size_t rxtab_bytes;
+  char* win_mem;         // window-staged kernels: tile lists, visiting order (and for dimension
+  size_t win_bytes;      // receive and none the receive table and reference phase), or null
   size_t coef_bytes;     // variant 3's coefficient buffer (G.coef)
   const int* tile_order; // band-major order (G.tile_order when selected)
   const int* tile_natural;  // tiles in index order, the same partition

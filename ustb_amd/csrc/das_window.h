@@ -1,0 +1,517 @@
+// das_window.h — delay-and-sum on patches of 256 pixels whose sample windows
+// are staged in LDS (dimension both with the separable or RF phase, receive
+// and none with any phase, on linear and sector scans).
+//
+// A tile is a patch of DZ consecutive depths by 256 / DZ neighbouring scan
+// lines (WinTiles), one lane per pixel. For a (channel, wave, frame) all of
+// the tile's terms read one short run of the trace, the tile's window: the
+// block loads it once, coalesced, into an LDS row, and every lane reads its
+// samples from there. That replaces one or two 16-byte gathers per term
+// through the texture path (20 cycles per 64 lanes, the roof of the gathering
+// kernels) by 8 cycles of LDS reads, and the windows that 256 pixels share by
+// one read of L2 or HBM instead of four.
+//
+// Window position. With per-tile integer bounds of a wave's transmit delay and
+// of a channel's receive delay in samples (floor of the tile's minimum and
+// maximum, tables of the plan), every term's index n0 lies in [lo_w + lo_n -
+// 1, hi_w + hi_n + 2]: the -1 and +2 cover both floors and the FP32 rounding
+// of das_c's index (below a quarter sample; the plan checks the magnitude). So a
+// window's place is one scalar addition, and whether all of a channel's terms
+// are inside the sample window (no lane tests anything) one comparison.
+//
+// Loop: rounds of up to WC waves (transmit state in VGPRs) x the tile's
+// channel list x chunks of FCK frames x sub-chunks of WSUB waves; a step
+// stages ROWS = NCH x WSUB x FCK windows (NCH channels at a time where one
+// channel has few waves) while the previous step's are used (two LDS buffers,
+// one barrier per step). The index, the fraction and the weights of a term are
+// formed once for its FCK frames.
+//
+// Rows hold 64 samples, or 128 on coarse scans. Linear interpolation with the
+// separable phase keeps {x, x[+1] - x} per sample in rows of 64, so a term
+// costs two FMAs and no subtraction; the other forms keep the samples.
+#pragma once
+#include <type_traits>
+#include <utility>
+
+#include "das_rxtab.h"
+
+namespace ustbx {
+
+// The sample positions a row must hold beyond hi - lo of the bounds: n0 from
+// lo - 1 to hi + 2, and the samples a term reads around n0.
+template <int SM>
+struct WinSpan {
+  static constexpr int kBack = SM == SM_CUBIC ? 1 : 0;
+  static constexpr int kSlack = 3 + (SM == SM_CUBIC ? 4 : 2);  // samples = (hi - lo) + kSlack
+};
+
+struct WinArgs {
+  const void* ch;      // [F][W][N][L] complex64
+  float2* out;
+  const float4* tx;    // [W][P]
+  const float4* rx;    // [N][P] float4, or float2 (RF plans)
+  const float2* ref;   // [P] or null
+  WinTiles T;
+  int P, N, W, L, F;
+  float t0, fs, wd;
+  int frame_bytes;
+};
+
+typedef const __attribute__((address_space(3))) f4v lds_f4;
+typedef __attribute__((address_space(3))) f4v lds_f4w;
+
+__device__ __forceinline__ int4 scalar_int4(const int4* p) {
+  const __attribute__((address_space(4))) int* q = (const __attribute__((address_space(4))) int*)p;
+  return make_int4(q[0], q[1], q[2], q[3]);
+}
+
+// v of the next lane (lane 63: zero)
+__device__ __forceinline__ float next_lane(float v) {
+  return __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), 0x130, 0xf, 0xf, true));  // wave_shl:1
+}
+
+// f(integral_constant 0), .., f(integral_constant N - 1): the indices of
+// register arrays are constants before any pass runs.
+template <typename F, int... I>
+__device__ __forceinline__ void static_for_seq(const F& f, std::integer_sequence<int, I...>) {
+  (f(std::integral_constant<int, I>()), ...);
+}
+template <int N, typename F>
+__device__ __forceinline__ void static_for(const F& f) {
+  static_for_seq(f, std::make_integer_sequence<int, N>());
+}
+
+template <int SM, int MODE, int PH, int ROW, int WC, int WSUB, int FT, int FCK, int NCH, int CG>
+struct WinKernel {
+  static_assert(MODE == MODE_BOTH || MODE == MODE_RX || MODE == MODE_NONE, "dimension transmit has its own kernel");
+  static_assert(NCH == 1 || (WSUB == WC && FT == FCK), "several channels per step: one sub-chunk, one frame chunk");
+  static_assert(WC % WSUB == 0 && FT % FCK == 0, "whole sub-chunks");
+  static constexpr bool kSep = MODE == MODE_BOTH || PH == PH_SEP;  // T and R from the tables
+  static_assert(ROW == 64 || ROW == 128, "samples of an LDS row");
+  static constexpr bool kDelta = SM == SM_LINEAR && kSep && ROW == 64;
+  static constexpr int kLd = ROW / 64;  // loads per row
+  static constexpr bool kCompact = PH == PH_RF;
+  static constexpr int kShift = kDelta ? 4 : 3;  // log2 bytes per staged sample
+  static constexpr int kRows = NCH * WSUB * FCK;
+  static constexpr int kRowBytes = ROW << kShift;
+  static constexpr int kBufBytes = kRows * kRowBytes;
+  static constexpr int kPer = (kRows + 3) / 4;  // rows a wave stages per step
+  static constexpr int kNF = FT / FCK, kNS = WC / WSUB;
+  static constexpr int kAcc = MODE == MODE_RX ? WC : 1;
+  static constexpr int kSmem = CG * 2 * kBufBytes;
+
+  // One staged term: the index, its row position and whether it counts.
+  struct Term1 {
+    float b;
+    unsigned la;
+    bool ok;
+  };
+
+  template <bool CHK>
+  static __device__ __forceinline__ Term1 term(float td, float rd, float t0, float fs, float lim, unsigned soff,
+                                               unsigned zero) {
+    const float d = term_index(td, rd, t0, fs);
+    Term1 t;
+    t.b = __builtin_amdgcn_fractf(d);
+    const int n0 = (int)d;
+    t.la = ((unsigned)n0 << kShift) + soff;
+    t.ok = true;
+    if (CHK) {
+      t.ok = d >= 1.0f && d < lim;
+      t.la = t.ok ? t.la : zero;  // in the buffer, whatever is there
+    }
+    return t;
+  }
+
+  struct Samples {
+    f4v lo, hi;
+  };
+  static __device__ __forceinline__ Samples fetch(unsigned la, int row) {
+    Samples s;
+    const unsigned a = la + (unsigned)(row * kRowBytes);
+    if (kDelta) {
+      s.lo = *reinterpret_cast<lds_f4*>((size_t)a);
+      s.hi = s.lo;
+    } else {
+      const f4a8 v = *reinterpret_cast<lds_f4a8*>((size_t)a);
+      s.lo = f4v{v.x, v.y, v.z, v.w};
+      if (SM == SM_CUBIC) {
+        const f4a8 u = *reinterpret_cast<lds_f4a8*>((size_t)a + 16);
+        s.hi = f4v{u.x, u.y, u.z, u.w};
+      } else {
+        s.hi = s.lo;
+      }
+    }
+    return s;
+  }
+  static __device__ __forceinline__ float2 interp(const Samples& s, float b, const float (&k)[4]) {
+    if (kDelta) return make_float2(fmaf(b, s.lo.z, s.lo.x), fmaf(b, s.lo.w, s.lo.y));
+    if (SM == SM_LINEAR) return make_float2(fmaf(b, s.lo.z - s.lo.x, s.lo.x), fmaf(b, s.lo.w - s.lo.y, s.lo.y));
+    return make_float2(fmaf(k[3], s.hi.z, fmaf(k[2], s.hi.x, fmaf(k[1], s.lo.z, k[0] * s.lo.x))),
+                       fmaf(k[3], s.hi.w, fmaf(k[2], s.hi.y, fmaf(k[1], s.lo.w, k[0] * s.lo.y))));
+  }
+
+  // das_c's weight of a term (das_c.cpp:372-387)
+  static __device__ __forceinline__ void exact_weight(float td, float rd, float ta, float ra, float wd, float& wr,
+                                                      float& wi) {
+#pragma clang fp contract(off)
+    const float c_apo = ta * ra;
+    wr = c_apo;
+    wi = 0.0f;
+    if (PH == PH_DASC) {
+      float sv, cv;
+      sincosf(wd * (td + rd), &sv, &cv);
+      wr = cv * c_apo;
+      wi = sv * c_apo;
+    }
+  }
+  static __device__ __forceinline__ float2 exact_value(const Samples& s, float b, const float (&k)[4], float wr,
+                                                       float wi) {
+#pragma clang fp contract(off)
+    if (SM == SM_LINEAR) {
+      ustbx::Term t;
+      t.a = 1.0f - b;
+      t.b = b;
+      t.wr = wr;
+      t.wi = wi;
+      return dasc_contrib(t, make_float4(s.lo.x, s.lo.y, s.lo.z, s.lo.w));  // das_c.cpp:389-399
+    }
+    const float2 sm = interp(s, b, k);
+    return make_float2(wr * sm.x - wi * sm.y, wr * sm.y + wi * sm.x);
+  }
+
+  static __device__ __forceinline__ void run(const WinArgs& A, char* smem) {
+    const int lane = threadIdx.x & 63;
+    const int lid = threadIdx.x & 255;
+    const int wave = __builtin_amdgcn_readfirstlane(lid >> 6);
+    const int g = CG > 1 ? __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 8) : 0;
+    const WinTiles& T = A.T;
+    const int tile = __builtin_amdgcn_readfirstlane(T.order[xcd_tile((int)blockIdx.x, (int)gridDim.x)]);
+    const int f0 = (int)blockIdx.y * FT;
+    const int nfr = min(FT, A.F - f0);
+    const size_t PS = (size_t)A.P;
+
+    // this lane's pixel; lanes past the scan's edge take the nearest pixel
+    // (their terms are computed like the others', their results dropped)
+    const int tz = tile % T.ntz, tg = tile / T.ntz;
+    const int gx = tg % T.nlx, gy = tg / T.nlx;
+    const int zl = T.zl, lb = T.lxb + T.lyb;
+    const int dz = (lid & ((1 << zl) - 1)) | ((lid >> (zl + lb)) << zl);
+    const int line = (lid >> zl) & ((1 << lb) - 1);
+    const int iz = (tz << T.dzb) + dz, ix = (gx << T.lxb) + (line & ((1 << T.lxb) - 1)),
+              iy = (gy << T.lyb) + (line >> T.lxb);
+    const bool act = iz < T.n0 && ix < T.n1 && iy < T.n2;
+    const int p = min(iz, T.n0 - 1) + T.n0 * (min(ix, T.n1 - 1) + T.n1 * min(iy, T.n2 - 1));
+
+    const int nw = __builtin_amdgcn_readfirstlane(T.nw[tile]);
+    const int nc = __builtin_amdgcn_readfirstlane(T.nc[tile]);
+    const int4* __restrict__ wl = T.wl + (size_t)tile * A.W;
+    const int4* __restrict__ cl = T.cl + (size_t)tile * A.N;
+    const float t0 = A.t0, fs = A.fs, wd = A.wd;
+    const int ilim = A.L - (SM == SM_LINEAR ? 1 : 2);
+    const float lim = (float)ilim;
+    const float2 refp = A.ref ? A.ref[p] : make_float2(1.0f, 0.0f);
+    const unsigned lds0 = (unsigned)(size_t)(__attribute__((address_space(3))) char*)smem + (unsigned)(g * 2 * kBufBytes);
+    const unsigned lane8 = (unsigned)lane * 8u;
+
+    // channel steps of this group: s = q, q + Q, ...
+    const int Q = CG * (int)gridDim.z, q = (int)blockIdx.z * CG + g;
+    const int steps = (nc + NCH - 1) / NCH;
+    const int nit = (steps + Q - 1) / Q;  // the same for every group (they share the barriers)
+
+    constexpr int kAF = MODE == MODE_NONE ? 1 : FT;
+    constexpr bool kT = !(MODE == MODE_RX && kSep);  // the transmit weight is held per wave
+    float2 acc[kAF][kAcc];
+    static_for<kAF>([&](auto f) { static_for<kAcc>([&](auto j) { acc[f][j] = make_float2(0.0f, 0.0f); }); });
+
+    for (int k0 = 0; k0 < nw; k0 += WC) {
+      const int nj = min(WC, nw - k0);
+      float td[WC];
+      float2 Tw[kT ? WC : 1];  // T, or {ta, -} in the exact phases
+      int alo[WC];             // scalars
+      int amin = 0x3fffffff, amax = -0x3fffffff, all_t = 1;
+      static_for<WC>([&](auto j) {
+        td[j] = kFar;
+        alo[j] = 0;
+        if constexpr (kT) Tw[j] = make_float2(0.0f, 0.0f);
+        // slots past the round's waves repeat the last one with weight zero
+        // (their rows are staged as zeros)
+        const int4 e = scalar_int4(wl + k0 + min((int)j, nj - 1));
+        alo[j] = e.y;
+        all_t &= e.w;
+        if (e.w & 2) {
+          amin = min(amin, e.y);
+          amax = max(amax, e.z);
+        }
+        const float4 v = A.tx[(size_t)e.x * PS + p];
+        if (v.y != 0.0f) {
+          td[j] = v.x;
+          if constexpr (kT) {
+            if (j < nj) Tw[j] = kSep ? make_float2(v.z, v.w) : make_float2(v.y, 0.0f);
+          }
+        }
+      });
+      const int njs = (nj + WSUB - 1) / WSUB, nfs = (nfr + FCK - 1) / FCK;
+      if constexpr (MODE == MODE_RX)
+        static_for<kAF>([&](auto f) { static_for<kAcc>([&](auto j) { acc[f][j] = make_float2(0.0f, 0.0f); }); });
+
+      // windows of step (channel step s, frame chunk fc, wave sub-chunk jc)
+      float2 st[kPer][kLd];
+      auto stage_load = [&](int s, int fc, int jc) {
+        static_for<kPer>([&](auto i) {
+          const int r = wave + 4 * i;
+          const int c = r / (WSUB * FCK), rem = r - c * (WSUB * FCK);
+          const int j = jc * WSUB + rem / FCK, f = fc * FCK + rem % FCK;
+          const int ci = s * NCH + c;
+          static_for<kLd>([&](auto h) { st[i][h] = make_float2(0.0f, 0.0f); });
+          if ((kRows % 4 == 0 || r < kRows) && j < nj && f < nfr && ci < nc) {
+            const int4 we = scalar_int4(wl + k0 + j), ce = scalar_int4(cl + ci);
+            const int base = we.y + ce.y - 1 - WinSpan<SM>::kBack;
+            const int cnt = (we.z - we.y) + (ce.z - ce.y) + WinSpan<SM>::kSlack;
+            const __amdgpu_buffer_rsrc_t rs =
+                make_rsrc((const char*)A.ch + (size_t)(f0 + f) * (size_t)A.frame_bytes, A.frame_bytes);
+            const unsigned off = (unsigned)((we.x * A.N + ce.x) * A.L + base) * 8u + lane8;
+            static_for<kLd>([&](auto h) {
+              if (h == 0 || cnt > 64 * h)  // uniform
+                st[i][h] = buf_load8(rs, lane + 64 * h < cnt ? (int)(off + 512u * h) : kOOB);
+            });
+          }
+        });
+      };
+      auto stage_store = [&](int buf) {
+        static_for<kPer>([&](auto i) {
+          const int r = wave + 4 * i;
+          if (kRows % 4 == 0 || r < kRows) {
+            const unsigned a = lds0 + (unsigned)(buf * kBufBytes + r * kRowBytes) + ((unsigned)lane << kShift);
+            if constexpr (kDelta) {
+              const float2 x = st[i][0];
+              const float nx = next_lane(x.x), ny = next_lane(x.y);
+              *reinterpret_cast<lds_f4w*>((size_t)a) = f4v{x.x, x.y, nx - x.x, ny - x.y};
+            } else {
+              static_for<kLd>([&](auto h) {
+                *reinterpret_cast<lds_f2*>((size_t)a + 512 * h) = f2v{st[i][h].x, st[i][h].y};
+              });
+            }
+          }
+        });
+      };
+      // receive entries of the step's channels
+      float4 rv[NCH];
+      static_for<NCH>([&](auto c) { rv[c] = make_float4(0.f, 0.f, 0.f, 0.f); });
+      auto rx_load = [&](int s) {
+        static_for<NCH>([&](auto c) {
+          rv[c] = make_float4(0.f, 0.f, 0.f, 0.f);
+          if (s * NCH + c < nc)
+            rv[c] = rx_entry_t<kCompact>(A.rx, (size_t)scalar_int4(cl + s * NCH + c).x * PS + p);
+        });
+      };
+
+      // the terms of channel c (list entry ce) in sub-chunk jc, frame chunk fc
+      auto compute = [&](auto chk, auto c, auto jc, auto fc, int n, int blo, int buf, float rd, float2 R, float ra,
+                         float2(&part)[NCH][FCK]) {
+        constexpr bool CHK = decltype(chk)::value;
+        constexpr int C = decltype(c)::value, JC = decltype(jc)::value, FC = decltype(fc)::value;
+        const unsigned bufo = lds0 + (unsigned)(buf * kBufBytes);
+        // batches of kB waves: their samples are all asked for before the first
+        // is used
+        constexpr int kB = WSUB * FCK <= 4 ? WSUB : (FCK >= 4 ? 1 : 4 / FCK);
+        static_assert(WSUB % kB == 0, "whole batches");
+        static_for<WSUB / kB>([&](auto gr) {
+          constexpr int J0 = JC * WSUB + kB * decltype(gr)::value;
+          Term1 t[kB];
+          Samples sm[kB][FCK];
+          static_for<kB>([&](auto u) {
+            constexpr int J = J0 + decltype(u)::value, jj = J - JC * WSUB;
+            unsigned soff = bufo + (unsigned)((C * WSUB * FCK + jj * FCK) * kRowBytes) -
+                            (unsigned)((alo[J] + blo - 1) << kShift);
+            asm("" : "+s"(soff));  // one scalar operand of the address
+            t[u] = term<CHK>(td[J], rd, t0, fs, lim, soff, bufo);
+            static_for<FCK>([&](auto f) { sm[u][f] = fetch(t[u].la, f); });
+          });
+          __builtin_amdgcn_sched_barrier(0);
+          static_for<kB>([&](auto u) {
+            constexpr int J = J0 + decltype(u)::value;
+            float kw[4] = {0.f, 0.f, 0.f, 0.f};
+            if constexpr (SM == SM_CUBIC) keys_weights_horner(t[u].b, kw[0], kw[1], kw[2], kw[3]);
+            float wr = 0.0f, wi = 0.0f;
+            if constexpr (!kSep) exact_weight(t[u].ok ? td[J] : 0.0f, t[u].ok ? rd : 0.0f, Tw[J].x, ra, wd, wr, wi);
+            static_for<FCK>([&](auto f) {
+              if constexpr (MODE == MODE_BOTH) {
+                float2 v = part[C][f];
+                cfma(v, Tw[J], interp(sm[u][f], t[u].b, kw));
+                part[C][f] = !CHK || t[u].ok ? v : part[C][f];
+              } else if constexpr (MODE == MODE_RX) {
+                float2 v = acc[FC * FCK + f][J];
+                if constexpr (kSep) cfma(v, R, interp(sm[u][f], t[u].b, kw));
+                else cadd(v, exact_value(sm[u][f], t[u].b, kw, wr, wi));
+                acc[FC * FCK + f][J] = !CHK || t[u].ok ? v : acc[FC * FCK + f][J];
+              } else {
+                float2 v;
+                if constexpr (kSep) v = cmul(cmul(R, Tw[J]), interp(sm[u][f], t[u].b, kw));
+                else v = exact_value(sm[u][f], t[u].b, kw, wr, wi);
+                if (CHK && !t[u].ok) v = make_float2(0.0f, 0.0f);
+                if (A.ref) v = cmul(v, refp);
+                const int ff = FC * FCK + f;
+                if (act && J < nj && ff < nfr) {
+                  const int w = scalar_int4(wl + k0 + J).x;
+                  A.out[(((size_t)(f0 + ff) * A.W + w) * A.N + n) * PS + p] = v;
+                }
+              }
+            });
+          });
+          __builtin_amdgcn_sched_barrier(0);
+        });
+      };
+
+      int buf = 0;
+      if (q < steps) {
+        stage_load(q, 0, 0);
+        stage_store(0);
+        rx_load(q);
+      }
+      __syncthreads();
+      for (int it = 0; it < nit; ++it) {
+        const int s = q + it * Q;
+        const bool live = s < steps;  // wave-uniform
+        static_for<kNF>([&](auto fc) {
+          if (fc < nfs) {
+            float2 part[NCH][FCK];
+            static_for<NCH>([&](auto c) { static_for<FCK>([&](auto f) { part[c][f] = make_float2(0.0f, 0.0f); }); });
+            static_for<kNS>([&](auto jc) {
+              if (jc < njs) {
+                // the next step
+                int ns = s, nf = fc, nj2 = jc + 1;
+                if (nj2 >= njs) {
+                  nj2 = 0;
+                  if (++nf >= nfs) {
+                    nf = 0;
+                    ns = s + Q;
+                  }
+                }
+                const bool more = ns < steps;
+                if (more) stage_load(ns, nf, nj2);
+                if (live) {
+                  static_for<NCH>([&](auto c) {
+                    const int ci = s * NCH + c;
+                    if (ci < nc) {
+                      const int4 ce = scalar_int4(cl + ci);
+                      const bool ron = rv[c].y != 0.0f;
+                      const float2 R = ron ? make_float2(rv[c].z, rv[c].w) : make_float2(0.0f, 0.0f);
+                      // every term of the channel in the sample window, every
+                      // weight nonzero (dimension both drops the sums of the
+                      // lanes with no receive weight below)
+                      const bool dense = (all_t & 1) && (MODE == MODE_BOTH || (ce.w & 1)) && amin + ce.y - 1 >= 1 &&
+                                         amax + ce.z + 2 < ilim;
+                      if (dense)
+                        compute(std::false_type(), c, jc, fc, ce.x, ce.y, buf, rv[c].x, R, rv[c].y, part);
+                      else
+                        compute(std::true_type(), c, jc, fc, ce.x, ce.y, buf, ron ? rv[c].x : kFar, R, rv[c].y, part);
+                    }
+                  });
+                }
+                if constexpr (MODE == MODE_BOTH) {
+                  if (live && jc + 1 >= njs)
+                    static_for<NCH>([&](auto c) {
+                      const bool ron = rv[c].y != 0.0f;
+                      static_for<FCK>([&](auto f) {
+                        float2 v = acc[fc * FCK + f][0];
+                        cfma(v, make_float2(rv[c].z, rv[c].w), part[c][f]);
+                        acc[fc * FCK + f][0] = ron ? v : acc[fc * FCK + f][0];
+                      });
+                    });
+                }
+                if (more && ns != s) rx_load(ns);
+                if (more) stage_store(buf ^ 1);
+                __syncthreads();
+                buf ^= 1;
+              }
+            });
+          }
+        });
+      }
+
+      if constexpr (MODE == MODE_RX) {
+        // out[f][w][p] = T * sum (the exact phases: the sum)
+        static_for<kAcc>([&](auto j) {
+          if (j < nj) {
+            const int w = scalar_int4(wl + k0 + j).x;
+            float2 Tj = make_float2(0.0f, 0.0f);
+            if constexpr (kSep) {
+              const float4 v = A.tx[(size_t)w * PS + p];
+              if (v.y != 0.0f) Tj = make_float2(v.z, v.w);
+            }
+            static_for<FT>([&](auto f) {
+              if (f < nfr) {
+                float2 v = group_sum(acc[f][j], smem, g, lid);
+                if constexpr (kSep) v = cmul(Tj, v);
+                if (A.ref) v = cmul(v, refp);
+                if (act && g == 0) A.out[((size_t)(f0 + f) * A.W + w) * PS + p] = v;
+              }
+            });
+          }
+        });
+      }
+    }  // round
+
+    if constexpr (MODE == MODE_BOTH)
+      static_for<FT>([&](auto f) {
+        if (f < nfr) {
+          float2 v = group_sum(acc[f][0], smem, g, lid);
+          if (A.ref) v = cmul(v, refp);
+          if (act && g == 0) A.out[(size_t)(f0 + f) * PS + p] = v;
+        }
+      });
+  }
+
+  // The channel groups' sums in group order (group 0 gets them).
+  static __device__ __forceinline__ float2 group_sum(float2 v, char* smem, int g, int lid) {
+    if constexpr (CG > 1) {
+      float2* red = reinterpret_cast<float2*>(smem);
+      red[threadIdx.x] = v;
+      __syncthreads();
+      if (g == 0)
+        static_for<CG - 1>([&](auto k) { cadd(v, red[(k + 1) * 256 + lid]); });
+      __syncthreads();
+    }
+    return v;
+  }
+};
+
+template <int SM, int MODE, int PH, int ROW, int WC, int WSUB, int FT, int FCK, int NCH, int CG>
+__global__ __launch_bounds__(256 * CG, 4) void das_window_kernel(WinArgs A) {
+  using K = WinKernel<SM, MODE, PH, ROW, WC, WSUB, FT, FCK, NCH, CG>;
+  __shared__ __align__(16) char smem[K::kSmem];
+  K::run(A, smem);
+}
+
+// Channel groups per tile: blocks of 1024 threads (or, in dimension none,
+// more blocks per tile) where the tiles alone leave the chip idle.
+template <int SM, int MODE, int PH, int ROW, int WC, int WSUB, int FT, int FCK, int NCH, int CG>
+static hipError_t launch_window_t(const GeomLaunch& G, int zsplit, hipStream_t stream) {
+  WinArgs A;
+  A.ch = G.ch;
+  A.out = reinterpret_cast<float2*>(G.out);
+  A.tx = G.tx_table;
+  A.rx = G.win_rx;
+  A.ref = G.ref_phase ? G.win_ref : nullptr;
+  A.T = G.win;
+  A.P = G.P;
+  A.N = G.N;
+  A.W = G.W;
+  A.L = G.L;
+  A.F = G.F;
+  A.t0 = G.t0;
+  A.fs = G.fs;
+  A.wd = G.wd;
+  A.frame_bytes = G.L * G.N * G.W * 8;
+  hipLaunchKernelGGL((das_window_kernel<SM, MODE, PH, ROW, WC, WSUB, FT, FCK, NCH, CG>),
+                     dim3((unsigned)G.win.tiles, (unsigned)((G.F + FT - 1) / FT), (unsigned)zsplit), dim3(256 * CG), 0,
+                     stream, A);
+  return hipGetLastError();
+}
+
+hipError_t launch_window_rx(const GeomLaunch& G, int ph, hipStream_t stream);
+hipError_t launch_window_none(const GeomLaunch& G, int ph, hipStream_t stream);
+hipError_t launch_window_both(const GeomLaunch& G, hipStream_t stream);
+
+}  // namespace ustbx
