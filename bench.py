@@ -855,7 +855,7 @@ def run_batch(args, torch, dev):
         p.set_tiles(*best)
         ref = p.run(chs[i])
         bitwise = bitwise and bool(torch.equal(ref, outs[i]))
-        p.set_tiles(v[1], v[2])
+        autotune.apply(p, v)
     units = wl.units
     act_k = {k: plans[k].active_terms() for k in set(k for k, _ in wl.acquisitions)}
     act = sum(act_k[k] for k, _ in wl.acquisitions)
@@ -957,7 +957,7 @@ def run_serve(args, torch, dev):
         v = p.variant
         p.set_tiles(*srv.tiles)
         alone = p.run(torch.from_numpy(datasets[r.config][r.data]).to(dev)).cpu().numpy()
-        p.set_tiles(v[1], v[2])
+        autotune.apply(p, v)
         same = same and bool(np.array_equal(alone, mixed.outputs[r.rid]))
         q = plain_chk.outputs[r.rid]
         err = max(err, float(np.max(np.abs(q - alone)) / max(np.max(np.abs(alone)), 1e-30)))

@@ -328,7 +328,12 @@ int ustbx_plan_set_staging(ustbx_plan* plan, int32_t on, ustbx_status* st);
  * transmit) that the plan marked for staging, and all pairs of the tiles'
  * channel lists (0, 0 otherwise). */
 int ustbx_plan_stage_stats(const ustbx_plan* plan, int64_t* staged, int64_t* listed, ustbx_status* st);
-/* Current variant (or -1 for NULL) and its tile shape. */
+/* Current variant (or -1 for NULL) and its tile shape: 0 and 0 where the
+ * library runs the plan on patch tiles with LDS-staged sample windows
+ * (dimension both on variant 2 while no tile shape was set; 9 or more waves
+ * and a few hundred tiles). Setting a tile shape selects the gathering kernel
+ * of that shape. Dimension receive and none use patch tiles wherever the scan
+ * and the weights allow, under variant 0. */
 int32_t ustbx_plan_variant(const ustbx_plan* plan, int32_t* wave_chunk, int32_t* split);
 
 /* ---------------------------------------------------------------------------
@@ -337,7 +342,8 @@ int32_t ustbx_plan_variant(const ustbx_plan* plan, int32_t* wave_chunk, int32_t*
  * ------------------------------------------------------------------------ */
 typedef struct ustbx_batch ustbx_batch;
 
-/* count acquisitions, acquisition i beamformed with plans[i] (a plan may be
+/* (Equality with a plan's own run: of a plan whose tile shape was set.)
+ * count acquisitions, acquisition i beamformed with plans[i] (a plan may be
  * listed more than once; every plan must have variant-2 state -- see
  * ustbx_plan_set_variant -- and all share one interpolation). Dimension both;
  * each image equals ustbx_plan_run of its plan with the same tile shape, bit

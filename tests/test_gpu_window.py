@@ -110,3 +110,56 @@ def test_samples_outside_the_weights_stay_out(cuda, dim):
     plan.close()
     ref = O.beamform_fp64(ch, 10.4e6, 0.0, ta, ra, td, rd, 5.2e6, dim, w0=O.dasc_wd(5.2e6), index="fp32")
     assert np.array_equal(np.isnan(got), np.isnan(ref)) and np.isnan(ref).any()
+
+
+BOTH = [
+    # kind, W, nx, nz, F, rf, cubic, L: at least 512 blocks of 256 pixels (x 2 frames)
+    ("linear", 9, 300, 450, 1, False, False, 512),
+    ("linear", 13, 131, 333, 7, True, False, 500),    # traces end inside the image
+    ("linear", 33, 301, 470, 1, False, False, 420),
+    ("sector", 17, 200, 331, 5, False, True, 512),
+    ("volume", 26, 60, 170, 3, False, False, 400),
+]
+
+
+@pytest.mark.parametrize("rx", [TUKEY, BOX], ids=["tukey", "boxcar"])
+@pytest.mark.parametrize("kind,W,nx,nz,F,rf,cubic,L", BOTH)
+def test_both_against_set_tiles(cuda, kind, W, nx, nz, F, rf, cubic, L, rx):
+    """Dimension both on the library's choice (staged windows) against the
+    gathering kernel of a set tile shape, with non-finite samples that only
+    zero weights meet somewhere; both sum the same FP32 terms in another order."""
+    print(f"case window both {kind} W={W} F={F} cubic={cubic}", flush=True)
+    prb, scan, seq = _setup(kind, W, nx, nz, 25e-3 if kind != "volume" else 14e-3)
+    fs, fd = (20.8e6, 0.0) if rf else (10.4e6, 5.2e6)
+    # plane waves: one weight per wave; sector: tiles partly outside the waves' cones
+    tx = {"linear": Apodization(Window.tukey25, f_number=1.5), "sector": Apodization(Window.boxcar, f_number=0.7),
+          "volume": Apodization()}[kind]
+    plan = make_plan(prb, scan, seq, n_samples=L, n_frames=F, sampling_frequency=fs, initial_time=0.0,
+                     modulation_frequency=fd, sound_speed=C, receive_apodization=rx, transmit_apodization=tx,
+                     dimension=3, interpolation=int(cubic), reference_phase=not rf)
+    assert plan.variant == (2, 0, 0)
+    g = torch.Generator(cuda).manual_seed(W)
+    ch = torch.randn((F, W, prb.N_elements, L), dtype=torch.complex64, device=cuda, generator=g)
+    ch[0, :, 2, 60:70] = float("nan")
+    got = plan.run(ch)
+    plan.set_tiles(8, 4)
+    assert plan.variant == (2, 8, 4)
+    ref = plan.run(ch)
+    plan.close()
+    a, b = torch.view_as_real(got), torch.view_as_real(ref)
+    assert torch.equal(torch.isnan(a), torch.isnan(b))
+    # sums of at most 33 x 21 FP32 terms in another order: sqrt(700) * 6e-8 of
+    # the RMS sum, ten times that of the peak
+    assert (torch.nan_to_num(a - b).abs().max() / torch.nan_to_num(b).abs().max()).item() <= 5e-6
+
+
+def test_both_keeps_small_plans_on_the_gathering_kernel(cuda):
+    prb, scan, seq = _setup("linear", 4, 300, 500)
+    kw = dict(n_samples=512, n_frames=1, sampling_frequency=10.4e6, initial_time=0.0, modulation_frequency=5.2e6,
+              sound_speed=C, receive_apodization=TUKEY, dimension=3)
+    few_waves = make_plan(prb, scan, seq, **kw)
+    prb, scan, seq = _setup("linear", 12, 40, 64)
+    few_tiles = make_plan(prb, scan, seq, **kw)
+    assert few_waves.variant[1:] != (0, 0) and few_tiles.variant[1:] != (0, 0)
+    few_waves.close()
+    few_tiles.close()

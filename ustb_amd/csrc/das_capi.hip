@@ -738,12 +738,13 @@ bool coef_build(ustbx_plan* pl, hipError_t& err) {
   return true;
 }
 
-// The window-staged kernels (das_window.h) cover dimension receive and none on
-// linear and sector scans with das_c's edge rule, frames below 2 GiB, every
-// nonzero weight and every delay finite, and scans fine enough that a patch
-// tile's windows fit an LDS row. Their receive table may take this fraction of
-// the device memory; where it cannot be had the per-lane kernel runs, as for
-// every other plan.
+// The window-staged kernels (das_window.h) cover dimension receive and none,
+// and dimension both with the resident receive table, on linear and sector
+// scans with das_c's edge rule, frames below 2 GiB, every nonzero weight and
+// every delay finite, and scans fine enough that a patch tile's windows fit an
+// LDS row. The receive table of dimension receive and none may take this
+// fraction of the device memory; where it cannot be had the per-lane kernel
+// runs, as for every other plan.
 constexpr double kWindowTableMaxFraction = 0.125;
 
 void window_free(ustbx_plan* pl) {
@@ -761,15 +762,16 @@ void window_free(ustbx_plan* pl) {
 bool window_build(ustbx_plan* pl, hipError_t& err) {
   err = hipSuccess;
   GeomLaunch& G = pl->G;
-  if (!(G.dim == 0 || G.dim == 1)) return true;
+  const bool both = G.dim == 3;
+  if (!(G.dim == 0 || G.dim == 1 || (both && pl->rxtab_state > 0 && !G.rx_otf))) return true;
   if (!(G.scan.kind == SCAN_LINEAR || G.scan.kind == SCAN_SECTOR)) return true;
   if (G.edge == USTBX_EDGE_PYTHON && G.interp == USTBX_INTERP_LINEAR) return true;
   if ((int64_t)G.L * G.N * G.W * 8 > 0x7FFFFE00 || G.L < 4) return true;
   G.rx_compact = G.wd == 0.0f ? 1 : 0;
   const size_t P = (size_t)G.P;
   auto al = [](size_t b) { return (b + 255) & ~size_t(255); };
-  const size_t b_rx = al((G.rx_compact ? sizeof(float2) : sizeof(float4)) * (size_t)G.N * P);
-  const size_t b_ref = G.ref_phase ? al(sizeof(float2) * P) : 0;
+  const size_t b_rx = both ? 0 : al((G.rx_compact ? sizeof(float2) : sizeof(float4)) * (size_t)G.N * P);
+  const size_t b_ref = !both && G.ref_phase ? al(sizeof(float2) * P) : 0;
   size_t free_b = 0, total_b = 0;
   if (hipMemGetInfo(&free_b, &total_b) != hipSuccess) return true;
   if (b_rx > (size_t)(kWindowTableMaxFraction * (double)total_b)) return true;
@@ -793,6 +795,11 @@ bool window_build(ustbx_plan* pl, hipError_t& err) {
   }
   std::stable_partition(shapes.begin(), shapes.end(), [&](const Shape& s) { return s.padded <= least + least / 10; });
   if (least > 2 * P + 1024) return true;  // a scan of a few lines or depths
+  // dimension both: no tables for a plan that the gathering kernel runs anyway
+  // (window_both_active)
+  if (both && (G.W < 9 || (G.interp == USTBX_INTERP_CUBIC && G.F == 1) ||
+               (int64_t)(least >> 8) * ((G.F + 1) / 2) < 512))
+    return true;
 
   size_t tiles_max = 0;
   for (const Shape& s : shapes) tiles_max = std::max(tiles_max, s.padded >> 8);
@@ -810,7 +817,7 @@ bool window_build(ustbx_plan* pl, hipError_t& err) {
     off += b;
     return q;
   };
-  float4* rx = (float4*)take(b_rx);
+  float4* rx = b_rx ? (float4*)take(b_rx) : nullptr;
   float2* ref = b_ref ? (float2*)take(b_ref) : nullptr;
   int4* wl = (int4*)take(b_wl);
   int4* cl = (int4*)take(b_cl);
@@ -818,8 +825,8 @@ bool window_build(ustbx_plan* pl, hipError_t& err) {
   int* nc = (int*)take(b_cnt);
   int* ord = (int*)take(b_cnt);
   int* info = (int*)take(b_info);
-  err = launch_window_state(G, rx, ref, nullptr);
-  G.win_rx = rx;
+  if (!both) err = launch_window_state(G, rx, ref, nullptr);
+  G.win_rx = both ? G.rx_table : rx;
   G.win_ref = ref;
   pl->win_mem = m;
   pl->win_bytes = total;
@@ -842,12 +849,12 @@ bool window_build(ustbx_plan* pl, hipError_t& err) {
     for (int i = 0; i < 8; ++i) h[i] = 0;
     if (err == hipSuccess) err = hipMemcpy(info, h, sizeof(int) * 8, hipMemcpyHostToDevice);
     // dimension none writes every (wave, channel), receive every wave
-    if (err == hipSuccess) err = launch_window_lists(G, nw, nc, wl, cl, info, 1, G.dim == 0, nullptr);
+    if (err == hipSuccess) err = launch_window_lists(G, nw, nc, wl, cl, info, !both, G.dim == 0, nullptr);
     if (err == hipSuccess) err = hipMemcpy(h, info, sizeof(int) * 8, hipMemcpyDeviceToHost);
     return err == hipSuccess;
   };
   const int slack = G.interp == USTBX_INTERP_CUBIC ? 7 : 5;  // WinSpan::kSlack
-  int best = -1, best_span = 129, last = -1;
+  int best = -1, best_span = 129, last = -1, max_nw = 0;
   for (int k = 0; k < (int)shapes.size(); ++k) {
     int h[8];
     if (!lists(shapes[k], h)) {
@@ -855,6 +862,7 @@ bool window_build(ustbx_plan* pl, hipError_t& err) {
       return false;
     }
     last = k;
+    max_nw = std::max(max_nw, h[2]);
     if (h[1]) break;  // weights or delays that are not finite: the per-lane kernel
     if (h[0] + slack < best_span) {
       best = k;
@@ -881,6 +889,8 @@ bool window_build(ustbx_plan* pl, hipError_t& err) {
     T.wl = wl;
     T.cl = cl;
     T.on = 1;
+    G.win_max_nw = max_nw;
+    if (both) G.win_rx = nullptr;  // the plan's receive table, which may be rebuilt
     return true;
   }
   window_free(pl);
@@ -1375,6 +1385,7 @@ int ustbx_plan_create(const ustbx_geometry* g, ustbx_plan** plan, ustbx_status* 
     G.otf.oxf = (float)a.ox;
     G.otf.oyf = (float)a.oy;
   }
+  G.auto_tiles = 1;
   if (rxtab_build(pl, e, otf_default(pl))) {
     G.variant = 2;
     rxtab_defaults(G, pl->max_nw, G.wave_chunk, G.split);
@@ -1411,6 +1422,7 @@ int ustbx_plan_set_variant(ustbx_plan* plan, int32_t variant, ustbx_status* st) 
     }
     if (plan->G.variant != 2) {
       plan->G.variant = 2;
+      plan->G.auto_tiles = 1;
       rxtab_defaults(plan->G, plan->max_nw, plan->G.wave_chunk, plan->G.split);
     }
     return ok(st);
@@ -1437,6 +1449,7 @@ int ustbx_plan_set_variant(ustbx_plan* plan, int32_t variant, ustbx_status* st) 
   const bool same_family = variant >= 2 && plan->G.variant >= 2;
   plan->G.variant = variant;
   if (same_family) return ok(st);
+  plan->G.auto_tiles = 1;
   if (variant >= 2) {
     rxtab_defaults(plan->G, plan->max_nw, plan->G.wave_chunk, plan->G.split);
   } else if (variant == 1) {
@@ -1463,6 +1476,7 @@ int ustbx_plan_set_tiles(ustbx_plan* plan, int32_t wave_chunk, int32_t split, us
       return set_status(st, USTBX_E_ARG, "waves per split must be 4, 5, 6, 8, 10, 12 or 16");
     if (split && split != 4 && split != 5 && split != 8)
       return set_status(st, USTBX_E_ARG, "wave-splits per block must be 4, 5 or 8");
+    if (wave_chunk || split) plan->G.auto_tiles = 0;
     if (wave_chunk) plan->G.wave_chunk = wave_chunk;
     if (split) plan->G.split = split;
     return ok(st);
@@ -1682,8 +1696,9 @@ int ustbx_plan_stage_stats(const ustbx_plan* plan, int64_t* staged, int64_t* lis
 
 int32_t ustbx_plan_variant(const ustbx_plan* plan, int32_t* wave_chunk, int32_t* split) {
   if (!plan) return -1;
-  if (wave_chunk) *wave_chunk = plan->G.wave_chunk;
-  if (split) *split = plan->G.split;
+  const bool window = window_both_active(plan->G);  // the library's choice, no tile shape
+  if (wave_chunk) *wave_chunk = window ? 0 : plan->G.wave_chunk;
+  if (split) *split = window ? 0 : plan->G.split;
   return (plan->G.variant == 2 && plan->G.rx_otf) ? 4 : plan->G.variant;
 }
 

@@ -118,9 +118,12 @@ struct GeomLaunch {
   // 4 = patches of 16 depths x 4 scan lines (dimension transmit on a linear
   // or sector scan whose axes divide evenly). Fixed when the plan is made.
   int tile_ps;
-  // Window-staged kernels (das_window.h), where win.on: receive table and
-  // reference phase they read.
+  // Window-staged kernels (das_window.h), where win.on; dimension both reads
+  // rx_table and ref_table and takes them while no tile shape is set
+  // (auto_tiles), the other modes win_rx and win_ref.
   WinTiles win;
+  int win_max_nw;        // largest wave count of a tile
+  int auto_tiles;
   const float4* win_rx;
   const float2* win_ref;
   // Stage sample windows through LDS (1) or gather every term's samples
@@ -128,6 +131,20 @@ struct GeomLaunch {
   // per (channel, wave). Results do not depend on it.
   int stage;
 };
+
+// Whether a dimension-both plan runs window-staged: while no tile shape is
+// set, with enough waves per staged window's receive entry and enough blocks
+// to fill the chip, and linear or over several frames. Measured against the
+// gathering kernel over 50 random plans: from 9 waves and 512 blocks (rows of
+// 64 samples) 1.25-3.0 times as fast; 4-8 waves 0.8-1.05, 1-3 waves 0.2-0.9,
+// 60-300 blocks 0.2-0.8 (0.9-1.6 with over 45 waves); one cubic frame of the 75
+// plane waves 2.37 against 2.26 ms. Rows of 128 hold a quarter of the data at
+// twice the LDS per sample pair: twice the blocks.
+inline bool window_both_active(const GeomLaunch& G) {
+  return G.dim == 3 && G.win.on && G.variant == 2 && G.auto_tiles && !G.rx_otf && G.rx_table != nullptr &&
+         (G.interp != INTERP_CUBIC || G.F > 1) && G.win_max_nw >= 9 &&
+         (int64_t)G.win.tiles * ((G.F + 1) / 2) >= (G.win.row == 64 ? 512 : 1024);
+}
 
 // Builds the transmit table of a plan (one lane per (wave, pixel)).
 hipError_t launch_geom_tx_table(const GeomLaunch& g, float4* table, hipStream_t stream);

@@ -20,11 +20,11 @@
 // are inside the sample window (no lane tests anything) one comparison.
 //
 // Loop: rounds of up to WC waves (transmit state in VGPRs) x the tile's
-// channel list x chunks of FCK frames x sub-chunks of WSUB waves; a step
-// stages ROWS = NCH x WSUB x FCK windows (NCH channels at a time where one
-// channel has few waves) while the previous step's are used (two LDS buffers,
-// one barrier per step). The index, the fraction and the weights of a term are
-// formed once for its FCK frames.
+// channel list; a step stages NCH channels' WC x FT windows (FT frames) while
+// the previous step's are used (two LDS buffers, one barrier per step). The
+// index, the fraction and the weights of a term are formed once for its FT
+// frames. A block is one group of 256 threads, or CG x WG groups that share
+// out the channels (CG) and the waves (WG) of one tile.
 //
 // Rows hold 64 samples, or 128 on coarse scans. Linear interpolation with the
 // separable phase keeps {x, x[+1] - x} per sample in rows of 64, so a term
@@ -81,26 +81,25 @@ __device__ __forceinline__ void static_for(const F& f) {
   static_for_seq(f, std::make_integer_sequence<int, N>());
 }
 
-template <int SM, int MODE, int PH, int ROW, int WC, int WSUB, int FT, int FCK, int NCH, int CG>
+template <int SM, int MODE, int PH, int ROW, int WC, int FT, int NCH, int CG, int WG>
 struct WinKernel {
   static_assert(MODE == MODE_BOTH || MODE == MODE_RX || MODE == MODE_NONE, "dimension transmit has its own kernel");
-  static_assert(NCH == 1 || (WSUB == WC && FT == FCK), "several channels per step: one sub-chunk, one frame chunk");
-  static_assert(WC % WSUB == 0 && FT % FCK == 0, "whole sub-chunks");
+  static_assert(WG == 1 || MODE == MODE_BOTH, "wave groups add into one image");
   static constexpr bool kSep = MODE == MODE_BOTH || PH == PH_SEP;  // T and R from the tables
   static_assert(ROW == 64 || ROW == 128, "samples of an LDS row");
   static constexpr bool kDelta = SM == SM_LINEAR && kSep && ROW == 64;
   static constexpr int kLd = ROW / 64;  // loads per row
   static constexpr bool kCompact = PH == PH_RF;
   static constexpr int kShift = kDelta ? 4 : 3;  // log2 bytes per staged sample
-  static constexpr int kRows = NCH * WSUB * FCK;
+  static constexpr int kRows = NCH * WC * FT;    // row (channel, wave, frame), frame fastest
   static constexpr int kRowBytes = ROW << kShift;
   static constexpr int kBufBytes = kRows * kRowBytes;
-  static constexpr int kPer = (kRows + 3) / 4;  // rows a wave stages per step
-  static constexpr int kNF = FT / FCK, kNS = WC / WSUB;
+  static constexpr int kPer = (kRows + 3) / 4;  // rows a wave stages per step: wave + 4 i
   static constexpr int kAcc = MODE == MODE_RX ? WC : 1;
-  static constexpr int kSmem = CG * 2 * kBufBytes;
+  static constexpr int kGroups = CG * WG;
+  static constexpr int kSmem = kGroups * 2 * kBufBytes;
 
-  // One staged term: the index, its row position and whether it counts.
+  // One staged term: its fraction, the LDS address of its samples and whether it counts.
   struct Term1 {
     float b;
     unsigned la;
@@ -184,10 +183,15 @@ struct WinKernel {
     const int lane = threadIdx.x & 63;
     const int lid = threadIdx.x & 255;
     const int wave = __builtin_amdgcn_readfirstlane(lid >> 6);
-    const int g = CG > 1 ? __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 8) : 0;
+    const int g = kGroups > 1 ? __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 8) : 0;
+    const int wgi = g / CG;  // this group's share of the waves
     const WinTiles& T = A.T;
-    const int tile = __builtin_amdgcn_readfirstlane(T.order[xcd_tile((int)blockIdx.x, (int)gridDim.x)]);
-    const int f0 = (int)blockIdx.y * FT;
+    // a tile's frame chunks next to each other on one XCD: they read the same
+    // receive rows at about the same time
+    const int fcs = (A.F + FT - 1) / FT;
+    const int item = xcd_tile((int)blockIdx.x, (int)gridDim.x);
+    const int tile = __builtin_amdgcn_readfirstlane(T.order[item / fcs]);
+    const int f0 = (item % fcs) * FT;
     const int nfr = min(FT, A.F - f0);
     const size_t PS = (size_t)A.P;
 
@@ -201,7 +205,7 @@ struct WinKernel {
     const int iz = (tz << T.dzb) + dz, ix = (gx << T.lxb) + (line & ((1 << T.lxb) - 1)),
               iy = (gy << T.lyb) + (line >> T.lxb);
     const bool act = iz < T.n0 && ix < T.n1 && iy < T.n2;
-    const int p = min(iz, T.n0 - 1) + T.n0 * (min(ix, T.n1 - 1) + T.n1 * min(iy, T.n2 - 1));
+    const unsigned p = (unsigned)(min(iz, T.n0 - 1) + T.n0 * (min(ix, T.n1 - 1) + T.n1 * min(iy, T.n2 - 1)));
 
     const int nw = __builtin_amdgcn_readfirstlane(T.nw[tile]);
     const int nc = __builtin_amdgcn_readfirstlane(T.nc[tile]);
@@ -215,7 +219,7 @@ struct WinKernel {
     const unsigned lane8 = (unsigned)lane * 8u;
 
     // channel steps of this group: s = q, q + Q, ...
-    const int Q = CG * (int)gridDim.z, q = (int)blockIdx.z * CG + g;
+    const int Q = CG * (int)gridDim.z, q = (int)blockIdx.z * CG + g % CG;
     const int steps = (nc + NCH - 1) / NCH;
     const int nit = (steps + Q - 1) / Q;  // the same for every group (they share the barriers)
 
@@ -223,27 +227,35 @@ struct WinKernel {
     constexpr bool kT = !(MODE == MODE_RX && kSep);  // the transmit weight is held per wave
     float2 acc[kAF][kAcc];
     static_for<kAF>([&](auto f) { static_for<kAcc>([&](auto j) { acc[f][j] = make_float2(0.0f, 0.0f); }); });
+    // dimension both, one frame: the sum is closed every 32 steps, so that its
+    // rounding grows with 32 + steps / 32 additions, not with the channels
+    // (1024 of the volume: 4.7e-7 by the gathering kernel's splits, 6.2e-7 in
+    // one running sum)
+    constexpr bool kClose = MODE == MODE_BOTH && FT == 1;
+    float2 tot = make_float2(0.0f, 0.0f);
 
-    for (int k0 = 0; k0 < nw; k0 += WC) {
-      const int nj = min(WC, nw - k0);
+    for (int kr = 0; kr < nw; kr += WG * WC) {
+      const int k0 = __builtin_amdgcn_readfirstlane(kr + wgi * WC);
+      const int nj = __builtin_amdgcn_readfirstlane(min(WC, max(0, nw - k0)));  // this group's waves of the round
       float td[WC];
       float2 Tw[kT ? WC : 1];  // T, or {ta, -} in the exact phases
-      int alo[WC];             // scalars
+      // scalars: of term J, the part of its LDS address that the wave fixes
+      unsigned woff[WC];
       int amin = 0x3fffffff, amax = -0x3fffffff, all_t = 1;
       static_for<WC>([&](auto j) {
         td[j] = kFar;
-        alo[j] = 0;
         if constexpr (kT) Tw[j] = make_float2(0.0f, 0.0f);
-        // slots past the round's waves repeat the last one with weight zero
-        // (their rows are staged as zeros)
-        const int4 e = scalar_int4(wl + k0 + min((int)j, nj - 1));
-        alo[j] = e.y;
+        // slots past the list repeat its last wave with weight zero (their rows
+        // are staged as zeros; a group with no waves computes no terms): no
+        // entry past the list is read
+        const int4 e = scalar_int4(wl + min(k0 + (int)j, nw - 1));
+        woff[j] = lds0 + (unsigned)(j * FT * kRowBytes) - (unsigned)((e.y - 1) << kShift);
         all_t &= e.w;
         if (e.w & 2) {
           amin = min(amin, e.y);
           amax = max(amax, e.z);
         }
-        const float4 v = A.tx[(size_t)e.x * PS + p];
+        const float4 v = (A.tx + (size_t)e.x * PS)[p];
         if (v.y != 0.0f) {
           td[j] = v.x;
           if constexpr (kT) {
@@ -251,31 +263,54 @@ struct WinKernel {
           }
         }
       });
-      const int njs = (nj + WSUB - 1) / WSUB, nfs = (nfr + FCK - 1) / FCK;
       if constexpr (MODE == MODE_RX)
         static_for<kAF>([&](auto f) { static_for<kAcc>([&](auto j) { acc[f][j] = make_float2(0.0f, 0.0f); }); });
 
-      // windows of step (channel step s, frame chunk fc, wave sub-chunk jc)
+      // The rows this wave stages, r = wave + 4 i: the byte offset that the
+      // wave (and the frame) fixes, the samples its delay's spread takes (0:
+      // no row), the channel of the step.
+      int roff[kPer], rcnt[kPer];
+      __amdgpu_buffer_rsrc_t rs[FT];
+      static_for<FT>([&](auto f) {
+        rs[f] = make_rsrc((const char*)A.ch + (size_t)(f0 + min((int)f, nfr - 1)) * (size_t)A.frame_bytes, A.frame_bytes);
+      });
+      static_for<kPer>([&](auto i) {
+        const int r = wave + 4 * i;
+        const int rem = r % (WC * FT);
+        const int j = rem / FT, f = rem % FT;
+        roff[i] = rcnt[i] = 0;
+        if ((kRows % 4 == 0 || r < kRows) && j < nj && f < nfr) {
+          const int4 we = scalar_int4(wl + k0 + j);
+          roff[i] = (we.x * A.N * A.L + we.y - 1 - WinSpan<SM>::kBack) * 8;
+          rcnt[i] = we.z - we.y + WinSpan<SM>::kSlack;
+        }
+        roff[i] = __builtin_amdgcn_readfirstlane(roff[i]);
+        rcnt[i] = __builtin_amdgcn_readfirstlane(rcnt[i]);
+      });
       float2 st[kPer][kLd];
-      auto stage_load = [&](int s, int fc, int jc) {
+      auto stage_load = [&](int s) {
+        int4 ce[NCH];
+        static_for<NCH>([&](auto c) { ce[c] = scalar_int4(cl + min(s * NCH + c, nc - 1)); });
         static_for<kPer>([&](auto i) {
           const int r = wave + 4 * i;
-          const int c = r / (WSUB * FCK), rem = r - c * (WSUB * FCK);
-          const int j = jc * WSUB + rem / FCK, f = fc * FCK + rem % FCK;
-          const int ci = s * NCH + c;
-          static_for<kLd>([&](auto h) { st[i][h] = make_float2(0.0f, 0.0f); });
-          if ((kRows % 4 == 0 || r < kRows) && j < nj && f < nfr && ci < nc) {
-            const int4 we = scalar_int4(wl + k0 + j), ce = scalar_int4(cl + ci);
-            const int base = we.y + ce.y - 1 - WinSpan<SM>::kBack;
-            const int cnt = (we.z - we.y) + (ce.z - ce.y) + WinSpan<SM>::kSlack;
-            const __amdgpu_buffer_rsrc_t rs =
-                make_rsrc((const char*)A.ch + (size_t)(f0 + f) * (size_t)A.frame_bytes, A.frame_bytes);
-            const unsigned off = (unsigned)((we.x * A.N + ce.x) * A.L + base) * 8u + lane8;
-            static_for<kLd>([&](auto h) {
-              if (h == 0 || cnt > 64 * h)  // uniform
-                st[i][h] = buf_load8(rs, lane + 64 * h < cnt ? (int)(off + 512u * h) : kOOB);
+          int4 e = ce[0];
+          static_for<NCH>([&](auto c) {
+            if (c > 0 && r >= c * WC * FT) e = ce[c];
+          });
+          const int cnt = rcnt[i] > 0 ? rcnt[i] + (e.z - e.y) : 0;
+          const unsigned off = (unsigned)(roff[i] + (e.x * A.L + e.y) * 8) + lane8;
+          // FT 1, 2 or 4: the row's frame is r % FT
+          __amdgpu_buffer_rsrc_t rsf = rs[0];
+          if constexpr (FT > 1) {
+            static_for<FT>([&](auto f) {
+              if ((r % FT) == f) rsf = rs[f];
             });
           }
+          static_for<kLd>([&](auto h) {
+            st[i][h] = make_float2(0.0f, 0.0f);
+            if (h == 0 || cnt > 64 * h)  // uniform
+              st[i][h] = buf_load8(rsf, lane + 64 * h < cnt ? (int)(off + 512u * h) : kOOB);
+          });
         });
       };
       auto stage_store = [&](int buf) {
@@ -301,32 +336,38 @@ struct WinKernel {
       auto rx_load = [&](int s) {
         static_for<NCH>([&](auto c) {
           rv[c] = make_float4(0.f, 0.f, 0.f, 0.f);
-          if (s * NCH + c < nc)
-            rv[c] = rx_entry_t<kCompact>(A.rx, (size_t)scalar_int4(cl + s * NCH + c).x * PS + p);
+          if (s * NCH + c < nc) {
+            const size_t row = (size_t)scalar_int4(cl + s * NCH + c).x * PS;
+            if constexpr (kCompact) {
+              const float2 v = (reinterpret_cast<const float2*>(A.rx) + row)[p];
+              rv[c] = make_float4(v.x, v.y, v.y, v.y * 0.0f);
+            } else {
+              rv[c] = (A.rx + row)[p];
+            }
+          }
         });
       };
 
-      // the terms of channel c (list entry ce) in sub-chunk jc, frame chunk fc
-      auto compute = [&](auto chk, auto c, auto jc, auto fc, int n, int blo, int buf, float rd, float2 R, float ra,
-                         float2(&part)[NCH][FCK]) {
+      // the terms of channel C of the step (channel n, receive bound blo)
+      auto compute = [&](auto chk, auto c, int n, int blo, int buf, float rd, float2 R, float ra, float2(&part)[FT]) {
         constexpr bool CHK = decltype(chk)::value;
-        constexpr int C = decltype(c)::value, JC = decltype(jc)::value, FC = decltype(fc)::value;
-        const unsigned bufo = lds0 + (unsigned)(buf * kBufBytes);
+        constexpr int C = decltype(c)::value;
+        const unsigned zero = lds0 + (unsigned)(buf * kBufBytes);
+        const unsigned coff = (unsigned)(buf * kBufBytes + C * WC * FT * kRowBytes) - (unsigned)(blo << kShift);
         // batches of kB waves: their samples are all asked for before the first
         // is used
-        constexpr int kB = WSUB * FCK <= 4 ? WSUB : (FCK >= 4 ? 1 : 4 / FCK);
-        static_assert(WSUB % kB == 0, "whole batches");
-        static_for<WSUB / kB>([&](auto gr) {
-          constexpr int J0 = JC * WSUB + kB * decltype(gr)::value;
+        constexpr int kBmax = WC * FT <= 4 ? WC : (FT >= 4 ? 1 : 4 / FT);
+        static_for<(WC + kBmax - 1) / kBmax>([&](auto gr) {
+          constexpr int J0 = kBmax * decltype(gr)::value;
+          constexpr int kB = WC - J0 < kBmax ? WC - J0 : kBmax;
           Term1 t[kB];
-          Samples sm[kB][FCK];
+          Samples sm[kB][FT];
           static_for<kB>([&](auto u) {
-            constexpr int J = J0 + decltype(u)::value, jj = J - JC * WSUB;
-            unsigned soff = bufo + (unsigned)((C * WSUB * FCK + jj * FCK) * kRowBytes) -
-                            (unsigned)((alo[J] + blo - 1) << kShift);
+            constexpr int J = J0 + decltype(u)::value;
+            unsigned soff = woff[J] + coff;
             asm("" : "+s"(soff));  // one scalar operand of the address
-            t[u] = term<CHK>(td[J], rd, t0, fs, lim, soff, bufo);
-            static_for<FCK>([&](auto f) { sm[u][f] = fetch(t[u].la, f); });
+            t[u] = term<CHK>(td[J], rd, t0, fs, lim, soff, zero);
+            static_for<FT>([&](auto f) { sm[u][f] = fetch(t[u].la, f); });
           });
           __builtin_amdgcn_sched_barrier(0);
           static_for<kB>([&](auto u) {
@@ -335,26 +376,25 @@ struct WinKernel {
             if constexpr (SM == SM_CUBIC) keys_weights_horner(t[u].b, kw[0], kw[1], kw[2], kw[3]);
             float wr = 0.0f, wi = 0.0f;
             if constexpr (!kSep) exact_weight(t[u].ok ? td[J] : 0.0f, t[u].ok ? rd : 0.0f, Tw[J].x, ra, wd, wr, wi);
-            static_for<FCK>([&](auto f) {
+            static_for<FT>([&](auto f) {
               if constexpr (MODE == MODE_BOTH) {
-                float2 v = part[C][f];
+                float2 v = part[f];
                 cfma(v, Tw[J], interp(sm[u][f], t[u].b, kw));
-                part[C][f] = !CHK || t[u].ok ? v : part[C][f];
+                part[f] = !CHK || t[u].ok ? v : part[f];
               } else if constexpr (MODE == MODE_RX) {
-                float2 v = acc[FC * FCK + f][J];
+                float2 v = acc[f][J];
                 if constexpr (kSep) cfma(v, R, interp(sm[u][f], t[u].b, kw));
                 else cadd(v, exact_value(sm[u][f], t[u].b, kw, wr, wi));
-                acc[FC * FCK + f][J] = !CHK || t[u].ok ? v : acc[FC * FCK + f][J];
+                acc[f][J] = !CHK || t[u].ok ? v : acc[f][J];
               } else {
                 float2 v;
                 if constexpr (kSep) v = cmul(cmul(R, Tw[J]), interp(sm[u][f], t[u].b, kw));
                 else v = exact_value(sm[u][f], t[u].b, kw, wr, wi);
                 if (CHK && !t[u].ok) v = make_float2(0.0f, 0.0f);
                 if (A.ref) v = cmul(v, refp);
-                const int ff = FC * FCK + f;
-                if (act && J < nj && ff < nfr) {
+                if (act && J < nj && f < nfr) {
                   const int w = scalar_int4(wl + k0 + J).x;
-                  A.out[(((size_t)(f0 + ff) * A.W + w) * A.N + n) * PS + p] = v;
+                  (A.out + (((size_t)(f0 + f) * A.W + w) * A.N + n) * PS)[p] = v;
                 }
               }
             });
@@ -365,69 +405,56 @@ struct WinKernel {
 
       int buf = 0;
       if (q < steps) {
-        stage_load(q, 0, 0);
+        stage_load(q);
         stage_store(0);
         rx_load(q);
       }
       __syncthreads();
       for (int it = 0; it < nit; ++it) {
         const int s = q + it * Q;
-        const bool live = s < steps;  // wave-uniform
-        static_for<kNF>([&](auto fc) {
-          if (fc < nfs) {
-            float2 part[NCH][FCK];
-            static_for<NCH>([&](auto c) { static_for<FCK>([&](auto f) { part[c][f] = make_float2(0.0f, 0.0f); }); });
-            static_for<kNS>([&](auto jc) {
-              if (jc < njs) {
-                // the next step
-                int ns = s, nf = fc, nj2 = jc + 1;
-                if (nj2 >= njs) {
-                  nj2 = 0;
-                  if (++nf >= nfs) {
-                    nf = 0;
-                    ns = s + Q;
-                  }
-                }
-                const bool more = ns < steps;
-                if (more) stage_load(ns, nf, nj2);
-                if (live) {
-                  static_for<NCH>([&](auto c) {
-                    const int ci = s * NCH + c;
-                    if (ci < nc) {
-                      const int4 ce = scalar_int4(cl + ci);
-                      const bool ron = rv[c].y != 0.0f;
-                      const float2 R = ron ? make_float2(rv[c].z, rv[c].w) : make_float2(0.0f, 0.0f);
-                      // every term of the channel in the sample window, every
-                      // weight nonzero (dimension both drops the sums of the
-                      // lanes with no receive weight below)
-                      const bool dense = (all_t & 1) && (MODE == MODE_BOTH || (ce.w & 1)) && amin + ce.y - 1 >= 1 &&
-                                         amax + ce.z + 2 < ilim;
-                      if (dense)
-                        compute(std::false_type(), c, jc, fc, ce.x, ce.y, buf, rv[c].x, R, rv[c].y, part);
-                      else
-                        compute(std::true_type(), c, jc, fc, ce.x, ce.y, buf, ron ? rv[c].x : kFar, R, rv[c].y, part);
-                    }
-                  });
-                }
-                if constexpr (MODE == MODE_BOTH) {
-                  if (live && jc + 1 >= njs)
-                    static_for<NCH>([&](auto c) {
-                      const bool ron = rv[c].y != 0.0f;
-                      static_for<FCK>([&](auto f) {
-                        float2 v = acc[fc * FCK + f][0];
-                        cfma(v, make_float2(rv[c].z, rv[c].w), part[c][f]);
-                        acc[fc * FCK + f][0] = ron ? v : acc[fc * FCK + f][0];
-                      });
-                    });
-                }
-                if (more && ns != s) rx_load(ns);
-                if (more) stage_store(buf ^ 1);
-                __syncthreads();
-                buf ^= 1;
-              }
-            });
+        const bool more = s + Q < steps;           // wave-uniform
+        if (more) stage_load(s + Q);
+        if (s < steps && nj > 0) {
+          static_for<NCH>([&](auto c) {
+            const int ci = s * NCH + c;
+            if (ci < nc) {
+              const int4 ce = scalar_int4(cl + ci);
+              const bool ron = rv[c].y != 0.0f;
+              const float2 R = ron ? make_float2(rv[c].z, rv[c].w) : make_float2(0.0f, 0.0f);
+              float2 part[FT];
+              static_for<FT>([&](auto f) { part[f] = make_float2(0.0f, 0.0f); });
+              // every term of the channel in the sample window, every weight
+              // nonzero (dimension both drops the sums of the lanes with no
+              // receive weight below)
+              const bool dense = (all_t & 1) && (MODE == MODE_BOTH || (ce.w & 1)) && amin + ce.y - 1 >= 1 &&
+                                 amax + ce.z + 2 < ilim;
+              if (dense)
+                compute(std::false_type(), c, ce.x, ce.y, buf, rv[c].x, R, rv[c].y, part);
+              else
+                compute(std::true_type(), c, ce.x, ce.y, buf, ron ? rv[c].x : kFar, R, rv[c].y, part);
+              if constexpr (MODE == MODE_BOTH)
+                static_for<FT>([&](auto f) {
+                  float2 v = acc[f][0];
+                  cfma(v, make_float2(rv[c].z, rv[c].w), part[f]);
+                  acc[f][0] = ron ? v : acc[f][0];
+                });
+            }
+          });
+        }
+        // the next entries into the same registers: a second set, in flight
+        // during the terms, costs a block per CU and time (cine 0.60 -> 0.77 ms)
+        if (more) {
+          rx_load(s + Q);
+          stage_store(buf ^ 1);
+        }
+        if constexpr (kClose) {
+          if ((it & 31) == 31) {
+            cadd(tot, acc[0][0]);
+            acc[0][0] = make_float2(0.0f, 0.0f);
           }
-        });
+        }
+        __syncthreads();
+        buf ^= 1;
       }
 
       if constexpr (MODE == MODE_RX) {
@@ -437,7 +464,7 @@ struct WinKernel {
             const int w = scalar_int4(wl + k0 + j).x;
             float2 Tj = make_float2(0.0f, 0.0f);
             if constexpr (kSep) {
-              const float4 v = A.tx[(size_t)w * PS + p];
+              const float4 v = (A.tx + (size_t)w * PS)[p];
               if (v.y != 0.0f) Tj = make_float2(v.z, v.w);
             }
             static_for<FT>([&](auto f) {
@@ -445,7 +472,7 @@ struct WinKernel {
                 float2 v = group_sum(acc[f][j], smem, g, lid);
                 if constexpr (kSep) v = cmul(Tj, v);
                 if (A.ref) v = cmul(v, refp);
-                if (act && g == 0) A.out[((size_t)(f0 + f) * A.W + w) * PS + p] = v;
+                if (act && g == 0) (A.out + ((size_t)(f0 + f) * A.W + w) * PS)[p] = v;
               }
             });
           }
@@ -456,44 +483,46 @@ struct WinKernel {
     if constexpr (MODE == MODE_BOTH)
       static_for<FT>([&](auto f) {
         if (f < nfr) {
-          float2 v = group_sum(acc[f][0], smem, g, lid);
+          float2 v = acc[f][0];
+          if constexpr (kClose) cadd(v, tot);
+          v = group_sum(v, smem, g, lid);
           if (A.ref) v = cmul(v, refp);
-          if (act && g == 0) A.out[(size_t)(f0 + f) * PS + p] = v;
+          if (act && g == 0) (A.out + (size_t)(f0 + f) * PS)[p] = v;
         }
       });
   }
 
-  // The channel groups' sums in group order (group 0 gets them).
+  // The groups' sums in group order (group 0 gets them).
   static __device__ __forceinline__ float2 group_sum(float2 v, char* smem, int g, int lid) {
-    if constexpr (CG > 1) {
+    if constexpr (kGroups > 1) {
       float2* red = reinterpret_cast<float2*>(smem);
       red[threadIdx.x] = v;
       __syncthreads();
       if (g == 0)
-        static_for<CG - 1>([&](auto k) { cadd(v, red[(k + 1) * 256 + lid]); });
+        static_for<kGroups - 1>([&](auto k) { cadd(v, red[(k + 1) * 256 + lid]); });
       __syncthreads();
     }
     return v;
   }
 };
 
-template <int SM, int MODE, int PH, int ROW, int WC, int WSUB, int FT, int FCK, int NCH, int CG>
-__global__ __launch_bounds__(256 * CG, 4) void das_window_kernel(WinArgs A) {
-  using K = WinKernel<SM, MODE, PH, ROW, WC, WSUB, FT, FCK, NCH, CG>;
+template <int SM, int MODE, int PH, int ROW, int WC, int FT, int NCH, int CG, int WG>
+__global__ __launch_bounds__(256 * CG * WG, 4) void das_window_kernel(WinArgs A) {
+  using K = WinKernel<SM, MODE, PH, ROW, WC, FT, NCH, CG, WG>;
   __shared__ __align__(16) char smem[K::kSmem];
   K::run(A, smem);
 }
 
 // Channel groups per tile: blocks of 1024 threads (or, in dimension none,
 // more blocks per tile) where the tiles alone leave the chip idle.
-template <int SM, int MODE, int PH, int ROW, int WC, int WSUB, int FT, int FCK, int NCH, int CG>
+template <int SM, int MODE, int PH, int ROW, int WC, int FT, int NCH, int CG, int WG>
 static hipError_t launch_window_t(const GeomLaunch& G, int zsplit, hipStream_t stream) {
   WinArgs A;
   A.ch = G.ch;
   A.out = reinterpret_cast<float2*>(G.out);
   A.tx = G.tx_table;
-  A.rx = G.win_rx;
-  A.ref = G.ref_phase ? G.win_ref : nullptr;
+  A.rx = G.dim == MODE_BOTH ? G.rx_table : G.win_rx;
+  A.ref = G.ref_phase ? (G.dim == MODE_BOTH ? G.ref_table : G.win_ref) : nullptr;
   A.T = G.win;
   A.P = G.P;
   A.N = G.N;
@@ -504,14 +533,20 @@ static hipError_t launch_window_t(const GeomLaunch& G, int zsplit, hipStream_t s
   A.fs = G.fs;
   A.wd = G.wd;
   A.frame_bytes = G.L * G.N * G.W * 8;
-  hipLaunchKernelGGL((das_window_kernel<SM, MODE, PH, ROW, WC, WSUB, FT, FCK, NCH, CG>),
-                     dim3((unsigned)G.win.tiles, (unsigned)((G.F + FT - 1) / FT), (unsigned)zsplit), dim3(256 * CG), 0,
+  hipLaunchKernelGGL((das_window_kernel<SM, MODE, PH, ROW, WC, FT, NCH, CG, WG>),
+                     dim3((unsigned)G.win.tiles * (unsigned)((G.F + FT - 1) / FT), 1u, (unsigned)zsplit), dim3(256 * CG * WG), 0,
                      stream, A);
   return hipGetLastError();
 }
 
 hipError_t launch_window_rx(const GeomLaunch& G, int ph, hipStream_t stream);
 hipError_t launch_window_none(const GeomLaunch& G, int ph, hipStream_t stream);
-hipError_t launch_window_both(const GeomLaunch& G, hipStream_t stream);
+hipError_t launch_window_both_iq(const GeomLaunch& G, hipStream_t stream);
+hipError_t launch_window_both_rf(const GeomLaunch& G, hipStream_t stream);
+hipError_t launch_window_both_cubic(const GeomLaunch& G, hipStream_t stream);
+inline hipError_t launch_window_both(const GeomLaunch& G, hipStream_t stream) {
+  if (G.interp == INTERP_CUBIC) return launch_window_both_cubic(G, stream);
+  return G.wd == 0.0f ? launch_window_both_rf(G, stream) : launch_window_both_iq(G, stream);
+}
 
 }  // namespace ustbx

@@ -1,0 +1,10 @@
+// das_window_both_rf.hip — the window-staged kernel of dimension both, linear RF data.
+#include "das_window_both.h"
+
+namespace ustbx {
+
+hipError_t launch_window_both_rf(const GeomLaunch& G, hipStream_t s) {
+  return G.win.row == 64 ? both_shape<SM_LINEAR, PH_RF, 64>(G, s) : both_shape<SM_LINEAR, PH_RF, 128>(G, s);
+}
+
+}  // namespace ustbx

@@ -5,7 +5,7 @@
 // 64 terms), none by its stores. Measured against the per-lane kernel, which
 // forms delay, weight and phase of every (pixel, channel) in FP64 for every 8
 // waves and every frame: 64 channels x 31 waves x 4 frames on 193 x 512 pixels
-// of a sector (receive, then the coherence factor) 4.69 -> 0.59 ms; 128
+// of a sector (receive, then the coherence factor) 4.69 -> 0.48 ms; 128
 // channels x 5 waves on 150 x 201 pixels (none, 154 MB of output) 0.42 -> 0.087
 // ms.
 //
@@ -25,23 +25,23 @@ static int tiles_short(const GeomLaunch& G, int ft) {
   return (int64_t)G.win.tiles * ((G.F + ft - 1) / ft) < 1024;
 }
 
-template <int SM, int PH, int ROW, int WC, int WSUB, int FT, int FCK, int NCH>
+template <int SM, int PH, int ROW, int WC, int FT, int NCH>
 static hipError_t rx_cg(const GeomLaunch& G, hipStream_t s) {
   // the exact phases add a wave's channels in das_c's ascending order
   constexpr int kCG = PH == PH_SEP && FT == 1 ? 4 : 1;
   if (kCG > 1 && tiles_short(G, FT))
-    return launch_window_t<SM, MODE_RX, PH, ROW, WC, WSUB, FT, FCK, NCH, kCG>(G, 1, s);
-  return launch_window_t<SM, MODE_RX, PH, ROW, WC, WSUB, FT, FCK, NCH, 1>(G, 1, s);
+    return launch_window_t<SM, MODE_RX, PH, ROW, WC, FT, NCH, kCG, 1>(G, 1, s);
+  return launch_window_t<SM, MODE_RX, PH, ROW, WC, FT, NCH, 1, 1>(G, 1, s);
 }
 
 template <int SM, int PH, int ROW>
 static hipError_t rx_shape(const GeomLaunch& G, hipStream_t s) {
   if (G.F > 1) {
-    if constexpr (PH == PH_SEP) return rx_cg<SM, PH, ROW, 8, 8, 2, 2, 1>(G, s);
-    else return rx_cg<SM, PH, ROW, 4, 4, 2, 2, 2>(G, s);
+    if constexpr (PH == PH_SEP) return rx_cg<SM, PH, ROW, 8, 2, 1>(G, s);
+    else return rx_cg<SM, PH, ROW, 4, 2, 2>(G, s);
   }
-  if (G.W <= 4) return rx_cg<SM, PH, ROW, 4, 4, 1, 1, 4>(G, s);
-  return rx_cg<SM, PH, ROW, 8, 8, 1, 1, 2>(G, s);
+  if (G.W <= 4) return rx_cg<SM, PH, ROW, 4, 1, 4>(G, s);
+  return rx_cg<SM, PH, ROW, 8, 1, 2>(G, s);
 }
 
 template <int SM, int ROW>
@@ -57,19 +57,19 @@ hipError_t launch_window_rx(const GeomLaunch& G, int ph, hipStream_t s) {
   return G.interp == INTERP_CUBIC ? rx_ph<SM_CUBIC, 128>(G, ph, s) : rx_ph<SM_LINEAR, 128>(G, ph, s);
 }
 
-template <int SM, int PH, int ROW, int WC, int WSUB, int FT, int FCK, int NCH>
+template <int SM, int PH, int ROW, int WC, int FT, int NCH>
 static hipError_t none_z(const GeomLaunch& G, hipStream_t s) {
   const int64_t blocks = (int64_t)G.win.tiles * ((G.F + FT - 1) / FT);
   const int steps = (G.N + NCH - 1) / NCH;
   int z = (int)std::min<int64_t>((2048 + blocks - 1) / blocks, std::max(1, steps / 4));
-  return launch_window_t<SM, MODE_NONE, PH, ROW, WC, WSUB, FT, FCK, NCH, 1>(G, std::max(1, std::min(z, 64)), s);
+  return launch_window_t<SM, MODE_NONE, PH, ROW, WC, FT, NCH, 1, 1>(G, std::max(1, std::min(z, 64)), s);
 }
 
 template <int SM, int PH, int ROW>
 static hipError_t none_shape(const GeomLaunch& G, hipStream_t s) {
-  if (G.F > 1) return none_z<SM, PH, ROW, 4, 4, 2, 2, 2>(G, s);
-  if (G.W <= 4) return none_z<SM, PH, ROW, 4, 4, 1, 1, 4>(G, s);
-  return none_z<SM, PH, ROW, 8, 8, 1, 1, 2>(G, s);
+  if (G.F > 1) return none_z<SM, PH, ROW, 4, 2, 2>(G, s);
+  if (G.W <= 4) return none_z<SM, PH, ROW, 4, 1, 4>(G, s);
+  return none_z<SM, PH, ROW, 8, 1, 2>(G, s);
 }
 
 template <int SM, int ROW>

@@ -260,7 +260,9 @@ class GeometryPlan:
 
     @property
     def variant(self) -> tuple[int, int, int]:
-        """(variant, waves per chunk or split, split) currently selected."""
+        """(variant, waves per chunk or split, split) currently selected;
+        (2, 0, 0) where the library runs the plan on patch tiles with staged
+        sample windows (no tile shape set)."""
         wc, sp = ctypes.c_int32(0), ctypes.c_int32(0)
         v = L.lib().ustbx_plan_variant(self.handle, ctypes.byref(wc), ctypes.byref(sp))
         return int(v), int(wc.value), int(sp.value)
