@@ -523,8 +523,19 @@ std::vector<int> line_band_order(int tpl, int tiles, int shares) {
 std::vector<int> band_major_order(const DevScan& sc, int tile_ps, int tiles, int shares) {
   std::vector<int> order(tiles);
   for (int t = 0; t < tiles; ++t) order[t] = t;
-  if (!(sc.kind == SCAN_LINEAR || sc.kind == SCAN_SECTOR) || (tile_ps == 0 && sc.n0 % 64 != 0) || tiles < shares)
+  if (!(sc.kind == SCAN_LINEAR || sc.kind == SCAN_SECTOR) || tiles < shares) return order;
+  if (tile_ps == 0 && sc.n0 % 64 != 0) {
+    // lines of a depth count that 64 does not divide: a tile may end one line
+    // and begin the next; it goes by the depth of its first pixel
+    const int64_t n0 = sc.n0;
+    const int q = tiles / shares, r = tiles % shares;
+    for (int k = 0; k < shares; ++k) {
+      const int s0 = k * q + std::min(k, r), cnt = q + (k < r ? 1 : 0);
+      std::stable_sort(order.begin() + s0, order.begin() + s0 + cnt,
+                       [n0](int a, int b) { return (a * (int64_t)64) % n0 / 64 < (b * (int64_t)64) % n0 / 64; });
+    }
     return order;
+  }
   return line_band_order(tile_ps ? sc.n0 >> tile_ps : sc.n0 / 64, tiles, shares);  // tiles per line (group)
 }
 
