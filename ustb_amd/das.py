@@ -20,7 +20,7 @@ from collections import OrderedDict
 import numpy as np
 
 from .enums import Code, Dimension, Interpolation, SphericalTransmitDelayModel, Window
-from .uff import Apodization, BeamformedData, ChannelData, Scan, probe_radius
+from .uff import Apodization, BeamformedData, ChannelData, LinearScan, Scan, SectorScan, probe_radius
 
 
 class DAS:
@@ -69,11 +69,25 @@ class DAS:
             h.update(repr(v.shape).encode())
             h.update(np.ascontiguousarray(v, dtype=np.float64).tobytes())
 
+    @staticmethod
+    def _scan_arrays(sc: Scan):
+        """The arrays a plan is built from (build_geometry): the axes of a
+        linear or sector scan, the pixel list of any other. Hashing the axes
+        instead of every pixel's coordinates takes 0.06 ms per go() instead of
+        0.6-1.1 ms on 193 x 321 pixels (10 ms on 512 x 1024)."""
+        if isinstance(sc, LinearScan):
+            return sc.z_axis, sc.x_axis, sc.y_axis
+        if isinstance(sc, SectorScan):
+            return sc.depth_axis, sc.azimuth_axis, sc.elevation_axis, sc.origin
+        return sc.x, sc.y, sc.z
+
     def _plan_key(self, n_samples, n_frames):
         cd, sc = self.channel_data, self.scan
         h = hashlib.sha1()
-        for a in (cd.probe.x, cd.probe.y, cd.probe.z, sc.x, sc.y, sc.z):
-            h.update(np.ascontiguousarray(a, dtype=np.float64).tobytes())
+        for a in (cd.probe.x, cd.probe.y, cd.probe.z, *self._scan_arrays(sc)):
+            a = np.ascontiguousarray(a, dtype=np.float64)
+            h.update(repr(a.shape).encode())  # two axes do not run into each other
+            h.update(a.tobytes())
         h.update(repr([(int(w.wavefront), w.source, w.origin, w.delay, w.sound_speed) for w in cd.sequence]).encode())
         self._apodization_key(h, self.receive_apodization)
         self._apodization_key(h, self.transmit_apodization)
