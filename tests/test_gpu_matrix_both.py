@@ -1,0 +1,70 @@
+"""Dimension both of the matrix contract in the library's own summation order,
+at the wave counts, frame counts and pixel counts where its blocks change,
+against das_c's order (split 1) on the same matrices."""
+from __future__ import annotations
+
+import numpy as np
+import pytest
+
+torch = pytest.importorskip("torch")
+
+from tests.cases import matrix_problem
+from ustb_amd import ops
+
+pytestmark = pytest.mark.gpu
+
+
+def _images(cuda, q, fd, **kw):
+    t = {k: torch.from_numpy(q[k]).to(cuda) for k in ("ch", "tx_apo", "rx_apo", "tx_delay", "rx_delay")}
+    args = (t["ch"], q["fs"], q["t0"], t["tx_apo"], t["rx_apo"], t["tx_delay"], t["rx_delay"], fd, 3)
+    return ops.das(*args, **kw), ops.das(*args, dasc_order=True, **kw)
+
+
+def _close(got, ref, terms):
+    a, b = torch.view_as_real(got), torch.view_as_real(ref)
+    assert torch.equal(torch.isnan(a), torch.isnan(b))
+    err = torch.nan_to_num(a - b).abs().max() / torch.nan_to_num(b).abs().max()
+    # the same terms (FP32, the same rounded phase) added in another order
+    assert err.item() <= 6e-8 * (4 + terms ** 0.5)
+
+
+@pytest.mark.parametrize("fd", [0.0, 0.11, -3.7])
+@pytest.mark.parametrize("P,N,W,F", [(63, 5, 2, 1), (64, 1, 3, 4), (65, 7, 8, 5), (1, 3, 9, 1), (130, 12, 33, 1),
+                                     (200, 9, 70, 6)])
+@pytest.mark.parametrize("interp,edge", [(0, 0), (0, 1), (1, 0)])
+def test_against_dasc_order(cuda, P, N, W, F, fd, interp, edge):
+    print(f"case matrix both P={P} N={N} W={W} F={F} fd={fd} interp={interp} edge={edge}", flush=True)
+    q = matrix_problem(seed=P + W, P=P, N=N, W=W, F=F)
+    got, ref = _images(cuda, q, fd, interp=interp, edge=edge)
+    _close(got, ref, N * W)
+
+
+def test_physical_delays(cuda):
+    """Phases of thousands of radians, an initial time, unlisted waves."""
+    rng = np.random.default_rng(9)
+    P, N, W, L = 300, 11, 12, 900
+    q = dict(ch=(rng.standard_normal((2, W, N, L)) + 1j * rng.standard_normal((2, W, N, L))).astype(np.complex64),
+             fs=20.8e6, t0=3.1e-6, tx_apo=rng.uniform(0.1, 1.0, (W, P)).astype(np.float32),
+             rx_apo=rng.uniform(-0.5, 1.0, (N, P)).astype(np.float32),
+             tx_delay=rng.uniform(-1e-6, 2.4e-5, (W, P)).astype(np.float32),
+             rx_delay=rng.uniform(2e-6, 2.4e-5, (N, P)).astype(np.float32))
+    q["tx_apo"][3:7] = 0.0
+    q["tx_apo"][8, :128] = 0.0
+    for fd in (5.2e6, 2.0e7):
+        _close(*_images(cuda, q, fd), N * W)
+
+
+def test_non_finite_weights_delays_and_samples(cuda):
+    """What das_c skips stays out of the sums, what it multiplies reaches them."""
+    q = matrix_problem(seed=5, P=200, N=9, W=6, F=2, L=80)
+    q["rx_apo"][2, 30:90] = np.nan
+    q["tx_apo"][1, 80:100] = np.nan
+    q["rx_delay"][4, 10:20] = np.nan
+    q["tx_delay"][0, 150:160] = np.inf
+    q["ch"][0, 3, 5, 20:24] = np.nan
+    q["ch"][1, 2, 1, 40] = np.inf
+    got, ref = _images(cuda, q, 0.13)
+    assert torch.equal(torch.isfinite(torch.view_as_real(got)), torch.isfinite(torch.view_as_real(ref)))
+    fine = torch.isfinite(ref.real) & torch.isfinite(ref.imag)
+    assert fine.any() and not fine.all()
+    assert (got[fine] - ref[fine]).abs().max() <= 1e-6 * ref[fine].abs().max()

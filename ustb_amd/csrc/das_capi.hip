@@ -425,7 +425,8 @@ int ustbx_das_run(const ustbx_das_desc* d, const void* ch, const float* tx_apo,
   m.split = (d->flags & USTBX_FLAG_DASC_ORDER) ? 1 : (d->split ? d->split : matrix_auto_split(d->P));
   if (m.split != 1 && m.split != 2 && m.split != 4 && m.split != 8)
     return set_status(st, USTBX_E_ARG, "split must be 1, 2, 4 or 8");
-  hipError_t e = launch_das_matrix(m, s);
+  const bool free_order = !(d->flags & USTBX_FLAG_DASC_ORDER) && d->split == 0;
+  hipError_t e = free_order && matrix_both_applies(m) ? launch_das_matrix_both(m, s) : launch_das_matrix(m, s);
   if (e != hipSuccess) return hip_fail(st, e, "das_matrix_kernel launch");
   return ok(st);
 }

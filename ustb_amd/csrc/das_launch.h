@@ -23,6 +23,10 @@ struct MatLaunch {
 };
 
 hipError_t launch_das_matrix(const MatLaunch& m, hipStream_t stream);
+// Dimension both with no summation order or channel split asked for
+// (das_matrix_both.hip), where it applies.
+bool matrix_both_applies(const MatLaunch& m);
+hipError_t launch_das_matrix_both(const MatLaunch& m, hipStream_t stream);
 
 // Fills n complex64 values with zeros (a kernel, so it can be graph-captured).
 hipError_t launch_zero_fill(void* p, size_t n_complex, hipStream_t stream);
