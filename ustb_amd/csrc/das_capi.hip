@@ -704,6 +704,7 @@ bool rxtab_build(ustbx_plan* pl, hipError_t& err, bool otf) {
   pl->tile_natural = nat;
   pl->n_bad = n_bad;
   pl->max_nw = max_nw;
+  G.max_nw = max_nw;
   pl->rxtab_state = 1;
   pl->h_order = std::move(batch_order);
   pl->h_cost.resize(tiles);

@@ -374,8 +374,22 @@ static hipError_t launch_rxtab_l(const GeomLaunch& G, hipStream_t stream) {
   return hipGetLastError();
 }
 
+template <int SM, int WC>
+static hipError_t launch_rxtab_few(const GeomLaunch& G, hipStream_t stream) {
+  return G.rx_compact ? launch_rxtab_l<SM, WC, 8, RXL_COMPACT>(G, stream)
+                      : launch_rxtab_l<SM, WC, 8, RXL_FULL>(G, stream);
+}
+
 template <int SM, int WC, int WS>
 static hipError_t launch_rxtab_t(const GeomLaunch& G, hipStream_t stream) {
+  // shapes of 4 x 8 whose tiles hold one or two waves run without the empty
+  // slots, several channels at a time (the same sums: with one round the
+  // channel groups do not depend on WC); plane wave of 128 channels RF on 256 x
+  // 256 pixels 24.7 -> 15.7 us
+  if constexpr (WC == 4 && WS == 8) {
+    if (!G.rx_otf && G.max_nw == 1) return launch_rxtab_few<SM, 1>(G, stream);
+    if (!G.rx_otf && G.max_nw == 2) return launch_rxtab_few<SM, 2>(G, stream);
+  }
   if (SM != SM_COEF && G.rx_otf) return launch_otf_t<SM == SM_COEF ? SM_LINEAR : SM, WC, WS>(G, stream);
   return G.rx_compact ? launch_rxtab_l<SM, WC, WS, RXL_COMPACT>(G, stream)
                       : launch_rxtab_l<SM, WC, WS, RXL_FULL>(G, stream);

@@ -126,7 +126,8 @@ struct GeomLaunch {
   // rx_table and ref_table and takes them while no tile shape is set
   // (auto_tiles), the other modes win_rx and win_ref.
   WinTiles win;
-  int win_max_nw;        // largest wave count of a tile
+  int win_max_nw;        // largest wave count of a patch tile
+  int max_nw;            // largest wave count of a variant-2 tile
   int auto_tiles;
   const float4* win_rx;
   const float2* win_ref;

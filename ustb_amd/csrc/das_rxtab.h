@@ -370,6 +370,94 @@ __device__ __forceinline__ void rxtab_channels(__amdgpu_buffer_rsrc_t rs, const 
   }
 }
 
+// rxtab_channels for tiles of at most WC = 1 or 2 waves: kU channels at a time,
+// their receive rows one step ahead and all their gathers issued together. (A
+// channel of one wave alone leaves a wave64 one gather in flight, and a shape
+// of 4 slots issues three empty ones beside it.) The sums are
+// rxtab_channels', channel for channel.
+template <int SM, int WC, bool SAFE, bool COMPACT>
+__device__ __forceinline__ void rxtab_channels_few(__amdgpu_buffer_rsrc_t rs, const float (&td)[WC],
+                                                   const float2 (&T)[WC], const int (&wb)[WC],
+                                                   const float4* __restrict__ rxt, const int* __restrict__ chl,
+                                                   int cstride, int nc, size_t PS, int p, bool active, int lst,
+                                                   float t0, float fs, float lim, float2& acc) {
+  using M = SampleMode<SM>;
+  constexpr int kU = 4 / WC;
+  float4 rn[kU];
+  int nn[kU];
+  auto load = [&](int k) {
+#pragma unroll
+    for (int u = 0; u < kU; ++u) {
+      rn[u] = make_float4(0.f, 0.f, 0.f, 0.f);  // past the list: no weight
+      nn[u] = 0;
+      if (k + u < nc) {
+        nn[u] = __builtin_amdgcn_readfirstlane(chl[(k + u) * cstride]);
+        if (active) rn[u] = rx_entry_t<COMPACT>(rxt, (size_t)nn[u] * PS + p);
+      }
+    }
+  };
+  load(0);
+  for (int k = 0; k < nc; k += kU) {
+    float4 rv[kU];
+    int nb[kU];
+#pragma unroll
+    for (int u = 0; u < kU; ++u) {
+      rv[u] = rn[u];
+      nb[u] = nn[u] * lst;
+    }
+    if (k + kU < nc) load(k + kU);
+    float4 q[kU][WC][M::kLoads];
+    float bb[kU][WC];
+    bool okb[kU][WC];
+#pragma unroll
+    for (int u = 0; u < kU; ++u) {
+      const float rd = rv[u].y != 0.0f ? rv[u].x : kFar;
+#pragma unroll
+      for (int j = 0; j < WC; ++j) {
+        const float d = term_index(td[j], rd, t0, fs);
+        const bool ok = d >= 1.0f && d < lim;
+        okb[u][j] = ok;
+        bb[u][j] = __builtin_amdgcn_fractf(d);
+        const int off = ok ? (int)d * M::kStride + (nb[u] + wb[j] + M::kLo) : kOOB;
+        q[u][j][0] = buf_load16(rs, off);
+        if (M::kLoads == 2) q[u][j][M::kLoads - 1] = buf_load16(rs, off + (M::kHi - M::kLo));
+      }
+    }
+    __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+    for (int u = 0; u < kU; ++u) {
+      float2 part = make_float2(0.0f, 0.0f);
+      bool any = false;
+#pragma unroll
+      for (int j = 0; j < WC; ++j) {
+        const float b = bb[u][j];
+        float2 sm;
+        const float4 lo = q[u][j][0], hi = q[u][j][M::kLoads - 1];
+        if (SM == SM_LINEAR) {
+          sm = make_float2(fmaf(b, lo.z - lo.x, lo.x), fmaf(b, lo.w - lo.y, lo.y));
+        } else if (SM == SM_CUBIC) {
+          float c0, c1, c2, c3;
+          keys_weights_horner(b, c0, c1, c2, c3);
+          sm = make_float2(fmaf(c3, hi.z, fmaf(c2, hi.x, fmaf(c1, lo.z, c0 * lo.x))),
+                           fmaf(c3, hi.w, fmaf(c2, hi.y, fmaf(c1, lo.w, c0 * lo.y))));
+        } else {
+          sm = make_float2(fmaf(fmaf(fmaf(hi.z, b, hi.x), b, lo.z), b, lo.x),
+                           fmaf(fmaf(fmaf(hi.w, b, hi.y), b, lo.w), b, lo.y));
+        }
+        float2 t = part;
+        cfma(t, T[j], sm);
+        part = !SAFE || okb[u][j] ? t : part;
+        any = any || okb[u][j];
+      }
+      const float2 R = rv[u].y != 0.0f ? make_float2(rv[u].z, rv[u].w) : make_float2(0.0f, 0.0f);
+      float2 t = acc;
+      cfma(t, R, part);
+      acc = !SAFE || any ? t : acc;
+    }
+    __builtin_amdgcn_sched_barrier(0);
+  }
+}
+
 // Receive-table layout of a kernel: float4 only, float2 only (RF plans), or
 // either, chosen per acquisition at run time (the batch kernel).
 enum { RXL_FULL = 0, RXL_COMPACT = 1, RXL_EITHER = 2 };
@@ -413,7 +501,7 @@ __device__ __forceinline__ void rxtab_tile(const RxAcq& A, int tile, int f, floa
   const int g = s / wsp;
   const int sw = s - g * wsp;           // split within the group
   const int ncg = g < cg ? (nc - g + cg - 1) / cg : 0;
-  constexpr bool kStg = STG && !SAFE && SM != SM_COEF;
+  constexpr bool kStg = STG && !SAFE && SM != SM_COEF && WC > 2;
   const unsigned long long* smask =
       kStg && A.stage_mask ? A.stage_mask + (size_t)tile * (size_t)A.stage_words : nullptr;
   float2* swin = kStg ? win + s * (StageBatch<SM>::RB * kStageWin) : nullptr;
@@ -447,7 +535,14 @@ __device__ __forceinline__ void rxtab_tile(const RxAcq& A, int tile, int f, floa
         }
       }
     }
-    if (nj == WC) {
+    if constexpr (WC <= 2) {
+      if (compact)
+        rxtab_channels_few<SM, WC, SAFE, true>(rs, td, T, wb, A.rx, chl + g, cg, ncg, PS, p, active, lst, A.t0, A.fs,
+                                               lim, acc);
+      else
+        rxtab_channels_few<SM, WC, SAFE, false>(rs, td, T, wb, A.rx, chl + g, cg, ncg, PS, p, active, lst, A.t0, A.fs,
+                                                lim, acc);
+    } else if (nj == WC) {
       if (compact)
         rxtab_channels<SM, WC, false, SAFE, true, kStg>(rs, td, T, wb, nj, A.rx, chl + g, cg, ncg, PS, p, active,
                                                         lst, A.t0, A.fs, lim, acc, smask, g, swin, lane8);
