@@ -948,6 +948,7 @@ def run_serve(args, torch, dev):
     plain = srv.plain_loop(trace)
     log(f"plain {plain.summary(names)}")
     # parity: a few requests alone (plan runs with the server's tiles) and in the mix
+    from ustb_amd import autotune
     chk = poisson_trace(12, rate=args.rate, n_configs=len(cfgs), n_data=len(datasets[0]), seed=7)
     mixed = srv.run(chk, keep_outputs=True)
     plain_chk = srv.plain_loop(chk, keep_outputs=True)
