@@ -113,12 +113,13 @@ def test_samples_outside_the_weights_stay_out(cuda, dim):
 
 
 BOTH = [
-    # kind, W, nx, nz, F, rf, cubic, L: at least 512 blocks of 256 pixels (x 2 frames)
-    ("linear", 9, 300, 450, 1, False, False, 512),
-    ("linear", 13, 131, 333, 7, True, False, 500),    # traces end inside the image
-    ("linear", 33, 301, 470, 1, False, False, 420),
-    ("sector", 17, 200, 331, 5, False, True, 512),
-    ("volume", 26, 60, 170, 3, False, False, 400),
+    # kind, W, nx, nz, F, rf, cubic, L: work of at least 640, 512 or 400 of the
+    # largest tiles (x 2 frames), with tiles of half of it
+    ("linear", 9, 540, 900, 1, False, False, 512),
+    ("linear", 13, 251, 333, 7, True, False, 500),    # traces end inside the image
+    ("linear", 33, 401, 700, 1, False, False, 420),
+    ("sector", 17, 401, 401, 5, False, True, 512),
+    ("volume", 26, 110, 170, 3, False, False, 400),
 ]
 
 

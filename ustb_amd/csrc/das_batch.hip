@@ -334,7 +334,10 @@ int ustbx_batch_create(const ustbx_plan* const* plans, int32_t count, ustbx_batc
   }
   int ws = 8, wc = 8;
   if (nw_med <= 32) {
-    ws = 4;  // as the one-plan default: 4 splits of 8 waves
+    // us per batch against 8 x 4: images of 5, 11, 16 and 25 waves 254 ->
+    // 202, 431 -> 380, 583 -> 517 and 962 -> 794; volumes of 25 waves 22515 ->
+    // 19305, of 9 waves as before (3506 and 3509; 4 x 8 takes 4649 there)
+    wc = nw_med <= 16 ? 8 : 16;
   } else {
     const int need = (nw_med + 7) / 8;
     wc = need <= 4 ? 4 : need <= 6 ? 6 : need <= 8 ? 8 : need <= 10 ? 10 : need <= 12 ? 12 : 16;

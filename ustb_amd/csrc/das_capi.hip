@@ -62,21 +62,17 @@ constexpr double kRxTableMaxFraction = 0.5;
 
 bool rxtab_wc_ok(int wc) { return wc == 4 || wc == 5 || wc == 6 || wc == 8 || wc == 10 || wc == 12 || wc == 16; }
 
-// Up to 8 waves: 8 splits of 4 waves, most of them in channel groups; up to
-// 32 waves: 4 splits of 8 waves (a whole round with enough terms per receive
-// row); more: 8 splits with the smallest waves-per-split covering the busiest
-// tile in one round (else 16 per round).
-void rxtab_default_tiles(int max_nw, int& wc, int& ws);
-
 // Dimension transmit: 8 frames per block (4 when fewer), 8 channels per block
 // (4 when fewer).
+void rxtab_default_tiles(int64_t blocks, int max_nw, bool cubic, bool otf, int& wc, int& ws);
+
 void rxtab_defaults(const GeomLaunch& G, int max_nw, int& wc, int& ws) {
   if (G.dim == 2) {  // frames per block, channels per block (measured best on 32 frames x 64 channels)
     wc = G.F >= 8 ? 8 : 4;
     ws = G.N >= 8 ? 8 : 4;
     return;
   }
-  rxtab_default_tiles(max_nw, wc, ws);
+  rxtab_default_tiles((int64_t)((G.P + 63) / 64) * G.F, max_nw, G.interp == USTBX_INTERP_CUBIC, G.rx_otf != 0, wc, ws);
   // Keys' cubic over many waves: 4 splits of 10 waves (C2, 75 waves:
   // 2.49 ms against 2.57 ms with 8 splits)
   if (G.interp == USTBX_INTERP_CUBIC && max_nw > 32) {
@@ -85,22 +81,58 @@ void rxtab_defaults(const GeomLaunch& G, int max_nw, int& wc, int& ws) {
   }
 }
 
-void rxtab_default_tiles(int max_nw, int& wc, int& ws) {
-  if (max_nw <= 8) {  // 1-2 wave-splits; the others take shares of the channels
-    ws = 8;
+// Waves per split and splits by the waves of the busiest tile and the blocks
+// (tiles x frames) there are to run. Measured on a linear array with plane
+// waves and a sector with diverging waves, 3..31 waves, 188, 600, 1500 and 4000
+// blocks, us per pass:
+// - Fewer than 400 blocks leave most of the chip idle, so a block's own chain
+//   counts: 8 splits, as many waves in each as one round holds (the other
+//   splits take channel groups). 12 waves linear 69.0 -> 31.4, sector 49.3 ->
+//   31.5; 16 waves 69.1 -> 38.7; 25 waves 97.1 -> 56.4 against 8 x 4 and 16 x 4.
+// - 5..8 waves in one round of one split beat two splits of 4 (5 waves at 600
+//   blocks 30.8 -> 23.4), and from 1000 blocks with half the splits (5 waves,
+//   4000 blocks 126.9 -> 83.5; 8 waves, sector 156.9 -> 140.9). Keys' cubic
+//   needs the registers: 6..8 waves keep 4 x 8 there (8 waves at 1500 blocks
+//   70.8 against 73.5).
+// - 9..12 waves: one split of 12 up to 1000 blocks (600: 70.7 -> 54.3, 10 x 4
+//   and 16 x 4 within 3 %), two of 6 beyond (1500: 79.5 -> 73.3; 4000: within
+//   2 % either way).
+// - 3 and 4 waves: 4 splits from 2000 blocks (4000: 89.5 -> 77.7).
+// 13..32 waves from 400 blocks as before: 8 x 4 and 16 x 4 (8 x 8 is up to 30 %
+// faster on the linear array and as much slower on the sector). The kernels
+// that compute the receive geometry have only been measured with the shapes
+// for many blocks. More waves: 8 splits with the smallest waves-per-split
+// covering the busiest tile in one round (else 16 per round).
+void rxtab_default_tiles(int64_t blocks, int max_nw, bool cubic, bool otf, int& wc, int& ws) {
+  if (max_nw <= 4) {  // one wave-split; the others take shares of the channels
     wc = 4;
+    ws = max_nw > 2 && blocks >= 2000 && !otf ? 4 : 8;
     return;
   }
-  if (max_nw <= 16) {
-    ws = 4;
-    wc = 8;
+  if (max_nw <= 8) {
+    const bool wide_cubic = cubic && (max_nw > 6 ? blocks >= 400 : max_nw == 6 && blocks >= 1000 && blocks < 2000);
+    if (otf || wide_cubic) {
+      wc = 4;
+      ws = 8;
+      return;
+    }
+    wc = max_nw > 6 ? 8 : max_nw == 6 || blocks < 1000 ? 6 : 5;
+    ws = blocks < 1000 ? 8 : 4;
     return;
   }
   if (max_nw <= 32) {
-    // two channel groups of two 16-wave splits (the 3-D class, 25 waves:
-    // 52.3 ms against 55.9 ms at 8 x 4)
     ws = 4;
-    wc = 16;
+    if (otf)
+      wc = max_nw <= 16 ? 8 : 16;
+    else if (blocks < 400) {
+      wc = max_nw <= 12 ? 12 : 16;
+      ws = 8;
+    } else if (max_nw <= 12)
+      wc = blocks < 1000 ? 12 : 6;
+    else
+      // above 16: two channel groups of two 16-wave splits (the 3-D class, 25
+      // waves: 52.3 ms against 55.9 ms at 8 x 4)
+      wc = max_nw <= 16 ? 8 : 16;
     return;
   }
   ws = 8;
@@ -811,7 +843,7 @@ bool window_build(ustbx_plan* pl, hipError_t& err) {
   // dimension both: no tables for a plan that the gathering kernel runs anyway
   // (window_both_active)
   if (both && (G.W < 9 || (G.interp == USTBX_INTERP_CUBIC && G.F == 1) ||
-               (int64_t)(least >> 8) * ((G.F + 1) / 2) < 512))
+               (int64_t)(least >> 8) * ((G.F + 1) / 2) < 400))
     return true;
 
   size_t tiles_max = 0;
@@ -903,7 +935,23 @@ bool window_build(ustbx_plan* pl, hipError_t& err) {
     T.cl = cl;
     T.on = 1;
     G.win_max_nw = max_nw;
-    if (both) G.win_rx = nullptr;  // the plan's receive table, which may be rebuilt
+    if (both) {
+      G.win_rx = nullptr;  // the plan's receive table, which may be rebuilt
+      // how many tiles of the largest one's terms the plan holds
+      std::vector<int> tw((size_t)T.tiles), tc((size_t)T.tiles);
+      err = hipMemcpy(tw.data(), nw, sizeof(int) * tw.size(), hipMemcpyDeviceToHost);
+      if (err == hipSuccess) err = hipMemcpy(tc.data(), nc, sizeof(int) * tc.size(), hipMemcpyDeviceToHost);
+      if (err != hipSuccess) {
+        window_free(pl);
+        return false;
+      }
+      int64_t sum = 0, most = 1;
+      for (int t = 0; t < T.tiles; ++t) {
+        sum += (int64_t)tw[t] * tc[t];
+        most = std::max(most, (int64_t)tw[t] * tc[t]);
+      }
+      G.win_even = (int)(sum / most);
+    }
     return true;
   }
   window_free(pl);

@@ -127,6 +127,7 @@ struct GeomLaunch {
   // (auto_tiles), the other modes win_rx and win_ref.
   WinTiles win;
   int win_max_nw;        // largest wave count of a patch tile
+  int win_even;          // the plan's terms over those of its largest patch tile
   int max_nw;            // largest wave count of a variant-2 tile
   int auto_tiles;
   const float4* win_rx;
@@ -138,17 +139,27 @@ struct GeomLaunch {
 };
 
 // Whether a dimension-both plan runs window-staged: while no tile shape is
-// set, with enough waves per staged window's receive entry and enough blocks
-// to fill the chip, and linear or over several frames. Measured against the
-// gathering kernel over 50 random plans: from 9 waves and 512 blocks (rows of
-// 64 samples) 1.25-3.0 times as fast; 4-8 waves 0.8-1.05, 1-3 waves 0.2-0.9,
-// 60-300 blocks 0.2-0.8 (0.9-1.6 with over 45 waves); one cubic frame of the 75
-// plane waves 2.37 against 2.26 ms. Rows of 128 hold a quarter of the data at
-// twice the LDS per sample pair: twice the blocks.
+// set, with enough waves per staged window's receive entry, linear or over
+// several frames, and enough blocks. Two of these blocks fill a CU and each
+// lives long, so what counts is the plan's work in units of its largest tile
+// (a linear array's shallow tiles hold few channels): under 512 the chip waits
+// for the deepest tiles. Measured against the gathering kernel, one frame, W 9
+// to 26, 131072 to 393216 pixels: 128 elements at f/1.7, whose tiles hold half
+// the channels of the largest on average, 11-16 waves 0.8-0.9 times as fast
+// at 512 tiles, 1.06-1.14 at 1024, 1.25-1.4 at 1536; a sector over 64
+// elements, all tiles alike, 1.3-1.4 at 512. 9, 10 and 17-24 waves leave a
+// third of the wave slots empty: 0.9 and 1.05 at 1024 and 1280 tiles, 1.0-1.1 and
+// 1.1-1.3 on the sector at 640. More waves, 26: 1.03 at 720, 0.95 at 512. Up to
+// 8 waves 0.8-1.05 at any size; one cubic frame of 75 plane waves 2.37 against
+// 2.26 ms. Rows of 128 hold a quarter of the data at twice the LDS per sample
+// pair: twice the work.
 inline bool window_both_active(const GeomLaunch& G) {
-  return G.dim == 3 && G.win.on && G.variant == 2 && G.auto_tiles && !G.rx_otf && G.rx_table != nullptr &&
-         (G.interp != INTERP_CUBIC || G.F > 1) && G.win_max_nw >= 9 &&
-         (int64_t)G.win.tiles * ((G.F + 1) / 2) >= (G.win.row == 64 ? 512 : 1024);
+  if (!(G.dim == 3 && G.win.on && G.variant == 2 && G.auto_tiles && !G.rx_otf && G.rx_table != nullptr &&
+        (G.interp != INTERP_CUBIC || G.F > 1) && G.win_max_nw >= 9))
+    return false;
+  const int nw = G.win_max_nw;
+  const int need = nw <= 10 || (nw > 16 && nw <= 24) ? 640 : nw <= 16 ? 512 : 400;
+  return (int64_t)G.win_even * ((G.F + 1) / 2) >= (G.win.row == 64 ? need : 2 * need);
 }
 
 // Builds the transmit table of a plan (one lane per (wave, pixel)).
