@@ -333,11 +333,16 @@ int ustbx_batch_create(const ustbx_plan* const* plans, int32_t count, ustbx_batc
     }
   }
   int ws = 8, wc = 8;
-  if (nw_med <= 32) {
-    // us per batch against 8 x 4: images of 5, 11, 16 and 25 waves 254 ->
-    // 202, 431 -> 380, 583 -> 517 and 962 -> 794; volumes of 25 waves 22515 ->
-    // 19305, of 9 waves as before (3506 and 3509; 4 x 8 takes 4649 there)
-    wc = nw_med <= 16 ? 8 : 16;
+  if (nw_med <= 32 && b->otf) {
+    ws = 4;  // measured with 8 x 4 only
+  } else if (nw_med <= 32) {
+    // us per batch against 8 x 4, linear array and sector: 12 images of 255 x
+    // 255 pixels of 3 waves 353, 376 -> 292, 306; of 7 450, 503 -> 432, 478; of 11
+    // 613, 718 -> 563, 641; of 14 674, 813 -> 659, 777; of 20 889, 1155 -> 894,
+    // 1076; 5 of 100 x 200, 11 waves 213, 244 -> 140, 160. Volumes of 9 waves 752
+    // -> 705, of 25 (larger ones) 22515 -> 19305. 12 x 4 is 3 % faster
+    // than 6 x 8 on the large batches and 20-40 % slower on the small ones.
+    wc = nw_med <= 4 ? 4 : nw_med <= 8 ? 8 : nw_med <= 12 ? 6 : nw_med <= 16 ? 8 : 16;
   } else {
     const int need = (nw_med + 7) / 8;
     wc = need <= 4 ? 4 : need <= 6 ? 6 : need <= 8 ? 8 : need <= 10 ? 10 : need <= 12 ? 12 : 16;
