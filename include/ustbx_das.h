@@ -311,7 +311,9 @@ int ustbx_plan_set_variant(ustbx_plan* plan, int32_t variant, ustbx_status* st);
 /* Tile visiting order of variants 2 and 3 (no reference counterpart):
  * 0 = scan order; 1 = depth band by depth band within each XCD's share of the
  * scan lines (the default; it keeps the sample windows that co-resident
- * blocks read in L2). Results do not depend on it. */
+ * blocks read in L2; scan order where 64 does not divide the depths and the
+ * traces are small, the lines short or the scan a volume). Results do not
+ * depend on it. */
 int ustbx_plan_set_order(ustbx_plan* plan, int32_t order, ustbx_status* st);
 /* LDS staging of sample windows (no reference counterpart); results do not
  * depend on it. Dimension both on the receive table (variants 2, 3 only for
@@ -331,7 +333,7 @@ int ustbx_plan_stage_stats(const ustbx_plan* plan, int64_t* staged, int64_t* lis
 /* Current variant (or -1 for NULL) and its tile shape: 0 and 0 where the
  * library runs the plan on patch tiles with LDS-staged sample windows
  * (dimension both on variant 2 while no tile shape was set; 9 or more waves
- * and a few hundred tiles). Setting a tile shape selects the gathering kernel
+ * and the work of a few hundred full tiles of 256 pixels). Setting a tile shape selects the gathering kernel
  * of that shape. Dimension receive and none use patch tiles wherever the scan
  * and the weights allow, under variant 0. */
 int32_t ustbx_plan_variant(const ustbx_plan* plan, int32_t* wave_chunk, int32_t* split);
@@ -342,12 +344,11 @@ int32_t ustbx_plan_variant(const ustbx_plan* plan, int32_t* wave_chunk, int32_t*
  * ------------------------------------------------------------------------ */
 typedef struct ustbx_batch ustbx_batch;
 
-/* (Equality with a plan's own run: of a plan whose tile shape was set.)
- * count acquisitions, acquisition i beamformed with plans[i] (a plan may be
+/* count acquisitions, acquisition i beamformed with plans[i] (a plan may be
  * listed more than once; every plan must have variant-2 state -- see
  * ustbx_plan_set_variant -- and all share one interpolation). Dimension both;
- * each image equals ustbx_plan_run of its plan with the same tile shape, bit
- * for bit. The plans must outlive the batch. */
+ * each image equals ustbx_plan_run of its plan with the same tile shape set,
+ * bit for bit. The plans must outlive the batch. */
 int ustbx_batch_create(const ustbx_plan* const* plans, int32_t count, ustbx_batch** batch,
                        ustbx_status* st);
 /* Device buffers of every acquisition: ch[i] [F][W][N][L] complex64, out[i]
@@ -356,9 +357,10 @@ int ustbx_batch_set_io(ustbx_batch* batch, const void* const* ch, void* const* o
                        ustbx_status* st);
 /* Tile shape of the persistent kernel (0 = keep): waves per split (4, 5, 6,
  * 8, 10, 12, 16) and wave-splits per 64-pixel tile (4, 5 or 8). The default
- * follows the wave count below which half of the batch's work lies: up to 32
- * waves 4 splits of 8, else 8 splits covering it in one round. Drops a
- * captured graph. */
+ * follows the wave count below which half of the batch's work lies: 8 splits of
+ * 4 (up to 4 waves), 8 (8), 6 (12), 8 (16) or 16 (32) waves, above that 8
+ * splits covering it in one round; 4 splits of 8 up to 32 waves where an
+ * acquisition computes its receive state in place. Drops a captured graph. */
 int ustbx_batch_set_tiles(ustbx_batch* batch, int32_t wave_chunk, int32_t split, ustbx_status* st);
 /* Enqueues the batch on stream: a counter-reset kernel and the persistent
  * kernel; allocates nothing and can be captured in a hipGraph. Launches of

@@ -7,10 +7,10 @@
 // waves per SIMD. Bound: VALU issue (12 instructions per 64 terms, half the
 // time) and the latency between a step's barrier and its receive entries.
 // Against the gathering kernel:
-//   volume, 1024 channels x 25 waves on 96 x 96 x 128 voxels: 29.9 -> 9.9 ms
+//   volume, 1024 channels x 25 waves on 96 x 96 x 128 voxels: 29.9 -> 10.1 ms
 //     (two groups of 13; one group of 16 in two rounds 11.5, of 25 at 3 waves
 //     per SIMD 9.8; four groups of 7: 14.1)
-//   cine, 128 channels x 11 waves x 16 frames on 301 x 387 pixels: 1.08 -> 0.60
+//   cine, 128 channels x 11 waves x 16 frames on 301 x 387 pixels: 1.08 -> 0.58
 //     ms (two groups of 6, 2 frames; one group of 12: 0.69; 4 frames: 1.0)
 #pragma once
 #include "das_window.h"
