@@ -312,7 +312,7 @@ int ustbx_plan_set_variant(ustbx_plan* plan, int32_t variant, ustbx_status* st);
  * 0 = scan order; 1 = depth band by depth band within each XCD's share of the
  * scan lines (the default; it keeps the sample windows that co-resident
  * blocks read in L2; scan order where 64 does not divide the depths and the
- * traces are small, the lines short or the scan a volume). Results do not
+ * image or its traces are small, the lines short or the scan a volume). Results do not
  * depend on it. */
 int ustbx_plan_set_order(ustbx_plan* plan, int32_t order, ustbx_status* st);
 /* LDS staging of sample windows (no reference counterpart); results do not

@@ -563,11 +563,14 @@ std::vector<int> band_major_order(const GeomLaunch& G, int tiles, int shares) {
     // lines of a depth count that 64 does not divide: a tile may end one line
     // and begin the next; it goes by the depth of its first pixel. Worth it
     // for images whose frame of traces is well beyond an XCD's 4 MB L2, with
-    // three bands or more. Against pixel order, dimension both, 40 such plans of
-    // 10-116 MB ran 0.98-1.31 times as fast (1.05 in the mean), below 10 MB
+    // three bands or more and, in dimension both, more tiles than are resident
+    // at once. Against pixel order, dimension both, 30 such plans of 10-116 MB
+    // ran 1.0-1.31 times as fast (1.06 in the mean), under 1000 tiles 0.90-1.16
+    // (193 x 321 pixels, 128 channels RF, 20 waves 103 -> 114 us), below 10 MB
     // 0.97-1.04, 23 volumes 0.94-1.03 at any size; dimension transmit
     // 0.99-1.7, below 10 MB 0.97-1.03, lines of 129 and 131 depths 0.72 and 0.82.
-    if (sc.n2 > 1 || sc.n0 < 192 || (int64_t)G.L * G.N * G.W * 8 < 10 * 1000 * 1000) return order;
+    if (sc.n2 > 1 || sc.n0 < 192 || (int64_t)G.L * G.N * G.W * 8 < 10 * 1000 * 1000 || (G.dim == 3 && tiles < 1000))
+      return order;
     const int64_t n0 = sc.n0;
     const int q = tiles / shares, r = tiles % shares;
     for (int k = 0; k < shares; ++k) {
