@@ -564,8 +564,8 @@ std::vector<int> band_major_order(const GeomLaunch& G, int tiles, int shares) {
     // and begin the next; it goes by the depth of its first pixel. Worth it
     // for images whose frame of traces is well beyond an XCD's 4 MB L2, with
     // three bands or more and, in dimension both, more tiles than are resident
-    // at once. Against pixel order, dimension both, 30 such plans of 10-116 MB
-    // ran 1.0-1.31 times as fast (1.06 in the mean), under 1000 tiles 0.90-1.16
+    // at once. Against pixel order, dimension both, 23 such plans of 10-116 MB
+    // ran 1.0-1.31 times as fast (1.07 in the mean), under 1000 tiles 0.90-1.16
     // (193 x 321 pixels, 128 channels RF, 20 waves 103 -> 114 us), below 10 MB
     // 0.97-1.04, 23 volumes 0.94-1.03 at any size; dimension transmit
     // 0.99-1.7, below 10 MB 0.97-1.03, lines of 129 and 131 depths 0.72 and 0.82.
