@@ -729,13 +729,17 @@ struct ConvTable {
   double* h = nullptr;  // [L], then g (the allocation's start)
   float* g = nullptr;   // [N]
   unsigned long long last_use = 0;
+  bool captured = false;  // a captured graph reads it: never released
 };
-constexpr int kMaxConvTables = 64;  // per device; at most 128 KiB each
+constexpr int kMaxConvTables = 64;  // per device, without the captured ones; at most 128 KiB each
 std::map<std::pair<int, int>, ConvTable> g_conv;
 
 // The spectrum table of length L on device dev (the current one): built once
 // (and waited for on the caller's stream); the least recently used beyond
-// kMaxConvTables is released after a device synchronisation. Caller holds g_mu.
+// kMaxConvTables is released after a device synchronisation. A table that a
+// call under stream capture uses is read by every later replay of its graph, so
+// it stays for the life of the process (at most one per length, 0.36 GB if all
+// 8190 lengths were captured). Caller holds g_mu.
 hipError_t conv_table(int dev, int L, hipStream_t s, const float** out) {
   const auto key = std::make_pair(dev, L);
   auto it = g_conv.find(key);
@@ -743,7 +747,7 @@ hipError_t conv_table(int dev, int L, hipStream_t s, const float** out) {
     int n = 0;
     auto lru = g_conv.end();
     for (auto c = g_conv.begin(); c != g_conv.end(); ++c) {
-      if (c->first.first != dev) continue;
+      if (c->first.first != dev || c->second.captured) continue;
       ++n;
       if (lru == g_conv.end() || c->second.last_use < lru->second.last_use) lru = c;
     }
@@ -769,6 +773,9 @@ hipError_t conv_table(int dev, int L, hipStream_t s, const float** out) {
     it = g_conv.emplace(key, t).first;
   }
   it->second.last_use = ++g_plan_clock;
+  hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
+  if (hipStreamIsCapturing(s, &cap) != hipSuccess) (void)hipGetLastError();  // the launch will say
+  if (cap != hipStreamCaptureStatusNone) it->second.captured = true;
   *out = it->second.g;
   return hipSuccess;
 }
