@@ -626,6 +626,27 @@ __device__ __forceinline__ void conv_fft(float2 (&v)[PT], float2* buf, const flo
   if (N == 16384) conv_stage<N, PT, 4, true>(v, buf, twg + kTw4096, 4096, s);
 }
 
+// The sum of the wave's v, in lane 63.
+__device__ __forceinline__ float wave_sum63(float v) {
+  auto step = [&](auto ctrl) {
+    v += __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), decltype(ctrl)::value, 0xf, 0xf, true));
+  };
+  step(std::integral_constant<int, 0x111>());  // row_shr 1, 2, 4, 8: lane 15 of each row of 16
+  step(std::integral_constant<int, 0x112>());
+  step(std::integral_constant<int, 0x114>());
+  step(std::integral_constant<int, 0x118>());
+  step(std::integral_constant<int, 0x142>());  // row_bcast 15, 31: the rows before
+  step(std::integral_constant<int, 0x143>());
+  return v;
+}
+
+// Whether a trace's sum of squares is in the range of FP32 with room to spare,
+// and the exponent of its square root there.
+__device__ __forceinline__ bool energy_ok(float e) { return e >= 1e-30f && e <= 1e37f; }
+__device__ __forceinline__ int norm_exponent(float e) {
+  return __builtin_amdgcn_readfirstlane(((__float_as_int(e) >> 23) - 127) >> 1);
+}
+
 template <int N>
 __global__ __launch_bounds__(N / conv_points(N), 4) void hilbert_conv_kernel(const float* __restrict__ rf,
                                                                          float2* __restrict__ z,
@@ -635,7 +656,8 @@ __global__ __launch_bounds__(N / conv_points(N), 4) void hilbert_conv_kernel(con
   constexpr int PT = conv_points(N), NT = N / PT;
   __shared__ float2 buf[N + N / 8];
   __shared__ float2 tws[kTw512];
-  __shared__ int nonfinite[NT / 64];
+  __shared__ float2 energy[NT / 64];
+  __shared__ uint2 peak[NT / 64];
   const int tid = threadIdx.x;
   const size_t ta = 2 * (size_t)blockIdx.x;
   const bool has_b = (long long)ta + 1 < traces;
@@ -643,27 +665,70 @@ __global__ __launch_bounds__(N / conv_points(N), 4) void hilbert_conv_kernel(con
   const float* __restrict__ xb = xa + L;
   // 2 L - 1 <= N, so the points m >= PT / 2 (beyond N / 2 >= L) are zeros
   float2 x[PT / 2];
-  float bad_a = 0.0f, bad_b = 0.0f;  // NaN where a sample is not finite
+  float sa = 0.0f, sb = 0.0f;
 #pragma unroll
   for (int m = 0; m < PT / 2; ++m) {
     const int i = tid + m * NT;
     x[m] = make_float2(i < L ? xa[i] : 0.0f, i < L && has_b ? xb[i] : 0.0f);
-    bad_a += x[m].x * 0.0f;
-    bad_b += x[m].y * 0.0f;
+    sa = fmaf(x[m].x, x[m].x, sa);
+    sb = fmaf(x[m].y, x[m].y, sb);
   }
   for (int i = tid; i < kTw512; i += NT) tws[i] = twg[i];
-  // a trace with a sample that is not finite is NaN throughout (as its own
-  // FFT would make it) and must not reach the other trace of the pair
-  const unsigned long long am = __ballot(bad_a != 0.0f), bm = __ballot(bad_b != 0.0f);
-  if ((tid & 63) == 0) nonfinite[tid >> 6] = (am ? 1 : 0) | (bm ? 2 : 0);
+  // The transform's rounding is relative to the pair's norm, so each trace is
+  // brought to a norm in [1, 2) by its own power of two (exact; a trace next to
+  // one 80 dB stronger would otherwise lose 13 bits).
+  sa = wave_sum63(sa);
+  sb = wave_sum63(sb);
+  if ((tid & 63) == 63) energy[tid >> 6] = make_float2(sa, sb);
   __syncthreads();
-  int bad = 0;
+  float2 en = energy[0];
 #pragma unroll
-  for (int w = 0; w < NT / 64; ++w) bad |= nonfinite[w];
+  for (int w = 1; w < NT / 64; ++w) {
+    en.x += energy[w].x;
+    en.y += energy[w].y;
+  }
+  int bad = 0;
+  int ea = norm_exponent(en.x), eb = norm_exponent(en.y);  // scale by 2^-ea, 2^-eb
+  int ra = ea, rb = eb;                                    // and back
+  if (!energy_ok(en.x) || !energy_ok(en.y)) {  // the same for the whole block
+    // a zero trace, squares out of range, or samples that are not finite: by
+    // the largest magnitude times sqrt(L), the norm's bound. A trace with a sample that is not finite is NaN
+    // throughout (as its own FFT would make it) and must not reach the other
+    // trace of the pair; a zero trace stays zero.
+    unsigned pa = 0, pb = 0;
+#pragma unroll
+    for (int m = 0; m < PT / 2; ++m) {
+      pa = max(pa, __float_as_uint(x[m].x) & 0x7fffffffu);
+      pb = max(pb, __float_as_uint(x[m].y) & 0x7fffffffu);
+    }
+#pragma unroll
+    for (int o = 32; o > 0; o >>= 1) {
+      pa = max(pa, (unsigned)__shfl_xor((int)pa, o));
+      pb = max(pb, (unsigned)__shfl_xor((int)pb, o));
+    }
+    if ((tid & 63) == 0) peak[tid >> 6] = make_uint2(pa, pb);
+    __syncthreads();
+#pragma unroll
+    for (int w = 0; w < NT / 64; ++w) {
+      pa = max(pa, peak[w].x);
+      pb = max(pb, peak[w].y);
+    }
+    bad = (pa >= 0x7f800000u ? 1 : 0) | (pb >= 0x7f800000u ? 2 : 0);
+    const int half = (32 - __builtin_clz((unsigned)L)) / 2;
+    if (!energy_ok(en.x)) {
+      ea = (int)(pa >> 23) - 126 + half;
+      ra = pa ? ea : -400;
+    }
+    if (!energy_ok(en.y)) {
+      eb = (int)(pb >> 23) - 126 + half;
+      rb = pb ? eb : -400;
+    }
+  }
   float2 v[PT];
 #pragma unroll
   for (int m = 0; m < PT; ++m)
-    v[m] = m < PT / 2 ? make_float2(bad & 1 ? 0.0f : x[m < PT / 2 ? m : 0].x, bad & 2 ? 0.0f : x[m < PT / 2 ? m : 0].y)
+    v[m] = m < PT / 2 ? make_float2(bad & 1 ? 0.0f : ldexpf(x[m < PT / 2 ? m : 0].x, -ea),
+                                    bad & 2 ? 0.0f : ldexpf(x[m < PT / 2 ? m : 0].y, -eb))
                       : make_float2(0.0f, 0.0f);
   conv_fft<N, PT>(v, buf, tws, twg, -1.0f);
 #pragma unroll
@@ -681,8 +746,8 @@ __global__ __launch_bounds__(N / conv_points(N), 4) void hilbert_conv_kernel(con
       // 16 points per thread: the samples again (L2) instead of 16 registers
       const float a = PT == 16 ? xa[i] : x[m].x, b = PT == 16 ? (has_b ? xb[i] : 0.0f) : x[m].y;
       const float nan = __builtin_nanf("");
-      za[i] = bad & 1 ? make_float2(nan, nan) : make_float2(a, v[m].x);
-      if (has_b) zb[i] = bad & 2 ? make_float2(nan, nan) : make_float2(b, v[m].y);
+      za[i] = bad & 1 ? make_float2(nan, nan) : make_float2(a, ldexpf(v[m].x, ra));
+      if (has_b) zb[i] = bad & 2 ? make_float2(nan, nan) : make_float2(b, ldexpf(v[m].y, rb));
     }
   }
 }
