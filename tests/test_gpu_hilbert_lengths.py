@@ -40,3 +40,14 @@ def test_non_finite_trace_stays_alone(cuda, L, bad):
     assert np.isnan(got[[1, 4]].real).all() and np.isnan(got[[1, 4]].imag).all()
     ref = O.hilbert(x[[0, 2, 3]].astype(np.float64), axis=-1)
     assert np.max(np.abs(got[[0, 2, 3]] - ref)) <= TOL * float(np.max(np.abs(ref)))
+
+
+def test_more_traces_than_one_grid(cuda):
+    """A grid holds fewer than 2^32 threads: 2^27 traces of the shortest transform."""
+    L, traces = 5, (1 << 27) + 12345
+    print(f"case hilbert L={L} traces={traces}", flush=True)
+    x = torch.randn((traces, L), device=cuda, generator=torch.Generator(cuda).manual_seed(5))
+    z = hilbert(x)
+    for at in (0, (1 << 27) - 200, traces - 200):  # even: the same pairs
+        at -= at % 2
+        assert torch.equal(z[at:at + 200], hilbert(x[at:at + 200].contiguous()))

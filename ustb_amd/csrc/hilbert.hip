@@ -848,9 +848,16 @@ hipError_t conv_table(int dev, int L, hipStream_t s, const float** out) {
 template <int N>
 hipError_t launch_hilbert_conv(const float* rf, float2* z, long long traces, int L, const float2* tw, const float* g,
                                hipStream_t s) {
-  hipLaunchKernelGGL(hilbert_conv_kernel<N>, dim3((unsigned)((traces + 1) / 2)), dim3(N / conv_points(N)), 0, s, rf, z,
-                     tw, g, traces, L);
-  return hipGetLastError();
+  constexpr int NT = N / conv_points(N);
+  constexpr long long kMost = 2 * (0xFFFFFFFFll / NT);  // a grid holds fewer than 2^32 threads
+  hipError_t e = hipSuccess;
+  for (long long t = 0; e == hipSuccess && t < traces; t += kMost) {
+    const long long n = traces - t < kMost ? traces - t : kMost;
+    hipLaunchKernelGGL(hilbert_conv_kernel<N>, dim3((unsigned)((n + 1) / 2)), dim3(NT), 0, s, rf + t * L, z + t * L,
+                       tw, g, n, L);
+    e = hipGetLastError();
+  }
+  return e;
 }
 
 template <int N>
