@@ -68,3 +68,21 @@ def test_non_finite_weights_delays_and_samples(cuda):
     fine = torch.isfinite(ref.real) & torch.isfinite(ref.imag)
     assert fine.any() and not fine.all()
     assert (got[fine] - ref[fine]).abs().max() <= 1e-6 * ref[fine].abs().max()
+
+
+@pytest.mark.parametrize("interp,F", [(0, 1), (0, 3), (1, 1)])
+@pytest.mark.parametrize("t0", [0.9e-3, 3.2e-3, 3.2e-2])
+def test_large_phases(cuda, t0, interp, F):
+    """Delays of any size: around 3e4, 1e5 and 1e6 rad, the first on both sides of where the rotation changes form."""
+    print(f"case matrix both phases t0={t0} interp={interp} F={F}", flush=True)
+    rng = np.random.default_rng(11)
+    P, N, W, L, fd = 300, 9, 11, 400, 5.2e6
+    q = dict(ch=(rng.standard_normal((F, W, N, L)) + 1j * rng.standard_normal((F, W, N, L))).astype(np.complex64),
+             fs=2.6e6, t0=t0, tx_apo=rng.uniform(0.1, 1.0, (W, P)).astype(np.float32),
+             rx_apo=rng.uniform(0.1, 1.0, (N, P)).astype(np.float32),
+             tx_delay=(0.4 * t0 + np.linspace(0.0, 1.4e-4, P) * rng.uniform(0.5, 1.0, (W, 1))).astype(np.float32),
+             rx_delay=(0.6 * t0 + rng.uniform(0.0, 1e-5, (N, P))).astype(np.float32))
+    if t0 == 0.9e-3:
+        p = 2 * np.pi * fd * (q["tx_delay"][:, None] + q["rx_delay"][None])
+        assert (p < 32768).any() and (p > 32768).any()
+    _close(*_images(cuda, q, fd, interp=interp), N * W)

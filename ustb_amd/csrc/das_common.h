@@ -168,6 +168,23 @@ __device__ __forceinline__ void keys_weights(float b, float& c0, float& c1,
   c3 = 0.5f * b3 - 0.5f * b2;
 }
 
+// Gather and weight one term for one frame.
+template <int INTERP>
+__device__ __forceinline__ float2 mat_contrib(const Term& t,
+                                              const float2* __restrict__ trace) {
+  if (INTERP == INTERP_LINEAR) {
+    return dasc_contrib(t, load_pair(trace, t.n0));
+  } else {
+    const float4 lo = load_pair(trace, t.n0 - 1);
+    const float4 hi = load_pair(trace, t.n0 + 1);
+    float c0, c1, c2, c3;
+    keys_weights(t.b, c0, c1, c2, c3);
+    const float sr = ((c0 * lo.x + c1 * lo.z) + c2 * hi.x) + c3 * hi.z;
+    const float si = ((c0 * lo.y + c1 * lo.w) + c2 * hi.y) + c3 * hi.w;
+    return make_float2(t.wr * sr - t.wi * si, t.wr * si + t.wi * sr);
+  }
+}
+
 __device__ __forceinline__ float2 cmul(float2 a, float2 b) {
   return make_float2(a.x * b.x - a.y * b.y, a.x * b.y + a.y * b.x);
 }

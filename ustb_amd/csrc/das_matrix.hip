@@ -92,23 +92,6 @@ __device__ __forceinline__ float2 py_contrib(const PyTerm& t, const float2* __re
   return make_float2(t.c * vr - t.s * vi, t.c * vi + t.s * vr);
 }
 
-// Gather and weight one term for one frame.
-template <int INTERP>
-__device__ __forceinline__ float2 mat_contrib(const Term& t,
-                                              const float2* __restrict__ trace) {
-  if (INTERP == INTERP_LINEAR) {
-    return dasc_contrib(t, load_pair(trace, t.n0));
-  } else {
-    const float4 lo = load_pair(trace, t.n0 - 1);
-    const float4 hi = load_pair(trace, t.n0 + 1);
-    float c0, c1, c2, c3;
-    keys_weights(t.b, c0, c1, c2, c3);
-    const float sr = ((c0 * lo.x + c1 * lo.z) + c2 * hi.x) + c3 * hi.z;
-    const float si = ((c0 * lo.y + c1 * lo.w) + c2 * hi.y) + c3 * hi.w;
-    return make_float2(t.wr * sr - t.wi * si, t.wr * si + t.wi * sr);
-  }
-}
-
 // Unit loop over channels [nb, ne) for fixed (pixel, wave), U channels per
 // step: rx loads of the U channels are issued first, then the gathers, then
 // the accumulation in channel order (das_c's order within the group).

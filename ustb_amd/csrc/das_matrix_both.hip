@@ -14,10 +14,12 @@
 // (two-sum) and p = wd c - r (one FMA), so p = wd td + wd rd - (r + wd e): the
 // rotation is exp(i wd td) exp(i wd rd) exp(i D), D = -(r + wd e), |D| below
 // 2^-23 |p|. The first two are formed once per (pixel, wave) and (pixel,
-// channel) with the FP64 argument of sincos_wd, the last to second order (its
-// third is below 1e-9 for |p| < 10^4). So a term keeps das_c's rounded phase
-// (the result is das_c's within FP32 rounding) at 11 instructions instead of
-// a sine and cosine of an unreduced argument (about 45).
+// channel) with the FP64 argument of sincos_wd, the last to second order: up to
+// |p| = 32768, |D| < 2^-8, what that leaves out is below 1e-8, a sixth of the
+// rounding of the rotation itself. So a term keeps das_c's rounded phase (the
+// result is das_c's within FP32 rounding) at 11 instructions instead of a sine
+// and cosine of an unreduced argument (about 45). A tile with larger phases is
+// summed from das_c's own terms (dasc_sum).
 //
 // Bound by VALU issue (about 35 instructions per 64 terms). Against
 // das_matrix_kernel, whose lanes take a sine, a cosine and two branches per
@@ -46,7 +48,7 @@ struct MatBoth {
   float2* out;
   int L, N, W, F, P;
   float fs, t0, wd, lo;
-  int frame_bytes;
+  int frame_bytes, edge;
 };
 
 // exp(i D) T for das_c's phase of the term (see above); d0 receives c.
@@ -61,12 +63,45 @@ __device__ __forceinline__ float2 dasc_rotation(float2 T, float td, float rd, fl
   return make_float2(__builtin_fmaf(-D, T.y, h * T.x), __builtin_fmaf(D, T.x, h * T.y));
 }
 
+constexpr float kNearPhase = 32768.0f;  // rad: |D| < 2^-8
+
+// The channels n = s, s + kWS, ... of pixel p summed from das_c's terms
+// (das_c.cpp:366-399), for tiles outside the range of the split rotation.
+template <int SM, bool IQ, int FC>
+__device__ __forceinline__ void dasc_sum(const MatBoth& A, const int* list, int nw, int s, unsigned p, int f0, int nfr,
+                                         float2 (&acc)[FC]) {
+  constexpr int INTERP = SM == SM_CUBIC ? INTERP_CUBIC : INTERP_LINEAR;
+  const size_t PS = (size_t)A.P, LN = (size_t)A.L * A.N;
+#pragma unroll
+  for (int f = 0; f < FC; ++f) acc[f] = make_float2(0.0f, 0.0f);
+#pragma unroll 1
+  for (int n = s; n < A.N; n += kWS) {
+    const float ra = (A.rx_apo + (size_t)n * PS)[p], rd = (A.rx_delay + (size_t)n * PS)[p];
+    if (!__any(ra != 0.0f)) continue;
+#pragma unroll 1
+    for (int k = 0; k < nw; ++k) {
+      const int w = __builtin_amdgcn_readfirstlane(list[k]);
+      const float ta = (A.tx_apo + (size_t)w * PS)[p], td = (A.tx_delay + (size_t)w * PS)[p];
+      if (ta != 0.0f && ra != 0.0f) {
+        const Term t = dasc_term<INTERP, IQ>(td, rd, ta, ra, A.t0, A.fs, A.wd, A.L, A.edge);
+        if (t.valid) {
+          const float2* trace = reinterpret_cast<const float2*>(A.ch) + (size_t)f0 * LN * A.W + (size_t)w * LN + (size_t)n * A.L;
+#pragma unroll
+          for (int f = 0; f < FC; ++f)
+            if (f < nfr) cadd(acc[f], mat_contrib<INTERP>(t, trace + (size_t)f * LN * A.W));
+        }
+      }
+    }
+  }
+}
+
 template <int SM, bool IQ, int FC>
 __global__ __launch_bounds__(64 * kWS) void das_matrix_both_kernel(MatBoth A) {
   constexpr int NL = SM == SM_CUBIC ? 2 : 1;
   __shared__ float2 red[kWS][64];
   __shared__ int list[kMaxList];
   __shared__ int count;
+  __shared__ int far_tile;
   const int lane = threadIdx.x & 63;
   const int s = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6);
   const int tile = xcd_tile((int)blockIdx.x, (int)gridDim.x);
@@ -93,7 +128,10 @@ __global__ __launch_bounds__(64 * kWS) void das_matrix_both_kernel(MatBoth A) {
       if (on) list[n + __popcll(m & ((1ull << lane) - 1ull))] = b + lane;
       n += __popcll(m);
     }
-    if (lane == 0) count = n;
+    if (lane == 0) {
+      count = n;
+      far_tile = 0;
+    }
   }
   __syncthreads();
   const int nw = __builtin_amdgcn_readfirstlane(count);
@@ -115,12 +153,14 @@ __global__ __launch_bounds__(64 * kWS) void das_matrix_both_kernel(MatBoth A) {
   float2 acc[FC];
 #pragma unroll
   for (int f = 0; f < FC; ++f) acc[f] = make_float2(0.0f, 0.0f);
-  for (int k0 = 0; g < cg && k0 < nw; k0 += wsp * kWC) {
+  bool far = false;  // wave-uniform: a phase beyond the split rotation's range
+  for (int k0 = 0; g < cg && k0 < nw && !far; k0 += wsp * kWC) {
     const int nj = __builtin_amdgcn_readfirstlane(min(kWC, max(0, (nw - k0 - sw + wsp - 1) / wsp)));
     if (nj == 0) break;
     float td[kWC];
     float2 T[kWC];
     int wb[kWC];
+    float tmax = 0.0f;  // largest |delay| of the round's waves
 #pragma unroll
     for (int j = 0; j < kWC; ++j) {
       td[j] = kFar;
@@ -132,6 +172,7 @@ __global__ __launch_bounds__(64 * kWS) void das_matrix_both_kernel(MatBoth A) {
         const float ta = (A.tx_apo + (size_t)w * PS)[p], d = (A.tx_delay + (size_t)w * PS)[p];
         if (ta != 0.0f) {
           td[j] = d;
+          if (IQ) tmax = fmaxf(tmax, fabsf(d));
           float sv = 0.0f, cv = 1.0f;
           if (IQ) sincos_wd(wd, d, sv, cv);
           T[j] = make_float2(ta * cv, IQ ? ta * sv : 0.0f);
@@ -140,6 +181,12 @@ __global__ __launch_bounds__(64 * kWS) void das_matrix_both_kernel(MatBoth A) {
     }
     // the next channel's receive rows are in flight during this one's terms
     float ran = (A.rx_apo + (size_t)min(g, A.N - 1) * PS)[p], rdn = (A.rx_delay + (size_t)min(g, A.N - 1) * PS)[p];
+    // a test here spares most far tiles the round; one per channel costs 3 %
+    float rmax = ran != 0.0f ? fabsf(rdn) : 0.0f;
+    if (IQ) {
+      far = __any(fabsf(wd) * (tmax + rmax) > kNearPhase);
+      if (far) break;
+    }
     for (int n = g; n < A.N; n += cg) {
       const float ra = ran, rdv = rdn;
       const size_t nx = (size_t)min(n + cg, A.N - 1) * PS;
@@ -147,6 +194,7 @@ __global__ __launch_bounds__(64 * kWS) void das_matrix_both_kernel(MatBoth A) {
       rdn = (A.rx_delay + nx)[p];
       const bool ron = ra != 0.0f;
       if (!__any(ron)) continue;  // wave-uniform
+      if (IQ) rmax = ron ? fmaxf(rmax, fabsf(rdv)) : rmax;
       const float rd = ron ? rdv : kFar;
       const int nb = n * lst;
       float2 part[FC];
@@ -216,6 +264,12 @@ __global__ __launch_bounds__(64 * kWS) void das_matrix_both_kernel(MatBoth A) {
         acc[f] = any ? v : acc[f];
       }
     }
+    if (IQ) far = __any(fabsf(wd) * (tmax + rmax) > kNearPhase);
+  }
+  if (IQ) {
+    if (far && lane == 0) far_tile = 1;
+    __syncthreads();
+    if (__builtin_amdgcn_readfirstlane(far_tile)) dasc_sum<SM, IQ, FC>(A, list, nw, s, p, f0, nfr, acc);
   }
 #pragma unroll
   for (int f = 0; f < FC; ++f) {
@@ -266,6 +320,7 @@ hipError_t launch_das_matrix_both(const MatLaunch& m, hipStream_t s) {
   A.wd = m.wd;
   A.lo = m.edge == EDGE_PYTHON && m.interp == INTERP_LINEAR ? 0.0f : 1.0f;
   A.frame_bytes = m.L * m.N * m.W * 8;
+  A.edge = m.edge;
   if (m.interp == INTERP_CUBIC)
     return m.wd != 0.0f ? matrix_both_t<SM_CUBIC, true>(A, s) : matrix_both_t<SM_CUBIC, false>(A, s);
   return m.wd != 0.0f ? matrix_both_t<SM_LINEAR, true>(A, s) : matrix_both_t<SM_LINEAR, false>(A, s);
