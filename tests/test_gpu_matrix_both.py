@@ -8,6 +8,7 @@ import pytest
 
 torch = pytest.importorskip("torch")
 
+from oracle import oracle as O
 from tests.cases import matrix_problem
 from ustb_amd import ops
 
@@ -86,3 +87,31 @@ def test_large_phases(cuda, t0, interp, F):
         p = 2 * np.pi * fd * (q["tx_delay"][:, None] + q["rx_delay"][None])
         assert (p < 32768).any() and (p > 32768).any()
     _close(*_images(cuda, q, fd, interp=interp), N * W)
+
+
+@pytest.mark.parametrize("interp", [0, 1])
+@pytest.mark.parametrize("fd", [0.0, 0.13])
+def test_infinities_stay_infinities(cuda, fd, interp):
+    """Infinite samples and weights, and weights whose product is moderate, give das_c's infinities and NaN."""
+    print(f"case matrix both infinities fd={fd} interp={interp}", flush=True)
+    q = matrix_problem(seed=6, P=260, N=9, W=6, F=5, L=80)
+    q["ch"].imag[0, 3, 5, 20] = np.inf
+    q["ch"].real[0, 2, 1, 40] = -np.inf
+    q["ch"].real[1, 2, 1, 41:43] = np.inf
+    q["rx_apo"][2, 230:240] = np.inf
+    q["tx_apo"][1, 235:250] = -np.inf
+    q["tx_apo"][:, 120:128] = 3e37       # with samples of 20: beyond FP32 before the receive weight
+    q["rx_apo"][:, 120:128] = 1e-37
+    q["ch"][2] *= 20.0
+    got, ref = _images(cuda, q, fd, interp=interp)
+    a, b = torch.view_as_real(got), torch.view_as_real(ref)
+    fine = torch.isfinite(b)
+    assert torch.isinf(b).any() and torch.isnan(b).any() and fine[2, 120:128].all()
+    assert torch.equal(torch.where(fine, 0.0, a).nan_to_num(7.0), torch.where(fine, 0.0, b).nan_to_num(7.0))
+    if fd == 0.0:  # no phase: FP64 is the better reference (das_c's order is 7e-7 from it at the moderate products)
+        ex = O.beamform_fp64(q["ch"], q["fs"], q["t0"], q["tx_apo"], q["rx_apo"], q["tx_delay"], q["rx_delay"], fd, 3,
+                             interp="cubic" if interp else "linear", w0=0.0, index="fp32")
+        b = torch.view_as_real(torch.from_numpy(np.ascontiguousarray(ex.reshape(got.shape))).to(cuda))
+    for f in range(5):
+        err = (a[f] - b[f])[fine[f]].abs().max() / b[f][fine[f]].abs().max()
+        assert err.item() <= 6e-8 * (4 + 54 ** 0.5)

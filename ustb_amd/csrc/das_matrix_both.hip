@@ -66,7 +66,8 @@ __device__ __forceinline__ float2 dasc_rotation(float2 T, float td, float rd, fl
 constexpr float kNearPhase = 32768.0f;  // rad: |D| < 2^-8
 
 // The channels n = s, s + kWS, ... of pixel p summed from das_c's terms
-// (das_c.cpp:366-399), for tiles outside the range of the split rotation.
+// (das_c.cpp:366-399), for tiles outside the range of the split rotation or
+// with sums that are not finite.
 template <int SM, bool IQ, int FC>
 __device__ __forceinline__ void dasc_sum(const MatBoth& A, const int* list, int nw, int s, unsigned p, int f0, int nfr,
                                          float2 (&acc)[FC]) {
@@ -101,7 +102,7 @@ __global__ __launch_bounds__(64 * kWS) void das_matrix_both_kernel(MatBoth A) {
   __shared__ float2 red[kWS][64];
   __shared__ int list[kMaxList];
   __shared__ int count;
-  __shared__ int far_tile;
+  __shared__ int far_tile, redo;
   const int lane = threadIdx.x & 63;
   const int s = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6);
   const int tile = xcd_tile((int)blockIdx.x, (int)gridDim.x);
@@ -130,7 +131,7 @@ __global__ __launch_bounds__(64 * kWS) void das_matrix_both_kernel(MatBoth A) {
     }
     if (lane == 0) {
       count = n;
-      far_tile = 0;
+      far_tile = redo = 0;
     }
   }
   __syncthreads();
@@ -280,8 +281,30 @@ __global__ __launch_bounds__(64 * kWS) void das_matrix_both_kernel(MatBoth A) {
 #pragma unroll
       for (int k = 1; k < kWS; ++k) cadd(v, red[k][lane]);
       A.out[(size_t)(f0 + f) * PS + p] = v;
+      if (!(isfinite(v.x) && isfinite(v.y))) redo = 1;
     }
     __syncthreads();
+  }
+  // Infinities: the split weights and x0 + b (x1 - x0) turn some into NaN that
+  // das_c's products keep, and weights far from 1 can overflow in between.
+  // Sums that are not finite are das_c's.
+  if (__builtin_amdgcn_readfirstlane(redo)) {
+    dasc_sum<SM, IQ, FC>(A, list, nw, s, p, f0, nfr, acc);
+#pragma unroll
+    for (int f = 0; f < FC; ++f) {
+      red[s][lane] = acc[f];
+      __syncthreads();
+      if (s == 0 && active && f < nfr) {
+        float2* o = A.out + (size_t)(f0 + f) * PS + p;
+        if (!(isfinite(o->x) && isfinite(o->y))) {
+          float2 v = red[0][lane];
+#pragma unroll
+          for (int k = 1; k < kWS; ++k) cadd(v, red[k][lane]);
+          *o = v;
+        }
+      }
+      __syncthreads();
+    }
   }
 }
 
