@@ -97,7 +97,17 @@ struct WinKernel {
   static constexpr int kPer = (kRows + 3) / 4;  // rows a wave stages per step: wave + 4 i
   static constexpr int kAcc = MODE == MODE_RX ? WC : 1;
   static constexpr int kGroups = CG * WG;
-  static constexpr int kSmem = kGroups * 2 * kBufBytes;
+  // dimension both: the sums are closed every 32 steps (and at the end of a
+  // round), so that their rounding grows with 32 + steps / 32 additions, not
+  // with the channels (1024 of the volume: 4.7e-7 by the gathering kernel's
+  // splits, 6.2e-7 in one running sum). One frame keeps its closed sum in
+  // registers; several keep one per pixel in LDS, which the groups add to in
+  // turn: two more register pairs leave a block less per CU (cine 0.56 -> 0.72
+  // ms).
+  static constexpr bool kClose = MODE == MODE_BOTH;
+  static constexpr bool kCloseLds = kClose && FT > 1;
+  static constexpr int kTot = kCloseLds ? FT * 256 * 8 : 0;
+  static constexpr int kSmem = kGroups * 2 * kBufBytes + kTot;
 
   // One staged term: its fraction, the LDS address of its samples and whether it counts.
   struct Term1 {
@@ -227,12 +237,34 @@ struct WinKernel {
     constexpr bool kT = !(MODE == MODE_RX && kSep);  // the transmit weight is held per wave
     float2 acc[kAF][kAcc];
     static_for<kAF>([&](auto f) { static_for<kAcc>([&](auto j) { acc[f][j] = make_float2(0.0f, 0.0f); }); });
-    // dimension both, one frame: the sum is closed every 32 steps, so that its
-    // rounding grows with 32 + steps / 32 additions, not with the channels
-    // (1024 of the volume: 4.7e-7 by the gathering kernel's splits, 6.2e-7 in
-    // one running sum)
-    constexpr bool kClose = MODE == MODE_BOTH && FT == 1;
     float2 tot = make_float2(0.0f, 0.0f);
+    // this lane's closed sum of frame f, its address formed where it is used (a
+    // register held through the loop would cost a block per CU)
+    auto closed = [&](int f) {
+      unsigned t = threadIdx.x;
+      asm volatile("" : "+v"(t));
+      return reinterpret_cast<lds_f2*>((size_t)((unsigned)(size_t)(__attribute__((address_space(3))) char*)smem +
+                                                (unsigned)(kSmem - kTot + f * 2048) + (t & 255u) * 8u));
+    };
+    auto close = [&]() {
+      if constexpr (kCloseLds) {
+        static_for<kGroups>([&](auto turn) {
+          if (g == turn)
+            static_for<FT>([&](auto f) {
+              lds_f2* t = closed(f);
+              const f2v v = *t;
+              *t = f2v{v.x + acc[f][0].x, v.y + acc[f][0].y};
+            });
+          __syncthreads();
+        });
+      } else {
+        cadd(tot, acc[0][0]);
+      }
+      static_for<kAF>([&](auto f) { acc[f][0] = make_float2(0.0f, 0.0f); });
+    };
+    if constexpr (kCloseLds) {
+      if (g == 0) static_for<FT>([&](auto f) { *closed(f) = f2v{0.0f, 0.0f}; });
+    }
 
     for (int kr = 0; kr < nw; kr += WG * WC) {
       const int k0 = __builtin_amdgcn_readfirstlane(kr + wgi * WC);
@@ -410,51 +442,49 @@ struct WinKernel {
         rx_load(q);
       }
       __syncthreads();
-      for (int it = 0; it < nit; ++it) {
-        const int s = q + it * Q;
-        const bool more = s + Q < steps;           // wave-uniform
-        if (more) stage_load(s + Q);
-        if (s < steps && nj > 0) {
-          static_for<NCH>([&](auto c) {
-            const int ci = s * NCH + c;
-            if (ci < nc) {
-              const int4 ce = scalar_int4(cl + ci);
-              const bool ron = rv[c].y != 0.0f;
-              const float2 R = ron ? make_float2(rv[c].z, rv[c].w) : make_float2(0.0f, 0.0f);
-              float2 part[FT];
-              static_for<FT>([&](auto f) { part[f] = make_float2(0.0f, 0.0f); });
-              // every term of the channel in the sample window, every weight
-              // nonzero (dimension both drops the sums of the lanes with no
-              // receive weight below)
-              const bool dense = (all_t & 1) && (MODE == MODE_BOTH || (ce.w & 1)) && amin + ce.y - 1 >= 1 &&
-                                 amax + ce.z + 2 < ilim;
-              if (dense)
-                compute(std::false_type(), c, ce.x, ce.y, buf, rv[c].x, R, rv[c].y, part);
-              else
-                compute(std::true_type(), c, ce.x, ce.y, buf, ron ? rv[c].x : kFar, R, rv[c].y, part);
-              if constexpr (MODE == MODE_BOTH)
-                static_for<FT>([&](auto f) {
-                  float2 v = acc[f][0];
-                  cfma(v, make_float2(rv[c].z, rv[c].w), part[f]);
-                  acc[f][0] = ron ? v : acc[f][0];
-                });
-            }
-          });
-        }
-        // the next entries into the same registers: a second set, in flight
-        // during the terms, costs a block per CU and time (cine 0.60 -> 0.77 ms)
-        if (more) {
-          rx_load(s + Q);
-          stage_store(buf ^ 1);
-        }
-        if constexpr (kClose) {
-          if ((it & 31) == 31) {
-            cadd(tot, acc[0][0]);
-            acc[0][0] = make_float2(0.0f, 0.0f);
+      for (int i0 = 0, i1; i0 < nit; i0 = i1) {
+        i1 = kClose ? min(i0 + 32, nit) : nit;
+        for (int it = i0; it < i1; ++it) {
+          const int s = q + it * Q;
+          const bool more = s + Q < steps;           // wave-uniform
+          if (more) stage_load(s + Q);
+          if (s < steps && nj > 0) {
+            static_for<NCH>([&](auto c) {
+              const int ci = s * NCH + c;
+              if (ci < nc) {
+                const int4 ce = scalar_int4(cl + ci);
+                const bool ron = rv[c].y != 0.0f;
+                const float2 R = ron ? make_float2(rv[c].z, rv[c].w) : make_float2(0.0f, 0.0f);
+                float2 part[FT];
+                static_for<FT>([&](auto f) { part[f] = make_float2(0.0f, 0.0f); });
+                // every term of the channel in the sample window, every weight
+                // nonzero (dimension both drops the sums of the lanes with no
+                // receive weight below)
+                const bool dense = (all_t & 1) && (MODE == MODE_BOTH || (ce.w & 1)) && amin + ce.y - 1 >= 1 &&
+                                   amax + ce.z + 2 < ilim;
+                if (dense)
+                  compute(std::false_type(), c, ce.x, ce.y, buf, rv[c].x, R, rv[c].y, part);
+                else
+                  compute(std::true_type(), c, ce.x, ce.y, buf, ron ? rv[c].x : kFar, R, rv[c].y, part);
+                if constexpr (MODE == MODE_BOTH)
+                  static_for<FT>([&](auto f) {
+                    float2 v = acc[f][0];
+                    cfma(v, make_float2(rv[c].z, rv[c].w), part[f]);
+                    acc[f][0] = ron ? v : acc[f][0];
+                  });
+              }
+            });
           }
+          // the next entries into the same registers: a second set, in flight
+          // during the terms, costs a block per CU and time (cine 0.60 -> 0.77 ms)
+          if (more) {
+            rx_load(s + Q);
+            stage_store(buf ^ 1);
+          }
+          __syncthreads();
+          buf ^= 1;
         }
-        __syncthreads();
-        buf ^= 1;
+        if constexpr (kClose) close();
       }
 
       if constexpr (MODE == MODE_RX) {
@@ -483,9 +513,13 @@ struct WinKernel {
     if constexpr (MODE == MODE_BOTH)
       static_for<FT>([&](auto f) {
         if (f < nfr) {
-          float2 v = acc[f][0];
-          if constexpr (kClose) cadd(v, tot);
-          v = group_sum(v, smem, g, lid);
+          float2 v;
+          if constexpr (kCloseLds) {
+            const f2v t = *closed(f);
+            v = make_float2(t.x, t.y);
+          } else {
+            v = group_sum(tot, smem, g, lid);
+          }
           if (A.ref) v = cmul(v, refp);
           if (act && g == 0) (A.out + (size_t)(f0 + f) * PS)[p] = v;
         }
