@@ -185,3 +185,25 @@ def test_both_sums_are_closed_over_many_channels(cuda):
                                                  device=cuda))).double()
     plan.close()
     assert (got / (prb.N_elements * W * c) - 1.0).abs().max().item() <= 58 * 2.0 ** -24
+
+
+def test_more_frames_than_one_grid(cuda):
+    """A grid holds fewer than 2^32 threads: 8200 frames of 528 x 1040 pixels, 36
+    GB of image, against plans of the first and last frames."""
+    print("case window both 8200 frames", flush=True)
+    W, F, L, Q = 9, 8200, 64, 3
+    prb = LinearArray(4, 0.3e-3)
+    seq = [Wave.plane(a, sound_speed=C) for a in np.deg2rad(np.linspace(-8, 8, W))]
+    scan = LinearScan(np.linspace(-2e-3, 2e-3, 528), np.linspace(1e-3, 4e-3, 1040))
+    kw = dict(n_samples=L, sampling_frequency=10.4e6, initial_time=0.0, modulation_frequency=5.2e6, sound_speed=C,
+              receive_apodization=Apodization(), transmit_apodization=Apodization(), dimension=3, interpolation=0)
+    g = torch.Generator(cuda).manual_seed(8)
+    ch = torch.randn((F, W, prb.N_elements, L), dtype=torch.complex64, device=cuda, generator=g)
+    plan = make_plan(prb, scan, seq, n_frames=F, **kw)
+    few = make_plan(prb, scan, seq, n_frames=Q, **kw)
+    assert plan.variant == few.variant == (2, 0, 0)
+    got = plan.run(ch)
+    for f in (0, 4000, F - Q):
+        assert torch.equal(got[f:f + Q], few.run(ch[f:f + Q].contiguous())), f
+    plan.close()
+    few.close()

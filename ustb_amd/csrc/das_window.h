@@ -30,6 +30,7 @@
 // separable phase keeps {x, x[+1] - x} per sample in rows of 64, so a term
 // costs two FMAs and no subtraction; the other forms keep the samples.
 #pragma once
+#include <algorithm>
 #include <type_traits>
 #include <utility>
 
@@ -567,10 +568,22 @@ static hipError_t launch_window_t(const GeomLaunch& G, int zsplit, hipStream_t s
   A.fs = G.fs;
   A.wd = G.wd;
   A.frame_bytes = G.L * G.N * G.W * 8;
-  hipLaunchKernelGGL((das_window_kernel<SM, MODE, PH, ROW, WC, FT, NCH, CG, WG>),
-                     dim3((unsigned)G.win.tiles * (unsigned)((G.F + FT - 1) / FT), 1u, (unsigned)zsplit), dim3(256 * CG * WG), 0,
-                     stream, A);
-  return hipGetLastError();
+  // a grid holds fewer than 2^32 threads: as many frames per launch as fit
+  constexpr int kThreads = 256 * CG * WG;
+  const size_t chunks = (size_t)(0xFFFFFFFFu / kThreads) / (size_t)G.win.tiles;
+  const int most = (int)std::min<size_t>((size_t)G.F, std::max<size_t>(chunks, 1) * FT);
+  const size_t frame_out = (size_t)G.P * (size_t)(MODE == MODE_BOTH ? 1 : G.W) * (size_t)(MODE == MODE_NONE ? G.N : 1);
+  hipError_t e = hipSuccess;
+  for (int64_t f = 0; e == hipSuccess && f < G.F; f += most) {
+    A.F = (int)std::min<int64_t>(most, G.F - f);
+    A.ch = (const char*)G.ch + (size_t)f * (size_t)A.frame_bytes;
+    A.out = reinterpret_cast<float2*>(G.out) + (size_t)f * frame_out;
+    hipLaunchKernelGGL((das_window_kernel<SM, MODE, PH, ROW, WC, FT, NCH, CG, WG>),
+                       dim3((unsigned)G.win.tiles * (unsigned)((A.F + FT - 1) / FT), 1u, (unsigned)zsplit),
+                       dim3(kThreads), 0, stream, A);
+    e = hipGetLastError();
+  }
+  return e;
 }
 
 hipError_t launch_window_rx(const GeomLaunch& G, int ph, hipStream_t stream);
