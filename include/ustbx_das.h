@@ -279,7 +279,10 @@ int ustbx_plan_run(const ustbx_plan* plan, const void* ch, void* out,
  * 16) and channel groups per pixel tile (1 or 4; dimension both/transmit).
  * Variants 1-3: waves per wave-split (variant 1: 8, 10, 12, 16; variants 2
  * and 3: 4, 5, 6, 8, 10, 12, 16) and wave-splits per 64-pixel tile (variant
- * 1: 4 or 8; variants 2 and 3: 4, 5 or 8). */
+ * 1: 4 or 8; variants 2 and 3: 4, 5 or 8).
+ * A tile shape selects the kernel of that shape; both 0 select the staged
+ * windows again where the library chose them (ustbx_plan_variant), so a shape
+ * that ustbx_plan_variant reported restores the plan. */
 int ustbx_plan_set_tiles(ustbx_plan* plan, int32_t wave_chunk, int32_t split,
                          ustbx_status* st);
 /* Kernel variant (results agree to FP32 rounding; no reference counterpart):
@@ -331,11 +334,10 @@ int ustbx_plan_set_staging(ustbx_plan* plan, int32_t on, ustbx_status* st);
  * channel lists (0, 0 otherwise). */
 int ustbx_plan_stage_stats(const ustbx_plan* plan, int64_t* staged, int64_t* listed, ustbx_status* st);
 /* Current variant (or -1 for NULL) and its tile shape: 0 and 0 where the
- * library runs the plan on patch tiles with LDS-staged sample windows
- * (dimension both on variant 2 while no tile shape was set; 9 or more waves
- * and the work of a few hundred full tiles of 256 pixels). Setting a tile shape selects the gathering kernel
- * of that shape. Dimension receive and none use patch tiles wherever the scan
- * and the weights allow, under variant 0. */
+ * library runs the plan on patch tiles with LDS-staged sample windows while no
+ * tile shape is set (dimension both on variant 2: 9 or more waves and the work
+ * of a few hundred full tiles of 256 pixels; dimension receive and none on
+ * variant 0: wherever the scan and the weights allow). */
 int32_t ustbx_plan_variant(const ustbx_plan* plan, int32_t* wave_chunk, int32_t* split);
 
 /* ---------------------------------------------------------------------------

@@ -207,3 +207,36 @@ def test_more_frames_than_one_grid(cuda):
         assert torch.equal(got[f:f + Q], few.run(ch[f:f + Q].contiguous())), f
     plan.close()
     few.close()
+
+
+@pytest.mark.parametrize("kind,W,nx,nz,F,dim,phase,shape", [
+    ("linear", 9, 540, 900, 1, 3, "separable", (2, 8, 4)), ("volume", 26, 110, 170, 3, 3, "separable", (2, 16, 4)),
+    ("sector", 6, 31, 70, 2, 1, "separable", (0, 16, 1)), ("linear", 5, 33, 65, 1, 0, "separable", (0, 8, 1)),
+    ("linear", 5, 33, 65, 1, 1, "dasc", (0, 8, 1))])
+def test_tile_shapes_select_and_restore(cuda, kind, W, nx, nz, F, dim, phase, shape):
+    """A set tile shape runs and is reported; the reported one restores the staged windows."""
+    print(f"case window shapes {kind} W={W} dim={dim} {phase}", flush=True)
+    prb, scan, seq = _setup(kind, W, nx, nz, 25e-3 if kind != "volume" else 14e-3)
+    plan = make_plan(prb, scan, seq, n_samples=512, n_frames=F, sampling_frequency=10.4e6, initial_time=0.0,
+                     modulation_frequency=5.2e6, sound_speed=C, receive_apodization=TUKEY,
+                     transmit_apodization=Apodization(), dimension=dim, interpolation=0,
+                     separable_phase=phase == "separable")
+    g = torch.Generator(cuda).manual_seed(W)
+    ch = torch.randn((F, W, prb.N_elements, 512), dtype=torch.complex64, device=cuda, generator=g)
+    v = plan.variant
+    assert v == (shape[0], 0, 0)
+    staged = plan.run(ch)
+    plan.set_tiles(*shape[1:])
+    assert plan.variant == shape and plan.has_variant(0) and plan.variant == shape
+    own = plan.run(ch)
+    # the same FP32 terms in another order (das_c's phase: the same order)
+    assert (own - staged).abs().max().item() <= (0.0 if phase == "dasc" else 5e-6) * staged.abs().max().item()
+    plan.set_tiles(0, shape[2])
+    assert plan.variant == shape
+    plan.set_tiles(*v[1:])
+    assert plan.variant == v and torch.equal(plan.run(ch), staged)
+    if dim == 3:
+        plan.set_variant(0)
+        plan.set_variant(2)
+        assert plan.variant == v and torch.equal(plan.run(ch), staged)
+    plan.close()

@@ -24,7 +24,7 @@ VARIANT1 = [(1, wc, ws) for ws in (4, 8) for wc in (8, 10, 12, 16)]
 VARIANT2 = [(2, wc, ws) for ws in (4, 5, 8) for wc in (4, 5, 6, 8, 10, 12, 16)]
 VARIANT3 = [(3, wc, ws) for ws in (4, 8) for wc in (6, 10, 16)]
 VARIANT2_TX = [(2, fc, cs) for fc in (4, 8) for cs in (4, 8)]   # frames per block, channels per block
-DEFAULT_SHAPE = (2, 0, 0)  # no tile shape set: staged windows on patch tiles, where the plan takes them
+STAGED = ((0, 0, 0), (2, 0, 0))  # no tile shape set: staged windows on patch tiles, where the plan takes them
 
 _cache: dict = {}
 _lock = threading.Lock()
@@ -46,17 +46,28 @@ def candidates(plan):
         c += VARIANT2_TX
     if plan.dim == L.DIM_BOTH and plan.has_variant(2):
         c += VARIANT2
-        if plan.variant == DEFAULT_SHAPE:
-            c.append(DEFAULT_SHAPE)
         if plan.interp == L.INTERP_CUBIC and plan.has_variant(3):
             c += VARIANT3
+    staged = _staged(plan)
+    if staged:
+        c.append(staged)
     return c
+
+
+def _staged(plan):
+    """The member of STAGED that the plan runs while no tile shape is set, or
+    None; the current selection is kept."""
+    v = plan.variant
+    if plan.dim == L.DIM_BOTH and v[0] != 2 and plan.has_variant(2):
+        plan.set_variant(2)
+    plan.set_tiles(0, 0)
+    d = plan.variant
+    apply(plan, v)
+    return d if d in STAGED else None
 
 
 def apply(plan, cand):
     variant, wc, sp = cand
-    if cand == DEFAULT_SHAPE and plan.variant != DEFAULT_SHAPE:
-        plan.set_variant(0)  # and back: drops the tile shape
     plan.set_variant(variant)
     plan.set_tiles(wc, sp)
 

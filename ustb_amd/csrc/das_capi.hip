@@ -1535,6 +1535,12 @@ int ustbx_plan_set_variant(ustbx_plan* plan, int32_t variant, ustbx_status* st) 
 
 int ustbx_plan_set_tiles(ustbx_plan* plan, int32_t wave_chunk, int32_t split, ustbx_status* st) {
   if (!plan) return set_status(st, USTBX_E_ARG, "NULL plan");
+  if (!wave_chunk && !split) {  // keep; the library's choice again where that has no tile shape
+    GeomLaunch G = plan->G;
+    G.auto_tiles = 1;
+    if (window_active(G)) plan->G.auto_tiles = 1;
+    return ok(st);
+  }
   if (plan->G.variant >= 2 && plan->G.dim == 2) {
     if (wave_chunk && wave_chunk != 4 && wave_chunk != 8)
       return set_status(st, USTBX_E_ARG, "frames per block must be 4 or 8");
@@ -1548,7 +1554,7 @@ int ustbx_plan_set_tiles(ustbx_plan* plan, int32_t wave_chunk, int32_t split, us
       return set_status(st, USTBX_E_ARG, "waves per split must be 4, 5, 6, 8, 10, 12 or 16");
     if (split && split != 4 && split != 5 && split != 8)
       return set_status(st, USTBX_E_ARG, "wave-splits per block must be 4, 5 or 8");
-    if (wave_chunk || split) plan->G.auto_tiles = 0;
+    plan->G.auto_tiles = 0;
     if (wave_chunk) plan->G.wave_chunk = wave_chunk;
     if (split) plan->G.split = split;
     return ok(st);
@@ -1570,12 +1576,14 @@ int ustbx_plan_set_tiles(ustbx_plan* plan, int32_t wave_chunk, int32_t split, us
     if (wave_chunk == 1 && plan->G.separable)
       return set_status(st, USTBX_E_ARG, "wave_chunk 1 needs the das_c phase");
     plan->G.wave_chunk = wave_chunk;
+    plan->G.auto_tiles = 0;
   }
   if (split) {
     if (split != 1 && split != 4) return set_status(st, USTBX_E_ARG, "split must be 1 or 4");
     if (split != 1 && !(plan->G.dim == 3 || plan->G.dim == 2))
       return set_status(st, USTBX_E_ARG, "split applies to dimension both/transmit only");
     plan->G.split = split;
+    plan->G.auto_tiles = 0;
   }
   if (plan->G.wave_chunk == 1) plan->G.split = 1;
   return ok(st);
@@ -1768,7 +1776,7 @@ int ustbx_plan_stage_stats(const ustbx_plan* plan, int64_t* staged, int64_t* lis
 
 int32_t ustbx_plan_variant(const ustbx_plan* plan, int32_t* wave_chunk, int32_t* split) {
   if (!plan) return -1;
-  const bool window = window_both_active(plan->G);  // the library's choice, no tile shape
+  const bool window = window_active(plan->G);  // the library's choice, no tile shape
   if (wave_chunk) *wave_chunk = window ? 0 : plan->G.wave_chunk;
   if (split) *split = window ? 0 : plan->G.split;
   return (plan->G.variant == 2 && plan->G.rx_otf) ? 4 : plan->G.variant;

@@ -8,13 +8,14 @@ namespace ustbx {
 
 hipError_t launch_das_geom(const GeomLaunch& G, hipStream_t stream) {
   const int ph = (G.wd == 0.0f) ? PH_RF : (G.separable ? PH_SEP : PH_DASC);
-  if (window_both_active(G)) return launch_window_both(G, stream);
+  if (window_active(G)) {
+    if (G.dim == MODE_BOTH) return launch_window_both(G, stream);
+    return G.dim == MODE_RX ? launch_window_rx(G, ph, stream) : launch_window_none(G, ph, stream);
+  }
   if (G.variant >= 2 && G.dim == MODE_BOTH) return launch_both_rxtab(G, stream);
   if (G.variant == 2 && G.dim == MODE_TX) return launch_tx_rxtab(G, stream);
   if (G.variant == 1 && G.dim == MODE_BOTH && ph == PH_SEP && G.F == 1)
     return launch_both_shared(G, stream);
-  if (G.win.on && G.dim == MODE_RX) return launch_window_rx(G, ph, stream);
-  if (G.win.on && G.dim == MODE_NONE) return launch_window_none(G, ph, stream);
   switch (G.dim) {
     case MODE_BOTH: return launch_geom_both(G, ph, G.wave_chunk, G.split, stream);
     case MODE_TX: return launch_geom_tx(G, ph, G.wave_chunk, G.split, stream);

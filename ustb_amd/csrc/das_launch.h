@@ -122,9 +122,9 @@ struct GeomLaunch {
   // 4 = patches of 16 depths x 4 scan lines (dimension transmit on a linear
   // or sector scan whose axes divide evenly). Fixed when the plan is made.
   int tile_ps;
-  // Window-staged kernels (das_window.h), where win.on; dimension both reads
-  // rx_table and ref_table and takes them while no tile shape is set
-  // (auto_tiles), the other modes win_rx and win_ref.
+  // Window-staged kernels (das_window.h), where win.on and while no tile shape
+  // is set (auto_tiles); dimension both reads rx_table and ref_table, the other
+  // modes win_rx and win_ref.
   WinTiles win;
   int win_max_nw;        // largest wave count of a patch tile
   int win_even;          // the plan's terms over those of its largest patch tile
@@ -160,6 +160,12 @@ inline bool window_both_active(const GeomLaunch& G) {
   const int nw = G.win_max_nw;
   const int need = nw <= 10 || (nw > 16 && nw <= 24) ? 640 : nw <= 16 ? 512 : 400;
   return (int64_t)G.win_even * ((G.F + 1) / 2) >= (G.win.row == 64 ? need : 2 * need);
+}
+
+// Whether a plan of any dimension runs window-staged.
+inline bool window_active(const GeomLaunch& G) {
+  if (G.dim == 0 || G.dim == 1) return G.win.on && G.variant == 0 && G.auto_tiles;
+  return window_both_active(G);
 }
 
 // Builds the transmit table of a plan (one lane per (wave, pixel)).

@@ -261,8 +261,8 @@ class GeometryPlan:
     @property
     def variant(self) -> tuple[int, int, int]:
         """(variant, waves per chunk or split, split) currently selected;
-        (2, 0, 0) where the library runs the plan on patch tiles with staged
-        sample windows (no tile shape set)."""
+        shape (0, 0) where the library runs the plan on patch tiles with
+        staged sample windows (no tile shape set)."""
         wc, sp = ctypes.c_int32(0), ctypes.c_int32(0)
         v = L.lib().ustbx_plan_variant(self.handle, ctypes.byref(wc), ctypes.byref(sp))
         return int(v), int(wc.value), int(sp.value)
@@ -291,6 +291,9 @@ class GeometryPlan:
         return a.value, b.value
 
     def set_tiles(self, wave_chunk: int = 0, split: int = 0):
+        """Select the kernel of a tile shape (0: keep); (0, 0) goes back to
+        staged sample windows where the library chose them, so
+        set_tiles(*variant[1:]) restores a shape that variant reported."""
         st = L.Status()
         L.check(L.lib().ustbx_plan_set_tiles(self.handle, wave_chunk, split, ctypes.byref(st)), st)
 
