@@ -12,6 +12,7 @@ from tests.cases import channel_noise, geom_cases
 from ustb_amd import autotune
 from ustb_amd.enums import Interpolation
 from ustb_amd.geometry import make_plan
+from ustb_amd.uff import LinearArray, LinearScan, Wave, XYZScan
 
 pytestmark = pytest.mark.gpu
 CASES = geom_cases()
@@ -55,3 +56,32 @@ def test_autotune_picks_applies_and_caches(cuda, tmp_path, name, dim, interp):
     assert again == best and t2 == {} and other.variant == best
     other.close()
     plan.close()
+
+
+def test_choices_stay_with_scans_of_their_kind(cuda, tmp_path):
+    """A shape tuned on a pixel list, or kept in a file of an older version,
+    is not given to a scan that can run staged windows."""
+    print("case autotune keys", flush=True)
+    prb = LinearArray(21, 0.3e-3)
+    seq = [Wave.plane(a, sound_speed=1540.0) for a in np.deg2rad(np.linspace(-16, 16, 9))]
+    lin = LinearScan(np.linspace(-8e-3, 8e-3, 540), np.linspace(4e-3, 25e-3, 600))
+    kw = dict(n_samples=512, n_frames=1, sampling_frequency=10.4e6, initial_time=0.0, modulation_frequency=5.2e6,
+              sound_speed=1540.0, dimension=3)
+    plan, pixels = make_plan(prb, lin, seq, **kw), make_plan(prb, XYZScan(lin.x, lin.y, lin.z), seq, **kw)
+    assert plan.variant == (2, 0, 0) and pixels.variant[1:] != (0, 0)
+    key, other = autotune.shape_class(plan), autotune.shape_class(pixels)
+    assert key != other and plan.variant == (2, 0, 0)
+    plan.set_tiles(8, 4)
+    assert autotune.shape_class(plan) == key and plan.variant == (2, 8, 4)
+    old = str(tmp_path / "old.json")
+    json.dump({key[key.index("dim"):]: [2, 4, 4], other: [2, 4, 4]}, open(old, "w"))
+    autotune._cache.clear()
+    ch = torch.randn((1, 9, 21, 512), dtype=torch.complex64, device=cuda)
+    best, times = autotune.tune(plan, ch, reps=1, cache_file=old)
+    assert (2, 0, 0) in times and best == plan.variant
+    autotune._cache[other] = (2, 0, 0)  # cannot run there: what runs is returned
+    best, times = autotune.tune(pixels, ch)
+    assert times == {} and best == pixels.variant and best[1:] != (0, 0)
+    autotune._cache.clear()
+    plan.close()
+    pixels.close()

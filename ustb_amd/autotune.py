@@ -5,7 +5,8 @@ plan on its own channel data with HIP events, checks that each candidate's
 image agrees with the first one (the candidates only regroup the same sums),
 and keeps the fastest. Results are cached per shape class -- (dimension,
 interpolation, phase, waves, channels, frames, pixels rounded to a power of
-two) -- in memory and, optionally, in a JSON file.
+two, scan kind, whether the plan can run staged windows) -- in memory and,
+optionally, in a JSON file.
 """
 from __future__ import annotations
 
@@ -32,7 +33,9 @@ _lock = threading.Lock()
 
 def shape_class(plan) -> str:
     P2 = 1 << max(0, int(math.ceil(math.log2(max(plan.P, 1)))))
-    return f"dim{plan.dim}-W{plan.W}-N{plan.N}-F{plan.F}-P{P2}-interp{plan.interp}-sep{int(plan.separable)}"
+    # the leading number changes with the candidates: choices of older files are not read
+    return (f"2-scan{plan.scan_kind}-staged{int(_staged(plan) is not None)}-"
+            f"dim{plan.dim}-W{plan.W}-N{plan.N}-F{plan.F}-P{P2}-interp{plan.interp}-sep{int(plan.separable)}")
 
 
 def candidates(plan):
@@ -83,7 +86,7 @@ def tune(plan, ch: torch.Tensor, reps: int = 3, cache_file: str | None = None, v
                 pass
         if key in _cache:
             apply(plan, _cache[key])
-            return _cache[key], {}
+            return plan.variant, {}
     out = torch.empty(plan.out_shape, dtype=torch.complex64, device=ch.device)
     ref = None
     times = {}

@@ -217,6 +217,7 @@ class GeometryPlan:
         self.N, self.W, self.L, self.F = geometry.N, geometry.W, geometry.L, geometry.F
         self.dim = geometry.dim
         self.interp = geometry.interp
+        self.scan_kind = int(geometry.scan.kind)
         self.separable = bool(geometry.flags & L.FLAG_SEPARABLE_PHASE) and not (geometry.flags & L.FLAG_DASC_ORDER)
         self.fd = geometry.fd
         self.P = int(L.lib().ustbx_plan_pixels(self.handle))
