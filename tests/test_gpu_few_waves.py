@@ -77,3 +77,20 @@ def test_against_one_channel_at_a_time(cuda, case):
     assert peak > 0
     assert float((got - ref)[fin].abs().max()) <= 2.0 * W * N * 2.0 ** -24 * peak * 4
     plan.close()
+
+
+def test_default_shape_follows_the_receive_state(cuda):
+    """The kernel that computes the receive state keeps the shapes it was
+    measured with, a shape that was set stays."""
+    plan = _plan(6, 33, False, False, 1, 500, TUKEY)
+    assert plan.variant == (2, 6, 8)
+    plan.set_variant(4)
+    assert plan.variant == (4, 4, 8)
+    assert plan.has_variant(2) and plan.variant == (4, 4, 8)
+    plan.set_variant(2)
+    assert plan.variant == (2, 6, 8)
+    assert plan.has_variant(4) and plan.variant == (2, 6, 8)
+    plan.set_tiles(12, 8)
+    plan.set_variant(4)
+    assert plan.variant == (4, 12, 8)
+    plan.close()

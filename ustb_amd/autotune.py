@@ -72,7 +72,8 @@ def _staged(plan):
 def apply(plan, cand):
     variant, wc, sp = cand
     plan.set_variant(variant)
-    plan.set_tiles(wc, sp)
+    if plan.variant != (variant, wc, sp):
+        plan.set_tiles(wc, sp)
 
 
 def tune(plan, ch: torch.Tensor, reps: int = 3, cache_file: str | None = None, verbose: bool = False):

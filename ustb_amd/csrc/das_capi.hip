@@ -1483,6 +1483,12 @@ int ustbx_plan_create(const ustbx_geometry* g, ustbx_plan** plan, ustbx_status* 
 int ustbx_plan_set_variant(ustbx_plan* plan, int32_t variant, ustbx_status* st) {
   if (!plan) return set_status(st, USTBX_E_ARG, "NULL plan");
   if (variant < 0 || variant > 4) return set_status(st, USTBX_E_ARG, "variant must be 0, 1, 2, 3 or 4");
+  const int otf = plan->G.rx_otf;
+  // a shape chosen by the library follows the kernel that forms the receive state
+  auto follow = [&]() {
+    if (plan->G.rx_otf != otf && plan->G.auto_tiles)
+      rxtab_defaults(plan->G, plan->max_nw, plan->G.wave_chunk, plan->G.split);
+  };
   if (variant == 4) {
     // variant 2 with the receive state on the fly
     hipError_t e;
@@ -1496,6 +1502,8 @@ int ustbx_plan_set_variant(ustbx_plan* plan, int32_t variant, ustbx_status* st) 
       plan->G.variant = 2;
       plan->G.auto_tiles = 1;
       rxtab_defaults(plan->G, plan->max_nw, plan->G.wave_chunk, plan->G.split);
+    } else {
+      follow();
     }
     return ok(st);
   }
@@ -1517,8 +1525,9 @@ int ustbx_plan_set_variant(ustbx_plan* plan, int32_t variant, ustbx_status* st) 
                         "per frame");
     }
   }
-  if (variant == plan->G.variant) return ok(st);
   const bool same_family = variant >= 2 && plan->G.variant >= 2;
+  if (same_family) follow();
+  if (variant == plan->G.variant) return ok(st);
   plan->G.variant = variant;
   if (same_family) return ok(st);
   plan->G.auto_tiles = 1;

@@ -247,7 +247,8 @@ class GeometryPlan:
         rc = L.lib().ustbx_plan_set_variant(self.handle, int(variant), ctypes.byref(st))
         if rc == 0:
             self.set_variant(cur[0])
-            self.set_tiles(cur[1], cur[2])
+            if self.variant != cur:
+                self.set_tiles(cur[1], cur[2])
             return True
         if rc != L.E_UNSUPPORTED:
             L.check(rc, st)
