@@ -94,3 +94,15 @@ def test_default_shape_follows_the_receive_state(cuda):
     plan.set_variant(4)
     assert plan.variant == (4, 12, 8)
     plan.close()
+
+
+def test_a_refused_variant_leaves_the_plan_as_it_was(cuda):
+    """The on-the-fly receive state does not take a tilted aperture; asking for it keeps the receive table."""
+    plan = _plan(5, 33, False, False, 1, 500, Apodization(Window.tukey25, f_number=1.7, tilt=(0.1, 0.0)))
+    ch = torch.randn((1, 5, 33, 500), dtype=torch.complex64, device=cuda)
+    v, ref = plan.variant, plan.run(ch)
+    assert v[0] == 2 and not plan.has_variant(4)
+    assert plan.variant == v
+    print("case refused variant", flush=True)
+    assert torch.equal(plan.run(ch), ref)
+    plan.close()

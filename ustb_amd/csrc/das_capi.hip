@@ -661,6 +661,7 @@ void rxtab_free(ustbx_plan* pl) {
 bool rxtab_build(ustbx_plan* pl, hipError_t& err, bool otf) {
   err = hipSuccess;
   if (pl->rxtab_state > 0 && (pl->G.rx_otf != 0) == otf) return true;
+  if (pl->rxtab_state > 0 && !rxtab_applies(pl, otf)) return false;  // the form that is there stays
   if (pl->rxtab_state > 0 || (pl->rxtab_state < 0 && (pl->G.rx_otf != 0) != otf)) rxtab_free(pl);
   if (pl->rxtab_state != 0) return false;
   pl->rxtab_state = -1;
@@ -1484,6 +1485,14 @@ int ustbx_plan_set_variant(ustbx_plan* plan, int32_t variant, ustbx_status* st) 
   if (!plan) return set_status(st, USTBX_E_ARG, "NULL plan");
   if (variant < 0 || variant > 4) return set_status(st, USTBX_E_ARG, "variant must be 0, 1, 2, 3 or 4");
   const int otf = plan->G.rx_otf;
+  // where the other form's tables could not be had, the kernel without tables runs
+  auto without_tables = [&]() {
+    if (plan->rxtab_state > 0 || plan->G.variant < 2) return;
+    plan->G.variant = 0;
+    plan->G.auto_tiles = 1;
+    plan->G.wave_chunk = plan->G.separable ? 16 : 8;
+    plan->G.split = auto_split(plan->G.P);
+  };
   // a shape chosen by the library follows the kernel that forms the receive state
   auto follow = [&]() {
     if (plan->G.rx_otf != otf && plan->G.auto_tiles)
@@ -1493,6 +1502,7 @@ int ustbx_plan_set_variant(ustbx_plan* plan, int32_t variant, ustbx_status* st) 
     // variant 2 with the receive state on the fly
     hipError_t e;
     if (!rxtab_build(plan, e, true)) {
+      without_tables();
       if (e != hipSuccess) return hip_fail(st, e, "receive-state tables");
       return set_status(st, USTBX_E_UNSUPPORTED,
                         "the on-the-fly receive state needs dimension both with the separable (or RF) phase, and a "
@@ -1513,6 +1523,7 @@ int ustbx_plan_set_variant(ustbx_plan* plan, int32_t variant, ustbx_status* st) 
   if (variant >= 2) {
     hipError_t e;
     if (!rxtab_build(plan, e, false)) {
+      without_tables();
       if (e != hipSuccess) return hip_fail(st, e, "receive table");
       return set_status(st, USTBX_E_UNSUPPORTED,
                         "the receive-table kernels need dimension both with the separable (or RF) phase outside das_c's "
