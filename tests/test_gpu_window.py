@@ -240,3 +240,21 @@ def test_tile_shapes_select_and_restore(cuda, kind, W, nx, nz, F, dim, phase, sh
         plan.set_variant(2)
         assert plan.variant == v and torch.equal(plan.run(ch), staged)
     plan.close()
+
+
+def test_receive_table_is_bounded(cuda):
+    """A receive plan whose table would take more than a 32nd of the device memory keeps none."""
+    total = torch.cuda.get_device_properties(cuda).total_memory
+    N = 128
+    nx = int(math.sqrt(total / 32 / 16 / N) * 1.02)
+    print(f"case window table bound {nx} x {nx}", flush=True)
+    seq = [Wave.plane(0.0, sound_speed=C)]
+    kw = dict(n_samples=256, n_frames=1, sampling_frequency=10.4e6, initial_time=0.0, modulation_frequency=5.2e6,
+              sound_speed=C, receive_apodization=TUKEY, dimension=1, interpolation=0)
+    scans = [LinearScan(np.linspace(-8e-3, 8e-3, n), np.linspace(4e-3, 15e-3, nx)) for n in (nx, 64)]
+    large, small = (make_plan(LinearArray(N, 0.3e-3), s, seq, **kw) for s in scans)
+    assert small.variant == (0, 0, 0) and large.variant[1:] != (0, 0) and large.device_bytes < total // 64
+    ch = torch.randn((1, 1, N, 256), dtype=torch.complex64, device=cuda)
+    assert torch.isfinite(torch.view_as_real(large.run(ch))).all()
+    large.close()
+    small.close()

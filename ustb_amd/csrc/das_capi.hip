@@ -799,10 +799,11 @@ bool coef_build(ustbx_plan* pl, hipError_t& err) {
 // and dimension both with the resident receive table, on linear and sector
 // scans with das_c's edge rule, frames below 2 GiB, every nonzero weight and
 // every delay finite, and scans fine enough that a patch tile's windows fit an
-// LDS row. The receive table of dimension receive and none may take this
-// fraction of the device memory; where it cannot be had the per-lane kernel
-// runs, as for every other plan.
-constexpr double kWindowTableMaxFraction = 0.125;
+// LDS row. The receive table of dimension receive and none may take these
+// fractions of the device memory and of what is free of it (the facade's four
+// plans then hold an eighth of the device at most); where it cannot be had the
+// per-lane kernel runs, as for every other plan.
+constexpr double kWindowTableMaxFraction = 1.0 / 32, kWindowTableMaxFree = 1.0 / 8;
 
 void window_free(ustbx_plan* pl) {
   (void)hipFree(pl->win_mem);
@@ -831,7 +832,7 @@ bool window_build(ustbx_plan* pl, hipError_t& err) {
   const size_t b_ref = !both && G.ref_phase ? al(sizeof(float2) * P) : 0;
   size_t free_b = 0, total_b = 0;
   if (hipMemGetInfo(&free_b, &total_b) != hipSuccess) return true;
-  if (b_rx > (size_t)(kWindowTableMaxFraction * (double)total_b)) return true;
+  if ((double)b_rx > std::min(kWindowTableMaxFraction * (double)total_b, kWindowTableMaxFree * (double)free_b)) return true;
 
   // tile shapes (depth bits, x bits, y bits), the squarest windows first; a
   // shape that pads the scan by more than a tenth over the least goes last
