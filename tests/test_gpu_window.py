@@ -258,3 +258,28 @@ def test_receive_table_is_bounded(cuda):
     assert torch.isfinite(torch.view_as_real(large.run(ch))).all()
     large.close()
     small.close()
+
+
+@pytest.mark.parametrize("N,nx,nz", [(12, 70, 90), (64, 300, 420)], ids=["one launch", "shape by shape"])
+@pytest.mark.parametrize("dim", [0, 1])
+def test_lists_of_wide_windows(cuda, N, nx, nz, dim):
+    """Coarse depths, where the first tile shape does not fit a short row: the
+    lists of all shapes from one launch (tables up to 96 MB) or shape by shape,
+    against the per-lane kernel."""
+    print(f"case window lists N={N} {nx} x {nz} dim={dim}", flush=True)
+    zmax, W = 4e-3 + nz * 0.75e-3, 3
+    L = int(2 * zmax / C * 10.4e6) + 200
+    prb, _, seq = _setup("linear", W, nx, nz, zmax, N)
+    scan = LinearScan(np.linspace(-8e-3, 8e-3, nx), np.linspace(4e-3, zmax, nz))
+    plan = make_plan(prb, scan, seq, n_samples=L, n_frames=1, sampling_frequency=10.4e6, initial_time=0.0,
+                     modulation_frequency=5.2e6, sound_speed=C, receive_apodization=TUKEY,
+                     transmit_apodization=Apodization(), dimension=dim, interpolation=0)
+    assert plan.variant == (0, 0, 0)
+    g = torch.Generator(cuda).manual_seed(N)
+    ch = torch.randn((1, W, N, L), dtype=torch.complex64, device=cuda, generator=g)
+    got = plan.run(ch)
+    plan.set_tiles(8, 1)
+    ref = plan.run(ch)
+    plan.close()
+    # the same FP32 terms, products and (receive) sums of 64 in another order
+    assert (got - ref).abs().max().item() <= 5e-6 * ref.abs().max().item()

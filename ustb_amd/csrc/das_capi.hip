@@ -828,11 +828,6 @@ bool window_build(ustbx_plan* pl, hipError_t& err) {
   G.rx_compact = G.wd == 0.0f ? 1 : 0;
   const size_t P = (size_t)G.P;
   auto al = [](size_t b) { return (b + 255) & ~size_t(255); };
-  const size_t b_rx = both ? 0 : al((G.rx_compact ? sizeof(float2) : sizeof(float4)) * (size_t)G.N * P);
-  const size_t b_ref = !both && G.ref_phase ? al(sizeof(float2) * P) : 0;
-  size_t free_b = 0, total_b = 0;
-  if (hipMemGetInfo(&free_b, &total_b) != hipSuccess) return true;
-  if ((double)b_rx > std::min(kWindowTableMaxFraction * (double)total_b, kWindowTableMaxFree * (double)free_b)) return true;
 
   // tile shapes (depth bits, x bits, y bits), the squarest windows first; a
   // shape that pads the scan by more than a tenth over the least goes last
@@ -859,40 +854,33 @@ bool window_build(ustbx_plan* pl, hipError_t& err) {
                (int64_t)(least >> 8) * ((G.F + 1) / 2) < 400))
     return true;
 
-  size_t tiles_max = 0;
-  for (const Shape& s : shapes) tiles_max = std::max(tiles_max, s.padded >> 8);
-  const size_t b_wl = al(sizeof(int4) * tiles_max * (size_t)G.W), b_cl = al(sizeof(int4) * tiles_max * (size_t)G.N);
-  const size_t b_cnt = al(sizeof(int) * tiles_max), b_info = al(sizeof(int) * 8);
-  const size_t total = b_rx + b_ref + b_wl + b_cl + 3 * b_cnt + b_info;
-  char* m = nullptr;
-  if (hipMalloc(&m, total) != hipSuccess) {
-    (void)hipGetLastError();
-    return true;
+  const size_t entry = G.rx_compact ? sizeof(float2) : sizeof(float4);
+  const size_t b_rx = both ? 0 : al(entry * (size_t)G.N * P);
+  const size_t b_ref = !both && G.ref_phase ? al(sizeof(float2) * P) : 0;
+  if (b_rx) {
+    size_t free_b = 0, total_b = 0;
+    if (hipMemGetInfo(&free_b, &total_b) != hipSuccess) return true;
+    if ((double)b_rx > std::min(kWindowTableMaxFraction * (double)total_b, kWindowTableMaxFree * (double)free_b))
+      return true;
   }
-  size_t off = 0;
-  auto take = [&](size_t b) {
-    char* q = m + off;
-    off += b;
-    return q;
-  };
-  float4* rx = b_rx ? (float4*)take(b_rx) : nullptr;
-  float2* ref = b_ref ? (float2*)take(b_ref) : nullptr;
-  int4* wl = (int4*)take(b_wl);
-  int4* cl = (int4*)take(b_cl);
-  int* nw = (int*)take(b_cnt);
-  int* nc = (int*)take(b_cnt);
-  int* ord = (int*)take(b_cnt);
-  int* info = (int*)take(b_info);
-  if (!both) err = launch_window_state(G, rx, ref, nullptr);
-  G.win_rx = both ? G.rx_table : rx;
-  G.win_ref = ref;
-  pl->win_mem = m;
-  pl->win_bytes = total;
-  WinTiles& T = G.win;
-  T.n0 = G.scan.n0;
-  T.n1 = G.scan.n1;
-  T.n2 = G.scan.n2;
-  auto lists = [&](const Shape& s, int* h) {
+
+  // Where a pass over the tables is short (up to 96 MB: 20 us), the lists of
+  // all shapes come from one launch and one readback (30 us); else shape by
+  // shape, since the first one mostly does. A plan of 150 x 201 pixels, 128
+  // channels, whose windows are wide: 0.46 -> 0.27 ms.
+  const int together = entry * (size_t)G.N * P + sizeof(float4) * (size_t)G.W * P <= (size_t)96 << 20 ? kWinShapes : 1;
+  const int count = (int)shapes.size();
+  std::vector<WinTiles> tiles((size_t)count);
+  std::vector<size_t> base((size_t)count);
+  size_t b_lists = 0, widest = 0;
+  for (int k = 0; k < count; ++k) {
+    const Shape& s = shapes[k];
+    WinTiles& T = tiles[k];
+    T.on = 0;
+    T.row = 0;
+    T.n0 = G.scan.n0;
+    T.n1 = G.scan.n1;
+    T.n2 = G.scan.n2;
     T.dzb = s.dzb;
     T.lxb = s.lxb;
     T.lyb = s.lyb;
@@ -904,70 +892,86 @@ bool window_build(ustbx_plan* pl, hipError_t& err) {
     T.nlx = (int)ceil_to(T.n1, s.lxb);
     T.nly = (int)ceil_to(T.n2, s.lyb);
     T.tiles = T.ntz * T.nlx * T.nly;
-    for (int i = 0; i < 8; ++i) h[i] = 0;
-    if (err == hipSuccess) err = hipMemcpy(info, h, sizeof(int) * 8, hipMemcpyHostToDevice);
-    // dimension none writes every (wave, channel), receive every wave
-    if (err == hipSuccess) err = launch_window_lists(G, nw, nc, wl, cl, info, !both, G.dim == 0, nullptr);
-    if (err == hipSuccess) err = hipMemcpy(h, info, sizeof(int) * 8, hipMemcpyDeviceToHost);
+    const size_t n = (size_t)T.tiles;
+    const size_t b = 3 * al(sizeof(int) * n) + al(sizeof(int4) * n * (size_t)G.W) + al(sizeof(int4) * n * (size_t)G.N);
+    base[k] = together > 1 ? b_lists : 0;
+    b_lists += b;
+    widest = std::max(widest, b);
+  }
+  if (together == 1) b_lists = widest;
+  const size_t b_info = al(sizeof(WinInfo) * kWinShapes);
+  const size_t total = b_rx + b_ref + b_info + b_lists;
+  char* m = nullptr;
+  if (hipMalloc(&m, total) != hipSuccess) {
+    (void)hipGetLastError();
+    return true;
+  }
+  float4* rx = b_rx ? (float4*)m : nullptr;
+  float2* ref = b_ref ? (float2*)(m + b_rx) : nullptr;
+  WinInfo* info = (WinInfo*)(m + b_rx + b_ref);
+  for (int k = 0; k < count; ++k) {
+    WinTiles& T = tiles[k];
+    char* q = m + b_rx + b_ref + b_info + base[k];
+    auto take = [&](size_t b) {
+      char* at = q;
+      q += al(b);
+      return at;
+    };
+    const size_t n = (size_t)T.tiles;
+    T.wl = (int4*)take(sizeof(int4) * n * (size_t)G.W);
+    T.cl = (int4*)take(sizeof(int4) * n * (size_t)G.N);
+    T.nw = (int*)take(sizeof(int) * n);
+    T.nc = (int*)take(sizeof(int) * n);
+    T.order = (int*)take(sizeof(int) * n);
+  }
+  if (!both) err = launch_window_state(G, rx, ref, nullptr);
+  G.win_rx = both ? G.rx_table : rx;
+  G.win_ref = ref;
+  pl->win_mem = m;
+  pl->win_bytes = total;
+  WinInfo h[kWinShapes];
+  // dimension none writes every (wave, channel), receive every wave
+  auto lists = [&](int k, int n) {
+    if (err == hipSuccess) err = hipMemsetAsync(info + k, 0, sizeof(WinInfo) * (size_t)n, nullptr);
+    if (err == hipSuccess) err = launch_window_lists(G, &tiles[k], n, info + k, !both, G.dim == 0, nullptr);
+    if (err == hipSuccess) err = hipMemcpy(h + k, info + k, sizeof(WinInfo) * (size_t)n, hipMemcpyDeviceToHost);
     return err == hipSuccess;
   };
   const int slack = G.interp == USTBX_INTERP_CUBIC ? 7 : 5;  // WinSpan::kSlack
-  int best = -1, best_span = 129, last = -1, max_nw = 0;
-  for (int k = 0; k < (int)shapes.size(); ++k) {
-    int h[8];
-    if (!lists(shapes[k], h)) {
+  int best = -1, best_span = 129, last = -1;
+  for (int k = 0; k < count; ++k) {
+    if ((together == 1 || k == 0) && !lists(k, together == 1 ? 1 : count)) {
       window_free(pl);
       return false;
     }
     last = k;
-    max_nw = std::max(max_nw, h[2]);
-    if (h[1]) break;  // weights or delays that are not finite: the per-lane kernel
-    if (h[0] + slack < best_span) {
+    if (h[k].bad) break;  // weights or delays that are not finite: the per-lane kernel
+    if (h[k].span + slack < best_span) {
       best = k;
-      best_span = h[0] + slack;
+      best_span = h[k].span + slack;
     }
     if (best_span <= 64) break;
   }
-  if (best >= 0) {
-    int h[8];
-    if (best != last && !lists(shapes[best], h)) {
-      window_free(pl);
-      return false;
-    }
-    const std::vector<int> order = line_band_order(T.ntz, T.tiles, 8);
-    err = hipMemcpy(ord, order.data(), sizeof(int) * order.size(), hipMemcpyHostToDevice);
-    if (err != hipSuccess) {
-      window_free(pl);
-      return false;
-    }
-    T.row = best_span <= 64 ? 64 : 128;
-    T.order = ord;
-    T.nw = nw;
-    T.nc = nc;
-    T.wl = wl;
-    T.cl = cl;
-    T.on = 1;
-    G.win_max_nw = max_nw;
-    if (both) {
-      G.win_rx = nullptr;  // the plan's receive table, which may be rebuilt
-      // how many tiles of the largest one's terms the plan holds
-      std::vector<int> tw((size_t)T.tiles), tc((size_t)T.tiles);
-      err = hipMemcpy(tw.data(), nw, sizeof(int) * tw.size(), hipMemcpyDeviceToHost);
-      if (err == hipSuccess) err = hipMemcpy(tc.data(), nc, sizeof(int) * tc.size(), hipMemcpyDeviceToHost);
-      if (err != hipSuccess) {
-        window_free(pl);
-        return false;
-      }
-      int64_t sum = 0, most = 1;
-      for (int t = 0; t < T.tiles; ++t) {
-        sum += (int64_t)tw[t] * tc[t];
-        most = std::max(most, (int64_t)tw[t] * tc[t]);
-      }
-      G.win_even = (int)(sum / most);
-    }
+  if (best < 0) {
+    window_free(pl);
     return true;
   }
-  window_free(pl);
+  if (together == 1 && best != last && !lists(best, 1)) {
+    window_free(pl);
+    return false;
+  }
+  G.win = tiles[best];
+  G.win.row = best_span <= 64 ? 64 : 128;
+  G.win.on = 1;
+  G.win_max_nw = h[best].max_nw;
+  // how many tiles of the largest one's terms the plan holds
+  G.win_even = (int)(h[best].terms / std::max(1ull, h[best].most));
+  if (both) {
+    G.win_rx = nullptr;  // the plan's receive table, which may be rebuilt
+    GeomLaunch own = G;
+    own.variant = 2;
+    if (!window_both_active(own)) window_free(pl);  // never run
+  }
   return true;
 }
 

@@ -41,15 +41,25 @@ struct WinTiles {
   int dzb, lxb, lyb, zl;
   int n0, n1, n2;      // the scan's axis lengths
   int ntz, nlx, nly, tiles;
-  const int* order;    // [tiles] visiting order
-  const int* nw;       // [tiles] entries of wl, cl
-  const int* nc;
+  int* order;          // [tiles] visiting order
+  int* nw;             // [tiles] entries of wl, cl
+  int* nc;
   // [tiles][W], [tiles][N] {index, floor of the tile's least delay in samples,
   // floor of its largest, bit 0: the weight is nonzero on every pixel of the
   // tile, bit 1: on some}; receive delays less t0
-  const int4* wl;
-  const int4* cl;
+  int4* wl;
+  int4* cl;
 };
+
+// What the lists of a tile shape hold.
+struct WinInfo {
+  int span;        // largest hi - lo sum of a tile's waves and channels
+  int bad;         // 1 where a nonzero weight or a delay is not finite
+  int max_nw;      // largest wave count of a tile
+  int unused;
+  unsigned long long terms, most;  // waves x channels of all tiles, of the largest
+};
+constexpr int kWinShapes = 4;  // candidate tile shapes of a plan
 
 // Geometry (on-the-fly) path: everything resident in device memory.
 struct GeomLaunch {
@@ -193,13 +203,11 @@ hipError_t launch_stage_mask(const GeomLaunch& g, const int* tile_bad, unsigned 
 // Receive table and reference phase of a window-staged plan (either may be
 // null: not written).
 hipError_t launch_window_state(const GeomLaunch& g, float4* rx_table, float2* ref_table, hipStream_t stream);
-// Tile lists of the window-staged kernels (g.win's shape, g.win_rx): nw, nc,
-// wl, cl as WinTiles names them; info[0] = largest hi - lo sum of a tile's
-// waves and channels, info[1] = 1 where a nonzero weight or a delay is not
-// finite, info[2] = largest wave count of a tile. full: every wave and channel
-// is listed.
-hipError_t launch_window_lists(const GeomLaunch& g, int* nw, int* nc, int4* wl, int4* cl, int* info, int full_w,
-                               int full_n, hipStream_t stream);
+// Tile lists of count tile shapes in one launch: T[k]'s order, nw, nc, wl, cl as
+// WinTiles names them and info[k], which starts as zeros (g.win_rx: the receive
+// table). full: every wave and channel is listed.
+hipError_t launch_window_lists(const GeomLaunch& g, const WinTiles* T, int count, WinInfo* info, int full_w, int full_n,
+                               hipStream_t stream);
 
 hipError_t launch_das_geom(const GeomLaunch& g, hipStream_t stream);
 

@@ -87,8 +87,9 @@ hipError_t launch_window_none(const GeomLaunch& G, int ph, hipStream_t s) {
 
 // ---------------------------------------------------------------------------
 // Tile lists, once per plan. One block of 16 wave64s per tile; wave s takes
-// every 16th wave and channel, its lanes the tile's 256 pixels in four passes. A slot of cl / wl is first filled in index order, then wave 0 closes
-// the gaps (ballots keep the order).
+// every 16th wave and channel, its lanes the tile's 256 pixels in four passes.
+// A slot of cl / wl is first filled in index order, then wave 0 closes the gaps
+// (ballots keep the order).
 // ---------------------------------------------------------------------------
 __device__ __forceinline__ int win_pixel(const WinTiles& T, int tile, int lid) {
   const int tz = tile % T.ntz, tg = tile / T.ntz;
@@ -122,19 +123,41 @@ __device__ __forceinline__ int sample_floor(float d, double t0, double fs, bool&
 
 constexpr int kListWaves = 16;
 
-__global__ __launch_bounds__(64 * kListWaves) void window_lists_kernel(GeomLaunch G, int* __restrict__ nw_out,
-                                                           int* __restrict__ nc_out, int4* __restrict__ wl,
-                                                           int4* __restrict__ cl, int* __restrict__ info, int full_w,
-                                                           int full_n) {
-  __shared__ int spans[2];  // largest hi - lo of the tile's waves, channels
-  const int tile = blockIdx.x;
+struct WinLists {
+  WinTiles t[kWinShapes];
+  int count;
+};
+
+// Place of tile t in the visiting order: each of 8 contiguous shares of the
+// tiles (one per XCD) depth band by depth band, tpl tiles down a line group.
+__device__ __forceinline__ int band_place(int t, int tpl, int tiles) {
+  const int q = tiles / 8, r = tiles % 8;
+  const int k = t < r * (q + 1) ? t / (q + 1) : r + (t - r * (q + 1)) / q;
+  const int s0 = k * q + min(k, r), cnt = q + (k < r ? 1 : 0);
+  const int b = t % tpl, r0 = s0 % tpl, rem = cnt % tpl;
+  // tiles of the share in a band: cnt / tpl, and one more in the rem bands from r0 on (cyclic)
+  const int wrap = r0 + rem - tpl;
+  const int more = wrap <= 0 ? max(0, min(b, r0 + rem) - r0) : min(b, wrap) + max(0, b - r0);
+  const int first = s0 + (b - r0 + tpl) % tpl;
+  return s0 + b * (cnt / tpl) + more + (t - first) / tpl;
+}
+
+__global__ __launch_bounds__(64 * kListWaves) void window_lists_kernel(GeomLaunch G, WinLists C,
+                                                                       WinInfo* __restrict__ infos, int full_w,
+                                                                       int full_n) {
+  __shared__ int spans[2];   // largest hi - lo of the tile's waves, channels
+  __shared__ int counts[2];  // entries
+  int k = 0, tile = blockIdx.x;
+  while (tile >= C.t[k].tiles) tile -= C.t[k++].tiles;
+  const WinTiles T = C.t[k];
+  WinInfo* info = infos + k;
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
   const size_t PS = (size_t)G.P;
   int px[4];
 #pragma unroll
-  for (int i = 0; i < 4; ++i) px[i] = win_pixel(G.win, tile, i * 64 + lane);
-  int4* tw = wl + (size_t)tile * G.W;
-  int4* tc = cl + (size_t)tile * G.N;
+  for (int i = 0; i < 4; ++i) px[i] = win_pixel(T, tile, i * 64 + lane);
+  int4* tw = T.wl + (size_t)tile * G.W;
+  int4* tc = T.cl + (size_t)tile * G.N;
   bool bad = false;
   for (int e = wave; e < G.W + G.N; e += kListWaves) {
     const bool rx = e >= G.W;
@@ -166,7 +189,7 @@ __global__ __launch_bounds__(64 * kListWaves) void window_lists_kernel(GeomLaunc
     }
     if (lane == 0) (rx ? tc : tw)[k] = out;
   }
-  if (__any(bad) && lane == 0) atomicOr(&info[1], 1);
+  if (__any(bad) && lane == 0) atomicOr(&info->bad, 1);
   __syncthreads();
   if (wave < 2) {  // wave 0: the transmit list, wave 1: the channels
     int4* t = wave == 0 ? tw : tc;
@@ -184,20 +207,32 @@ __global__ __launch_bounds__(64 * kListWaves) void window_lists_kernel(GeomLaunc
 #pragma unroll
     for (int o = 32; o > 0; o >>= 1) span = max(span, __shfl_xor(span, o));
     if (lane == 0) {
-      (wave == 0 ? nw_out : nc_out)[tile] = cnt;
+      (wave == 0 ? T.nw : T.nc)[tile] = cnt;
+      counts[wave] = cnt;
       spans[wave] = span;
-      if (wave == 0) atomicMax(&info[2], cnt);
     }
   }
   __syncthreads();
-  if (threadIdx.x == 0) atomicMax(&info[0], spans[0] + spans[1]);
+  if (threadIdx.x == 0) {
+    const unsigned long long terms = (unsigned long long)counts[0] * (unsigned long long)counts[1];
+    atomicMax(&info->span, spans[0] + spans[1]);
+    atomicMax(&info->max_nw, counts[0]);
+    atomicAdd(&info->terms, terms);
+    atomicMax(&info->most, terms);
+    T.order[band_place(tile, T.ntz, T.tiles)] = tile;
+  }
 }
 
-hipError_t launch_window_lists(const GeomLaunch& G, int* nw, int* nc, int4* wl, int4* cl, int* info, int full_w,
-                               int full_n, hipStream_t stream) {
-  hipLaunchKernelGGL(window_lists_kernel, dim3((unsigned)G.win.tiles), dim3(64 * kListWaves), 0, stream, G, nw, nc, wl,
-                     cl, info,
-                     full_w, full_n);
+hipError_t launch_window_lists(const GeomLaunch& G, const WinTiles* T, int count, WinInfo* info, int full_w, int full_n,
+                               hipStream_t stream) {
+  WinLists C;
+  unsigned tiles = 0;
+  for (int k = 0; k < count; ++k) {
+    C.t[k] = T[k];
+    tiles += (unsigned)T[k].tiles;
+  }
+  C.count = count;
+  hipLaunchKernelGGL(window_lists_kernel, dim3(tiles), dim3(64 * kListWaves), 0, stream, G, C, info, full_w, full_n);
   return hipGetLastError();
 }
 
