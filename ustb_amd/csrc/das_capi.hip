@@ -849,10 +849,19 @@ bool window_build(ustbx_plan* pl, hipError_t& err) {
   std::stable_partition(shapes.begin(), shapes.end(), [&](const Shape& s) { return s.padded <= least + least / 10; });
   if (least > 2 * P + 1024) return true;  // a scan of a few lines or depths
   // dimension both: no tables for a plan that the gathering kernel runs anyway
-  // (window_both_active)
-  if (both && (G.W < 9 || (G.interp == USTBX_INTERP_CUBIC && G.F == 1) ||
-               (int64_t)(least >> 8) * ((G.F + 1) / 2) < 400))
-    return true;
+  // (window_both_active). Its work in full tiles is near a quarter of that in
+  // the receive-table kernel's tiles of 64: at most 1.11 times on 59 linear,
+  // sector and volume plans.
+  if (both) {
+    if (G.W < 9 || (G.interp == USTBX_INTERP_CUBIC && G.F == 1)) return true;
+    int64_t sum = 0, most = 1;
+    for (int64_t c : pl->h_cost) {
+      sum += c;
+      most = std::max(most, c);
+    }
+    const int64_t even = std::min<int64_t>((int64_t)(least >> 8), sum * 5 / (most * 16));  // 1.25 / 4
+    if (even * ((G.F + 1) / 2) < (G.W <= 10 ? 640 : G.W <= 24 ? 512 : 400)) return true;
+  }
 
   const size_t entry = G.rx_compact ? sizeof(float2) : sizeof(float4);
   const size_t b_rx = both ? 0 : al(entry * (size_t)G.N * P);
