@@ -204,7 +204,7 @@ __device__ __forceinline__ void tx_channel(const RxAcq& A, float wd, int tile, i
     }
     __builtin_amdgcn_sched_barrier(0);
     float c0 = 0.f, c1 = 0.f, c2 = 0.f, c3 = 0.f;
-    if (SM == SM_CUBIC) keys_weights_short(b, c0, c1, c2, c3);
+    if (SM == SM_CUBIC) keys_weights_horner(b, c0, c1, c2, c3);
 #pragma unroll
     for (int f = 0; f < FC; ++f) {
       float2 np = part[f];

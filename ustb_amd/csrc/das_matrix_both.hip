@@ -234,7 +234,7 @@ __global__ __launch_bounds__(64 * kWS) void das_matrix_both_kernel(MatBoth A) {
             const float2 w = IQ ? dasc_rotation(T[j], ok[i] ? td[j] : 0.0f, ok[i] ? rd : 0.0f, wd, ok[i] ? c[i] : 0.0f)
                                 : T[j];
             float k0w = 0.f, k1w = 0.f, k2w = 0.f, k3w = 0.f;
-            if (SM == SM_CUBIC) keys_weights_short(b[i], k0w, k1w, k2w, k3w);
+            if (SM == SM_CUBIC) keys_weights_horner(b[i], k0w, k1w, k2w, k3w);
 #pragma unroll
             for (int f = 0; f < FC; ++f) {
               float2 sm;

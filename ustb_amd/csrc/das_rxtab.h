@@ -91,17 +91,13 @@ __device__ __forceinline__ float4 rx_entry(const float4* __restrict__ rxt, int c
   return compact ? rx_entry_t<true>(rxt, idx) : rx_entry_t<false>(rxt, idx);
 }
 
-// Keys' cubic weights (a = -1/2) of the fraction b, u = 1 - b: the outer two are
-// -b u^2 / 2 and -b^2 u / 2, and the inner two follow from sum 1 and first
-// moment b. 9 instructions; four polynomials in Horner form take 11 (75 plane
-// waves on 512 x 1024 pixels: 2.20 -> 2.15 ms), with errors of 0.26 to 1.1 times
-// theirs (RMS over [0, 1)).
-__device__ __forceinline__ void keys_weights_short(float b, float& c0, float& c1, float& c2, float& c3) {
-  const float u = 1.0f - b, h = (-0.5f * b) * u;
-  c0 = h * u;
-  c3 = h * b;
-  c1 = fmaf(-2.0f, c0, fmaf(h, b, u));
-  c2 = fmaf(-2.0f, c3, fmaf(h, u, b));
+// Keys' cubic weights (a = -1/2) in Horner form.
+__device__ __forceinline__ void keys_weights_horner(float b, float& c0, float& c1, float& c2, float& c3) {
+  const float b2 = b * b;
+  c0 = b * fmaf(b, fmaf(-0.5f, b, 1.0f), -0.5f);
+  c1 = fmaf(b2, fmaf(1.5f, b, -2.5f), 1.0f);
+  c2 = b * fmaf(b, fmaf(-1.5f, b, 2.0f), 0.5f);
+  c3 = b2 * fmaf(0.5f, b, -0.5f);
 }
 
 // das_c's sample index of a term (das_c.cpp:372,375), FMA contraction off:
@@ -206,7 +202,7 @@ __device__ __forceinline__ float2 rxtab_channel(__amdgpu_buffer_rsrc_t rs, const
         } else if (SM == SM_CUBIC) {
           const float4 lo = q[i][0], hi = q[i][M::kLoads - 1];
           float c0, c1, c2, c3;
-          keys_weights_short(b, c0, c1, c2, c3);
+          keys_weights_horner(b, c0, c1, c2, c3);
           sm = make_float2(fmaf(c3, hi.z, fmaf(c2, hi.x, fmaf(c1, lo.z, c0 * lo.x))),
                            fmaf(c3, hi.w, fmaf(c2, hi.y, fmaf(c1, lo.w, c0 * lo.y))));
         } else {
@@ -300,7 +296,7 @@ __device__ __forceinline__ float2 rxtab_channel_staged(__amdgpu_buffer_rsrc_t rs
           const f4a8 lo = wp[0];
           const f4a8 hi = wp[1];
           float c0, c1, c2, c3;
-          keys_weights_short(b, c0, c1, c2, c3);
+          keys_weights_horner(b, c0, c1, c2, c3);
           sm = make_float2(fmaf(c3, hi.z, fmaf(c2, hi.x, fmaf(c1, lo.z, c0 * lo.x))),
                            fmaf(c3, hi.w, fmaf(c2, hi.y, fmaf(c1, lo.w, c0 * lo.y))));
         }
@@ -441,7 +437,7 @@ __device__ __forceinline__ void rxtab_channels_few(__amdgpu_buffer_rsrc_t rs, co
           sm = make_float2(fmaf(b, lo.z - lo.x, lo.x), fmaf(b, lo.w - lo.y, lo.y));
         } else if (SM == SM_CUBIC) {
           float c0, c1, c2, c3;
-          keys_weights_short(b, c0, c1, c2, c3);
+          keys_weights_horner(b, c0, c1, c2, c3);
           sm = make_float2(fmaf(c3, hi.z, fmaf(c2, hi.x, fmaf(c1, lo.z, c0 * lo.x))),
                            fmaf(c3, hi.w, fmaf(c2, hi.y, fmaf(c1, lo.w, c0 * lo.y))));
         } else {

@@ -406,7 +406,7 @@ struct WinKernel {
           static_for<kB>([&](auto u) {
             constexpr int J = J0 + decltype(u)::value;
             float kw[4] = {0.f, 0.f, 0.f, 0.f};
-            if constexpr (SM == SM_CUBIC) keys_weights_short(t[u].b, kw[0], kw[1], kw[2], kw[3]);
+            if constexpr (SM == SM_CUBIC) keys_weights_horner(t[u].b, kw[0], kw[1], kw[2], kw[3]);
             float wr = 0.0f, wi = 0.0f;
             if constexpr (!kSep) exact_weight(t[u].ok ? td[J] : 0.0f, t[u].ok ? rd : 0.0f, Tw[J].x, ra, wd, wr, wi);
             static_for<FT>([&](auto f) {
