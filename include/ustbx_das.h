@@ -360,9 +360,11 @@ int ustbx_batch_set_io(ustbx_batch* batch, const void* const* ch, void* const* o
 /* Tile shape of the persistent kernel (0 = keep): waves per split (4, 5, 6,
  * 8, 10, 12, 16) and wave-splits per 64-pixel tile (4, 5 or 8). The default
  * follows the wave count below which half of the batch's work lies: 8 splits of
- * 4 (up to 4 waves), 8 (8), 6 (12), 8 (16) or 16 (32) waves, above that 8
- * splits covering it in one round; 4 splits of 8 up to 32 waves where an
- * acquisition computes its receive state in place. Drops a captured graph. */
+ * 4 (up to 4 waves), 5 (5), 8 (8), 5 (10), 6 (12), 8 (16) or 16 (32) waves, with
+ * 8 for 16 above 8000 work items; above 32 waves 8 splits covering them in one
+ * round; 4 splits of 8 up to 32 waves for batches of some 15000 to 30000 items
+ * and where an acquisition computes its receive state in place. Drops a
+ * captured graph. */
 int ustbx_batch_set_tiles(ustbx_batch* batch, int32_t wave_chunk, int32_t split, ustbx_status* st);
 /* Enqueues the batch on stream: a counter-reset kernel and the persistent
  * kernel; allocates nothing and can be captured in a hipGraph. Launches of

@@ -82,7 +82,7 @@ def test_against_one_channel_at_a_time(cuda, case):
 def test_default_shape_follows_the_receive_state(cuda):
     """The kernel that computes the receive state keeps the shapes it was
     measured with, a shape that was set stays."""
-    plan = _plan(6, 33, False, False, 1, 500, TUKEY)
+    plan = _plan(5, 33, False, False, 1, 500, TUKEY)
     assert plan.variant == (2, 6, 8)
     plan.set_variant(4)
     assert plan.variant == (4, 4, 8)
@@ -105,4 +105,26 @@ def test_a_refused_variant_leaves_the_plan_as_it_was(cuda):
     assert plan.variant == v
     print("case refused variant", flush=True)
     assert torch.equal(plan.run(ch), ref)
+    plan.close()
+
+
+@pytest.mark.parametrize("kind,W,nx,nz,F,cubic,shape", [
+    ("volume", 4, 30, 70, 1, False, (4, 8)),    # 2297 blocks: images of 3 and 4 waves take 4 splits there
+    ("linear", 4, 400, 330, 1, False, (4, 4)),  # 2063
+    ("sector", 5, 150, 154, 2, True, (5, 8)),   # 722
+    ("sector", 9, 150, 164, 1, True, (5, 4)),   # 385
+    ("sector", 20, 150, 147, 1, False, (16, 4)),  # 345
+    ("sector", 20, 100, 147, 1, False, (16, 8)),  # 230
+])
+def test_default_shapes(cuda, kind, W, nx, nz, F, cubic, shape):
+    """Where a shape for few blocks, few splits or many registers was slower than the one before it."""
+    print(f"case default shape {kind} W={W} {nx} x {nz}", flush=True)
+    seq = [Wave.spherical(x, 0.0, -10e-3, sound_speed=C, origin=(x, 0.0, -10e-3)) for x in np.linspace(-4e-3, 4e-3, W)]
+    x, z = np.linspace(-8e-3, 8e-3, nx), np.linspace(2e-3, 25e-3, nz)
+    scan = (SectorScan(np.deg2rad(np.linspace(-40, 40, nx)), z) if kind == "sector" else
+            LinearScan(x, z, np.linspace(-8e-3, 8e-3, 70) if kind == "volume" else (0.0,)))
+    plan = make_plan(LinearArray(33, 0.3e-3), scan, seq, n_samples=500, n_frames=F, sampling_frequency=10.4e6,
+                     initial_time=0.0, modulation_frequency=5.2e6, sound_speed=C, receive_apodization=TUKEY,
+                     interpolation=int(cubic), separable_phase=True)
+    assert plan.variant == (2, *shape)
     plan.close()

@@ -336,13 +336,29 @@ int ustbx_batch_create(const ustbx_plan* const* plans, int32_t count, ustbx_batc
   if (nw_med <= 32 && b->otf) {
     ws = 4;  // measured with 8 x 4 only
   } else if (nw_med <= 32) {
-    // us per batch against 8 x 4, linear array and sector: 12 images of 255 x
-    // 255 pixels of 3 waves 353, 376 -> 292, 306; of 7 450, 503 -> 432, 478; of 11
-    // 613, 718 -> 563, 641; of 14 674, 813 -> 659, 777; of 20 889, 1155 -> 894,
-    // 1076; 5 of 100 x 200, 11 waves 213, 244 -> 140, 160. Volumes of 9 waves 752
-    // -> 705, of 25 (larger ones) 22515 -> 19305. 12 x 4 is 3 % faster
-    // than 6 x 8 on the large batches and 20-40 % slower on the small ones.
-    wc = nw_med <= 4 ? 4 : nw_med <= 8 ? 8 : nw_med <= 12 ? 6 : nw_med <= 16 ? 8 : 16;
+    // 180 random batches of 3-24 images (linear arrays, sectors and volumes, 2-31
+    // waves, 570-67000 items) against 8 x 4: 1.18 times as fast in the mean, none
+    // more than 1 % slower. 8 splits of what one round holds, since an item's own
+    // chain counts at the end of a batch (a batch of 700 items of 7 waves 1.7);
+    // where many items keep every CU busy until then, the shapes with fewer
+    // splits win: 8 x 8 of 7 waves 1.13 at 9600 items, 0.92 at 35000; of 14 waves,
+    // cubic, 1.37 at 650, 0.94 and 0.88 at 16000 and 27000; 16 x 8 of 24-31 waves
+    // 1.9 at 570, 1.0-1.1 at 8000, 0.75-0.97 beyond 14000 (8 x 8 0.99-1.06).
+    const int64_t n = (int64_t)items.size();
+    const bool cubic = interp == USTBX_INTERP_CUBIC;
+    wc = nw_med <= 4 ? 4 : nw_med <= 5 ? 5 : nw_med <= 8 ? 8 : nw_med <= 10 ? 5 : nw_med <= 12 ? 6 : 8;
+    bool few = false;
+    if (nw_med > 5 && nw_med <= 8) few = n >= 20000;
+    if (nw_med > 10 && nw_med <= 12) few = cubic && n >= 15000;
+    if (nw_med > 12 && nw_med <= 16) few = n >= 15000;
+    if (nw_med > 16) {
+      if (n < 8000) wc = 16;
+      few = n >= 30000;
+    }
+    if (few) {
+      wc = 8;
+      ws = 4;
+    }
   } else {
     const int need = (nw_med + 7) / 8;
     wc = need <= 4 ? 4 : need <= 6 ? 6 : need <= 8 ? 8 : need <= 10 ? 10 : need <= 12 ? 12 : 16;

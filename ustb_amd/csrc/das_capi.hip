@@ -62,17 +62,17 @@ constexpr double kRxTableMaxFraction = 0.5;
 
 bool rxtab_wc_ok(int wc) { return wc == 4 || wc == 5 || wc == 6 || wc == 8 || wc == 10 || wc == 12 || wc == 16; }
 
+void rxtab_default_tiles(const GeomLaunch& G, int max_nw, int& wc, int& ws);
+
 // Dimension transmit: 8 frames per block (4 when fewer), 8 channels per block
 // (4 when fewer).
-void rxtab_default_tiles(int64_t blocks, int max_nw, bool cubic, bool otf, int& wc, int& ws);
-
 void rxtab_defaults(const GeomLaunch& G, int max_nw, int& wc, int& ws) {
   if (G.dim == 2) {  // frames per block, channels per block (measured best on 32 frames x 64 channels)
     wc = G.F >= 8 ? 8 : 4;
     ws = G.N >= 8 ? 8 : 4;
     return;
   }
-  rxtab_default_tiles((int64_t)((G.P + 63) / 64) * G.F, max_nw, G.interp == USTBX_INTERP_CUBIC, G.rx_otf != 0, wc, ws);
+  rxtab_default_tiles(G, max_nw, wc, ws);
   // Keys' cubic over many waves: 4 splits of 10 waves (C2, 75 waves:
   // 2.49 ms against 2.57 ms with 8 splits)
   if (G.interp == USTBX_INTERP_CUBIC && max_nw > 32) {
@@ -82,62 +82,60 @@ void rxtab_defaults(const GeomLaunch& G, int max_nw, int& wc, int& ws) {
 }
 
 // Waves per split and splits by the waves of the busiest tile and the blocks
-// (tiles x frames) there are to run. Measured on a linear array with plane
-// waves and a sector with diverging waves, 3..31 waves, 188, 600, 1500 and 4000
-// blocks, us per pass:
-// - Fewer than 400 blocks leave most of the chip idle, so a block's own chain
-//   counts: 8 splits, as many waves in each as one round holds (the other
-//   splits take channel groups). 12 waves linear 69.0 -> 31.4, sector 49.3 ->
-//   31.5; 16 waves 69.1 -> 38.7; 25 waves 97.1 -> 56.4 against 8 x 4 and 16 x 4.
-// - 5..8 waves in one round of one split beat two splits of 4 (5 waves at 600
-//   blocks 30.8 -> 23.4), and from 1000 blocks with half the splits (5 waves,
-//   4000 blocks 126.9 -> 83.5; 8 waves, sector 156.9 -> 140.9). Keys' cubic
-//   needs the registers: 6..8 waves keep 4 x 8 there (8 waves at 1500 blocks
-//   70.8 against 73.5).
-// - 9..12 waves: one split of 12 up to 1000 blocks (600: 70.7 -> 54.3, 10 x 4
-//   and 16 x 4 within 3 %), two of 6 beyond (1500: 79.5 -> 73.3; 4000: within
-//   2 % either way).
-// - 3 and 4 waves: 4 splits from 2000 blocks (4000: 89.5 -> 77.7).
-// 13..32 waves from 400 blocks as before: 8 x 4 and 16 x 4 (8 x 8 is up to 30 %
-// faster on the linear array and as much slower on the sector). The kernels
-// that compute the receive geometry have only been measured with the shapes
-// for many blocks. More waves: 8 splits with the smallest waves-per-split
-// covering the busiest tile in one round (else 16 per round).
-void rxtab_default_tiles(int64_t blocks, int max_nw, bool cubic, bool otf, int& wc, int& ws) {
-  if (max_nw <= 4) {  // one wave-split; the others take shares of the channels
-    wc = 4;
-    ws = max_nw > 2 && blocks >= 2000 && !otf ? 4 : 8;
-    return;
-  }
+// (tiles x frames) there are to run. Against 4 x 8 (up to 8 waves), 8 x 4 (16)
+// and 16 x 4 (32) on 690 random plans (linear arrays, sectors, volumes; linear
+// and cubic, IQ and RF, 1-3 frames, 32-400 channels, 100-6000 blocks) the
+// choice is 1.08 times as fast in the mean, and 2 of the plans lose 2 %:
+// - Under 256 blocks a CU has at most one, so its own chain counts: 8 splits,
+//   as many waves in each as one round holds (the other splits take channel
+//   groups). 9-12 waves 1.24-1.89 times as fast, 17-32 waves 1.04-1.72; from 256
+//   blocks on as often slower. Cubic plans, which need the registers, with less
+//   in each split: 9 and 10 waves in 5 x 8 1.14-1.83.
+// - 12 x 4 has 5 blocks on a CU, so up to 1280 blocks all are resident: 11 and 12
+//   waves on linear arrays 0.99-1.29 there, beyond 0.83-1.18 against 0.99-1.12 in 6
+//   x 4. On sectors, whose tiles differ more, 0.99-1.28 up to 768 blocks and
+//   0.94-1.30 up to 1280. 9 and 10 waves leave slots of it empty: on linear arrays
+//   0.98-1.19 up to 1000 blocks, on sectors 0.94-1.26, so 6 x 4 there (0.99-1.02).
+// - 5..8 waves in one split: 5 x 4 and 6 x 4 from 1000 blocks, 1.07-1.61 and
+//   1.16-1.27; under 1000 only 5 waves gain (6 x 8, 1.07-1.24). Cubic: 5 x 8
+//   0.98-1.22, from 1000 blocks 5 x 4 1.06-1.45, 6 waves in 8 x 4 1.02-1.22, 7 and 8
+//   waves keep 4 x 8 (others 0.83-1.26).
+// - 3 and 4 waves: 4 splits from 2000 blocks on images (1.05-1.30; on volumes
+//   0.94-1.20).
+// - The rest: 8 x 4 and 16 x 4 (13-32 waves, 256 blocks and more: 8 x 8 and 16 x 8
+//   0.6-1.6 without a line between; the 3-D class, 25 waves, 52.3 ms in two
+//   channel groups of two 16-wave splits against 55.9 at 8 x 4).
+// The kernels that compute the receive geometry have only been measured with
+// the shapes compared against. More waves: 8 splits with the smallest
+// waves-per-split covering the busiest tile in one round (else 16 per round).
+void rxtab_default_tiles(const GeomLaunch& G, int max_nw, int& wc, int& ws) {
+  const int64_t blocks = (int64_t)((G.P + 63) / 64) * G.F;
+  const bool cubic = G.interp == USTBX_INTERP_CUBIC, one_per_cu = blocks < 256;
+  auto shape = [&](int c, int s) {
+    wc = c;
+    ws = s;
+  };
+  if (G.rx_otf && max_nw <= 32) return max_nw <= 8 ? shape(4, 8) : max_nw <= 16 ? shape(8, 4) : shape(16, 4);
+  if (max_nw <= 2) return shape(4, 8);  // the others take shares of the channels
+  if (max_nw <= 4) return shape(4, blocks >= 2000 && G.scan.n2 <= 1 ? 4 : 8);
+  if (max_nw == 5) return blocks >= 1000 ? shape(5, 4) : cubic ? shape(5, 8) : shape(6, 8);
+  if (max_nw == 6) return blocks < 1000 ? shape(4, 8) : cubic ? shape(8, 4) : shape(6, 4);
   if (max_nw <= 8) {
-    const bool wide_cubic = cubic && (max_nw > 6 ? blocks >= 400 : max_nw == 6 && blocks >= 1000 && blocks < 2000);
-    if (otf || wide_cubic) {
-      wc = 4;
-      ws = 8;
-      return;
-    }
-    wc = max_nw > 6 ? 8 : max_nw == 6 || blocks < 1000 ? 6 : 5;
-    ws = blocks < 1000 ? 8 : 4;
-    return;
+    if (cubic) return shape(4, 8);
+    return blocks >= 1000 ? shape(8, 4) : one_per_cu ? shape(8, 8) : shape(4, 8);
   }
-  if (max_nw <= 32) {
-    ws = 4;
-    if (otf)
-      wc = max_nw <= 16 ? 8 : 16;
-    else if (blocks < 400) {
-      wc = max_nw <= 12 ? 12 : 16;
-      ws = 8;
-    } else if (max_nw <= 12)
-      wc = blocks < 1000 ? 12 : 6;
-    else
-      // above 16: two channel groups of two 16-wave splits (the 3-D class, 25
-      // waves: 52.3 ms against 55.9 ms at 8 x 4)
-      wc = max_nw <= 16 ? 8 : 16;
-    return;
+  if (max_nw <= 10 && cubic) return one_per_cu ? shape(5, 8) : shape(5, 4);
+  if (max_nw <= 12) {
+    if (cubic) return one_per_cu ? shape(6, 8) : shape(8, 4);
+    if (one_per_cu) return shape(12, 8);
+    const bool sector = G.scan.kind == SCAN_SECTOR;
+    const int64_t resident = max_nw <= 10 ? (sector ? 0 : 1000) : sector ? 768 : 1280;
+    return blocks < resident ? shape(12, 4) : shape(6, 4);
   }
-  ws = 8;
+  if (max_nw <= 16) return one_per_cu ? shape(8, 8) : shape(8, 4);
+  if (max_nw <= 32) return one_per_cu ? shape(16, 8) : shape(16, 4);
   const int need = (max_nw + 7) / 8;
-  wc = need <= 4 ? 4 : need <= 6 ? 6 : need <= 8 ? 8 : need <= 10 ? 10 : need <= 12 ? 12 : 16;
+  shape(need <= 4 ? 4 : need <= 6 ? 6 : need <= 8 ? 8 : need <= 10 ? 10 : need <= 12 ? 12 : 16, 8);
 }
 
 }  // namespace
