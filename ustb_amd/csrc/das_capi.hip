@@ -562,11 +562,12 @@ std::vector<int> band_major_order(const GeomLaunch& G, int tiles, int shares) {
     // and begin the next; it goes by the depth of its first pixel. Worth it
     // for images whose frame of traces is well beyond an XCD's 4 MB L2, with
     // three bands or more and, in dimension both, more tiles than are resident
-    // at once. Against pixel order, dimension both, 23 such plans of 10-116 MB
-    // ran 1.0-1.31 times as fast (1.07 in the mean), under 1000 tiles 0.90-1.16
-    // (193 x 321 pixels, 128 channels RF, 20 waves 103 -> 114 us), below 10 MB
-    // 0.97-1.04, 23 volumes 0.94-1.03 at any size; dimension transmit
-    // 0.99-1.7, below 10 MB 0.97-1.03, lines of 129 and 131 depths 0.72 and 0.82.
+    // at once. Against pixel order, dimension both, 91 such plans of 10-154 MB
+    // ran 0.98-1.82 times as fast (sectors 1.26 in the mean, linear arrays 1.10;
+    // two more lost 3 %). Linear arrays under 1000 tiles: 20 plans 0.90-1.17, five
+    // of them 2-10 % slower; below 10 MB 0.97-1.04, 23 volumes 0.94-1.03 at any
+    // size. Dimension transmit: 48 plans 0.97-1.06, lines of 129 and 131 depths
+    // 0.72 and 0.82.
     if (sc.n2 > 1 || sc.n0 < 192 || (int64_t)G.L * G.N * G.W * 8 < 10 * 1000 * 1000 || (G.dim == 3 && tiles < 1000))
       return order;
     const int64_t n0 = sc.n0;

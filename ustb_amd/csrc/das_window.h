@@ -389,7 +389,7 @@ struct WinKernel {
         const unsigned coff = (unsigned)(buf * kBufBytes + C * WC * FT * kRowBytes) - (unsigned)(blo << kShift);
         // batches of kB waves: their samples are all asked for before the first
         // is used
-        constexpr int kBmax = WC * FT <= 4 ? WC : (FT >= 4 ? 1 : 4 / FT);
+        constexpr int kBmax = WC * FT <= 4 ? WC : 4 / FT;  // FT 1 or 2
         static_for<(WC + kBmax - 1) / kBmax>([&](auto gr) {
           constexpr int J0 = kBmax * decltype(gr)::value;
           constexpr int kB = WC - J0 < kBmax ? WC - J0 : kBmax;
