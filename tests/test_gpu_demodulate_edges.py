@@ -57,3 +57,12 @@ def test_edges_against_fp64(cuda, K, n, down, mode):
     assert np.array_equal(np.isnan(got.real), np.isnan(bad.real))
     ok = ~np.isnan(bad.real)
     assert (np.abs(got - bad)[ok] <= (2 * K + 8) * 2.0 ** -24 * mag[ok] + 1e-30).all()
+
+
+@pytest.mark.parametrize("mode,K", [(L.FIR_CAUSAL, 63), (L.FIR_CAUSAL, 64), (L.FIR_CAUSAL, 65), (L.FIR_CAUSAL, 767),
+                                    (L.FIR_ZERO_PHASE, 32), (L.FIR_ZERO_PHASE, 33), (L.FIR_ZERO_PHASE, 129),
+                                    (L.FIR_ZERO_PHASE, 384)])
+@pytest.mark.parametrize("n", [1156, 2311])
+def test_long_filters_without_decimation(cuda, mode, K, n):
+    """Taps in LDS from 64 on (zero phase: of the autocorrelation), up to the longest filters."""
+    test_edges_against_fp64(cuda, K, n, 1, mode)

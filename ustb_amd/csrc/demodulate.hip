@@ -34,8 +34,11 @@
 // 68 us at decimation 2 with the standard low-pass (53 us is a copy of the
 // bytes); with 21 taps at decimation 1, 2, 3 and 4 causal 200 -> 128, 74 -> 55,
 // 76 -> 59 and 98 -> 72 us, zero-phase 201 -> 130, 84 -> 70, 92 -> 78 and 122 ->
-// 102 us; the longest zero-phase filters (257 taps) are at their multiply-adds
-// either way (445 and 471 us). The sums are the same bits.
+// 102 us. A scalar load's wait is a wait for every LDS read before it, so long
+// filters at decimation 1, whose time is the tap loop, read their taps from LDS,
+// eight at a time: zero-phase 65 taps 175 -> 161 us, 129 247 -> 210, 257 470 -> 375;
+// causal 65 taps 138 -> 136, 129 240 -> 203; 57 and fewer 0-20 % slower, mostly on
+// few traces. The sums are the same bits.
 #include <hip/hip_runtime.h>
 #include <math.h>
 
@@ -59,6 +62,7 @@ constexpr int kDB = 256;         // threads per block
 constexpr int kSB = 9;
 constexpr int kMaxTaps = 767;    // passed by value (kernel arguments stay under 4 KB); zero-phase: K <= 384
 constexpr size_t kLdsMax = 64 * 1024;
+constexpr int kLdsTaps = 64;     // decimation 1: from here on the taps lie in LDS
 
 struct DemodArgs {
   const float* rf;
@@ -104,7 +108,7 @@ __device__ __forceinline__ float2 mixed(const float* __restrict__ x, int m, cons
 // two complex outputs in one store, at the alignment of one
 typedef float out4 __attribute__((ext_vector_type(4), aligned(8)));
 
-template <int kR, int DOWN, bool ZP>
+template <int kR, int DOWN, bool ZP, bool LT = false>
 __global__ __launch_bounds__(kDB) void demodulate_kernel(DemodArgs A) {
   extern __shared__ float2 lds[];
   const int down = DOWN ? DOWN : A.down, T = A.ntaps, PS = A.PS;
@@ -166,6 +170,10 @@ __global__ __launch_bounds__(kDB) void demodulate_kernel(DemodArgs A) {
       }
     }
   }
+  // LT: the taps beside the samples, for lanes to read together
+  const float* tl = reinterpret_cast<const float*>(lds + ((down * PS + 1) & ~1));
+  if (LT)
+    for (int i = tid; i < T; i += kDB) const_cast<float*>(tl)[i] = A.taps[i];
   __syncthreads();
   const int jt = kR * tid;                      // first output of this lane (block-local)
   if (jt >= jn) return;
@@ -181,7 +189,7 @@ __global__ __launch_bounds__(kDB) void demodulate_kernel(DemodArgs A) {
 #pragma unroll
     for (int k = 0; k < kR; ++k) w[k] = p[k];
     auto tap = [&](int q, int u) {
-      const float t = A.taps[tq + q + u];
+      const float t = LT ? tl[tq + q + u] : A.taps[tq + q + u];
 #pragma unroll
       for (int k = 0; k < kR; ++k) {
         const float2 s = w[(u + k) % kR];
@@ -344,9 +352,12 @@ int ustbx_demodulate(const float* rf, void* iq, int32_t L, int64_t traces, doubl
   const int64_t gy = (A.Lout + A.OB - 1) / A.OB;
   if (gy > 65535) return set_status(st, USTBX_E_ARG, "trace too long for the decimation factor");
   const dim3 grid((unsigned)traces, (unsigned)gy);
-  const size_t bytes = sizeof(float2) * (size_t)down * A.PS;
-  const bool zp = mode == USTBX_FIR_ZERO_PHASE;
-  if (down == 1)
+  const bool zp = mode == USTBX_FIR_ZERO_PHASE, lt = down == 1 && T >= kLdsTaps;
+  const size_t bytes = sizeof(float2) * (((size_t)down * A.PS + 1) & ~size_t(1)) + (lt ? sizeof(float) * (size_t)T : 0);
+  if (lt)
+    hipLaunchKernelGGL((zp ? demodulate_kernel<8, 1, true, true> : demodulate_kernel<8, 1, false, true>), grid,
+                       dim3(kDB), bytes, s, A);
+  else if (down == 1)
     hipLaunchKernelGGL((zp ? demodulate_kernel<8, 1, true> : demodulate_kernel<8, 1, false>), grid, dim3(kDB), bytes, s, A);
   else if (down == 2)
     hipLaunchKernelGGL((zp ? demodulate_kernel<4, 2, true> : demodulate_kernel<4, 2, false>), grid, dim3(kDB), bytes, s, A);
