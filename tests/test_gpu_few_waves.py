@@ -128,3 +128,22 @@ def test_default_shapes(cuda, kind, W, nx, nz, F, cubic, shape):
                      interpolation=int(cubic), separable_phase=True)
     assert plan.variant == (2, *shape)
     plan.close()
+
+
+@pytest.mark.parametrize("W,N,F,sector", [(1, 33, 1, False), (2, 21, 2, True)])
+def test_coefficient_variant(cuda, W, N, F, sector):
+    """Variant 3 (cubic coefficients) with one and two waves against variant 2's shapes of six slots."""
+    print("case few coefficients", W, N, F, flush=True)
+    plan = _plan(W, N, False, True, F, 500, TUKEY, sector=sector)
+    ch = torch.randn((F, W, N, 500), dtype=torch.complex64, device=cuda, generator=torch.Generator(cuda).manual_seed(N))
+    plan.set_tiles(6, 8)
+    ref = plan.run(ch)
+    plan.set_tiles(4, 8)
+    plan.set_variant(3)
+    assert plan.variant == (3, 4, 8)
+    got = plan.run(ch)
+    fin = torch.isfinite(torch.view_as_real(ref)).all(-1)
+    assert torch.equal(fin, torch.isfinite(torch.view_as_real(got)).all(-1))
+    # the same cubic by its polynomial's coefficients (FP32, magnitudes up to 10 samples), W * N terms
+    assert float((got - ref)[fin].abs().max()) <= 40 * W * N * 2.0 ** -24 * float(ref[fin].abs().max())
+    plan.close()

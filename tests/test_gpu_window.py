@@ -283,3 +283,66 @@ def test_lists_of_wide_windows(cuda, N, nx, nz, dim):
     plan.close()
     # the same FP32 terms, products and (receive) sums of 64 in another order
     assert (got - ref).abs().max().item() <= 5e-6 * ref.abs().max().item()
+
+
+SHAPES = [
+    # W, N, nx, nz, zmax, F, rf, cubic: the groups of 6, 8, 13 and 16 waves, more
+    # than 64 channels (no whole number of 32), rows of 128 samples (depths of
+    # 0.4 mm at 20.8 MHz, 0.8 mm at 10.4) for every data type
+    (9, 65, 640, 560, 25e-3, 1, False, False),
+    (15, 70, 420, 470, 25e-3, 1, False, False),
+    (26, 67, 360, 400, 25e-3, 1, True, False),
+    (31, 65, 360, 400, 25e-3, 1, False, False),
+    (16, 66, 200, 300, 25e-3, 5, False, False),
+    (11, 20, 1100, 256, 106e-3, 1, True, False),
+    (14, 20, 1100, 256, 208e-3, 1, False, False),
+    (26, 20, 1000, 256, 106e-3, 1, True, False),
+    (30, 20, 1000, 256, 208e-3, 1, False, False),
+    (12, 20, 600, 256, 106e-3, 4, True, False),
+    (15, 20, 600, 256, 208e-3, 3, False, False),
+    (11, 20, 600, 256, 106e-3, 3, True, True),
+    (15, 20, 600, 256, 208e-3, 4, False, True),
+]
+
+
+@pytest.mark.parametrize("W,N,nx,nz,zmax,F,rf,cubic", SHAPES)
+def test_both_every_shape(cuda, W, N, nx, nz, zmax, F, rf, cubic):
+    """Every shape that the dispatch of dimension both picks, against the gathering kernel."""
+    print(f"case window both shape W={W} N={N} {nx} x {nz} F={F} rf={rf} cubic={cubic}", flush=True)
+    fs, fd = (20.8e6, 0.0) if rf else (10.4e6, 5.2e6)
+    L = int(2.1 * zmax / C * fs)
+    prb, _, seq = _setup("linear", W, nx, nz, zmax, N)
+    scan = LinearScan(np.linspace(-8e-3, 8e-3, nx), np.linspace(4e-3, zmax, nz))
+    plan = make_plan(prb, scan, seq, n_samples=L, n_frames=F, sampling_frequency=fs, initial_time=0.0,
+                     modulation_frequency=fd, sound_speed=C, receive_apodization=Apodization(),
+                     transmit_apodization=Apodization(), dimension=3, interpolation=int(cubic), reference_phase=not rf)
+    assert plan.variant == (2, 0, 0)
+    g = torch.Generator(cuda).manual_seed(W)
+    ch = torch.randn((F, W, N, L), dtype=torch.complex64, device=cuda, generator=g)
+    ch[0, :, 2, 60:70] = float("nan")
+    got = plan.run(ch)
+    plan.set_tiles(8, 4)
+    ref = plan.run(ch)
+    plan.close()
+    a, b = torch.view_as_real(got), torch.view_as_real(ref)
+    assert torch.equal(torch.isnan(a), torch.isnan(b))
+    # as test_both_against_set_tiles: sums of at most 31 x 65 terms
+    assert (torch.nan_to_num(a - b).abs().max() / torch.nan_to_num(b).abs().max()).item() <= 5e-6
+
+
+@pytest.mark.parametrize("dim", [0, 1])
+@pytest.mark.parametrize("kind,W,nx,nz,F,cubic", [("linear", 5, 33, 65, 2, False), ("sector", 9, 29, 50, 1, False),
+                                                  ("volume", 3, 9, 20, 1, False), ("linear", 1, 37, 61, 1, False)])
+def test_iq_in_das_c_order_is_das_c(cuda, kind, W, nx, nz, F, cubic, dim):
+    """das_c's phase: every term as das_c forms it, the channels in its order."""
+    print(f"case window das_c {kind} W={W} dim={dim}", flush=True)
+    prb, scan, seq = _setup(kind, W, nx, nz, 12e-3)
+    plan = make_plan(prb, scan, seq, n_samples=400, n_frames=F, sampling_frequency=10.4e6, initial_time=0.0,
+                     modulation_frequency=5.2e6, sound_speed=C, receive_apodization=BOX,
+                     transmit_apodization=Apodization(), dimension=dim, interpolation=int(cubic), separable_phase=False)
+    assert plan.variant == (0, 0, 0)
+    g = torch.Generator(cuda).manual_seed(W)
+    ch = torch.randn((F, W, prb.N_elements, 400), dtype=torch.complex64, device=cuda, generator=g)
+    ta, ra, td, rd = plan.materialize()
+    assert torch.equal(plan.run(ch), ops.das(ch, 10.4e6, 0.0, ta, ra, td, rd, 5.2e6, dim, dasc_order=True))
+    plan.close()
