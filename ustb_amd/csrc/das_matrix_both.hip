@@ -21,7 +21,8 @@
 // and cosine of an unreduced argument (about 45). A tile with larger phases is
 // summed from das_c's own terms (dasc_sum).
 //
-// Bound by VALU issue (about 35 instructions per 64 terms). Against
+// Bound by latency (the waves wait 46 % of their cycles; about 35 VALU instructions
+// per 64 terms take 32-64 % of the issue slots, 25 waves 25 of 32 wave slots). Against
 // das_matrix_kernel, whose lanes take a sine, a cosine and two branches per
 // term and read the receive rows once per wave (128 channels, 256 x 256 pixels,
 // IQ): 25 waves 0.401 -> 0.180 ms, 16 0.264 -> 0.099, 8 0.135 -> 0.057, 4 0.071

@@ -4,8 +4,9 @@
 // A block is two groups of 256 threads that share out the tile's waves: the
 // receive entries are read once from memory for both (the second read hits
 // the CU's cache), and the 6-13 waves a group holds leave registers for 4-6
-// waves per SIMD. Bound: VALU issue (12 instructions per 64 terms, half the
-// time) and the latency between a step's barrier and its receive entries.
+// waves per SIMD. Bound: the latency between a step's barrier and its receive
+// entries (the waves wait 51 and 52 % of their cycles on the two below); 12 VALU
+// instructions per 64 terms take 26-66 % of the issue slots.
 // Against the gathering kernel:
 //   volume, 1024 channels x 25 waves on 96 x 96 x 128 voxels: 29.9 -> 10.1 ms
 //     (two groups of 13; one group of 16 in two rounds 11.5, of 25 at 3 waves

@@ -1,8 +1,8 @@
 // das_window_rxnone.hip — the window-staged kernels of dimension receive (sum
 // over channels per wave) and none, and the tile lists they all read.
 //
-// Bound: dimension receive by VALU and LDS issue (10 VALU and 8 LDS cycles per
-// 64 terms), none by its stores. Measured against the per-lane kernel, which
+// Bound: dimension receive by the wait for a step's receive entries (53 % of the
+// wave cycles; VALU 32-64 %, LDS 27 %), none by its stores. Measured against the per-lane kernel, which
 // forms delay, weight and phase of every (pixel, channel) in FP64 for every 8
 // waves and every frame: 64 channels x 31 waves x 4 frames on 193 x 512 pixels
 // of a sector (receive, then the coherence factor) 4.69 -> 0.48 ms; 128

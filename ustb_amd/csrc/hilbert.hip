@@ -559,13 +559,12 @@ hipError_t twiddles(int dev, int N, hipStream_t s, const float2** out) {
 // transform and the last, whose points are the thread's own (so the product
 // with g and the global loads and stores need no LDS pass). Bound by the LDS
 // passes and their barriers (6 passes per pair at N = 4096; the floor of HBM
-// traffic is 0.035 ms where this takes 0.081). 9600 traces, against hipFFT
-// (Bluestein's algorithm, or its own radices 11 and 13 at 2176):
-//   L = 257: 0.022 (0.130) ms; 1021: 0.036 (0.308); 1527: 0.082 (0.615);
-//   2049: 0.218 (1.56); 2176: 0.22 (0.63); 4095: 0.28 (1.83); 5000: 0.68
-//   (1.10); 7919: 0.75 (4.67); 8192: 0.74 (0.90)
-// with errors against FP64 of 0.9-1.3e-7 (2-4e-7): the real parts are the
-// samples themselves and there is half the arithmetic.
+// traffic is 0.035 ms where this takes 0.072). 9600 traces, against hipFFT
+// (Bluestein's algorithm):
+//   L = 257: 0.021 (0.130) ms; 1021: 0.034 (0.308); 1527: 0.072 (0.615); 2049:
+//   0.186 (1.56); 5000: 0.64 (1.10); 8191: 0.69 (4.7)
+// with errors against FP64 of 0.9-1.3e-7 of a trace's norm (2-4e-7): the real
+// parts are the samples themselves and there is half the arithmetic.
 constexpr int kConvMaxL = 8192;
 constexpr int conv_points(int N) { return N <= 4096 ? 8 : 16; }
 
