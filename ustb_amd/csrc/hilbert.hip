@@ -561,8 +561,8 @@ hipError_t twiddles(int dev, int N, hipStream_t s, const float2** out) {
 // passes and their barriers (6 passes per pair at N = 4096; the floor of HBM
 // traffic is 0.035 ms where this takes 0.072). 9600 traces, against hipFFT
 // (Bluestein's algorithm):
-//   L = 257: 0.021 (0.130) ms; 1021: 0.034 (0.308); 1527: 0.072 (0.615); 2049:
-//   0.186 (1.56); 5000: 0.64 (1.10); 8191: 0.69 (4.7)
+//   L = 257: 0.021 (0.119) ms; 1021: 0.035 (0.268); 1527: 0.071 (0.575); 2049:
+//   0.186 (1.55); 5000: 0.64 (1.08); 8191: 0.69 (4.86)
 // with errors against FP64 of 0.9-1.3e-7 of a trace's norm (2-4e-7): the real
 // parts are the samples themselves and there is half the arithmetic.
 constexpr int kConvMaxL = 8192;
